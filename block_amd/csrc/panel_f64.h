@@ -1,0 +1,262 @@
+// FP64 panel kernel of the medium blocks (included by sigma.hip inside its
+// anonymous namespace).
+//
+// Every pair of a V block that reads the same C block needs the same C
+// operands, so the planner orders a block's pairs by C block and a workgroup
+// keeps C in LDS (transposed, zero-padded to 16s) while it walks them.  A
+// wavefront owns 16 rows of the V block (all its columns, up to 80): per pair
+// it holds its rows of op(A) in registers, forms W^T = C^T op(A)^T 16 W columns
+// at a time (C^T from LDS), and the result registers are at once the A operand
+// of the product with B'.  What a wavefront streams per pair is op(A)'s rows
+// and B'; both are requested a step ahead (op(A) a pair, B' 16 rows) in a
+// second register set.  The waves of a workgroup (the 16-row panels of one
+// V block) meet only where the C block changes.
+//
+// K order: a 16-byte load takes two K of an operand whose K is contiguous,
+// so K step (s, e) of lane lk is 8 s + 2 lk + e in op(A) C, and W column
+// 4 lk + i of a 16-column group in W B' (the C^T rows are permuted for that).
+struct PanelPair {
+  int64_t a, c, b;       // offsets; a, b < 0: identity
+  double alpha;
+  int32_t k1, k2, trans, pad;  // trans: bit 0 op(A) stored k1 x m, bit 1 B' stored n x k2
+};
+
+constexpr int PANEL_MAX = 80;  // rows, columns and contraction depths the kernel takes
+// LDS place of C(k, col): 16-byte pairs of K, the eight pairs of 16 K in an
+// order that lets 8 lanes (columns 0, 4, 8, 12, 1, 5, 9, 13 or those two on)
+// meet every bank once
+__device__ __forceinline__ int panel_at(int col, int k, int kp) {
+  const int f = ((col >> 2) & 3) | ((col & 1) << 2);
+  return col * kp + (k & ~15) + ((((k >> 1) ^ f) & 7) << 1) + (k & 1);
+}
+
+// One run of pairs with the same C block, k1 <= 16 KB and n <= 16 NB (a whole
+// wavefront: rows row0 .. row0 + 15 of the block)
+template <int KB, int NB>
+__device__ __forceinline__ void panel_run(const PanelPair* __restrict__ prs, int count,
+                                          const double* __restrict__ arena, const double* cl, int kp, int m, int n,
+                                          int k1, int k2, int row0, int li, int lk, dbl4 (&acc)[NB]) {
+  const int nk = (k1 + 7) >> 3, njb = (k2 + 15) >> 4;
+  // byte offsets in a block, the same for every pair of the run: op(A)
+  // (row row0 + li) and B' (column li of a 16-column group)
+  const uint32_t oa0 = (uint32_t)((row0 + li) * k1 + 2 * lk) * 8u;   // m x k1, K contiguous
+  const uint32_t oa1 = (uint32_t)(2 * lk * m + row0 + li) * 8u;      // k1 x m
+  const uint32_t ob0 = (uint32_t)(4 * lk * n + li) * 8u;             // k2 x n
+  const uint32_t ob1 = (uint32_t)(li * k2 + 4 * lk) * 8u;            // n x k2, K contiguous
+  const double* cp[2];  // this lane's C^T row of a 16-column group (permuted), K pairs lk and 4 + lk
+  {
+    const int col = 4 * (li & 3) + (li >> 2);
+    cp[0] = cl + panel_at(col, 2 * lk, kp);
+    cp[1] = cl + panel_at(col, 8 + 2 * lk, kp);
+  }
+  dbl2 an[2 * KB], bn[2 * NB];
+  auto load_a = [&](const PanelPair& p) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t r = block_rsrc(arena + p.a, (int64_t)m * k1);
+    if (p.trans & 1) {
+#pragma unroll
+      for (int s = 0; s < 2 * KB; ++s)
+        if (s < nk) {
+          an[s][0] = bload2(r, oa1, (uint32_t)(8 * s * m) * 8u);
+          an[s][1] = bload2(r, oa1, (uint32_t)(8 * s * m + m) * 8u);
+        }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 2 * KB; ++s)
+        if (s < nk) an[s] = bload128(r, oa0, 64u * s);
+    }
+  };
+  auto load_b = [&](const PanelPair& p, int jb) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t r = block_rsrc(arena + p.b, (int64_t)n * k2);
+    if (p.trans & 2) {
+#pragma unroll
+      for (int t = 0; t < NB; ++t) {
+        const uint32_t o = ob1 + (uint32_t)(t * k2) * 128u;
+        bn[2 * t] = bload128(r, o, 128u * jb);
+        bn[2 * t + 1] = bload128(r, o + 16u, 128u * jb);
+      }
+    } else {
+      const uint32_t s0 = (uint32_t)(jb * n) * 128u;
+#pragma unroll
+      for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bn[2 * t + (i >> 1)][i & 1] = bload2(r, ob0 + 128u * t, s0 + (uint32_t)(i * n) * 8u);
+    }
+  };
+  PanelPair cur = prs[0];
+  PanelPair nxt = prs[count > 1 ? 1 : 0];
+  load_a(cur);
+  load_b(cur, 0);
+  for (int q = 0; q < count; ++q) {
+    dbl2 a[2 * KB];
+#pragma unroll
+    for (int s = 0; s < 2 * KB; ++s) a[s] = an[s];
+    const PanelPair pr = cur;
+    cur = nxt;
+    if (q + 2 < count) nxt = prs[q + 2];
+    if (q + 1 < count) load_a(cur);
+    for (int jb = 0; jb < njb; ++jb) {
+      dbl2 b[2 * NB];
+#pragma unroll
+      for (int t = 0; t < 2 * NB; ++t) b[t] = bn[t];
+      if (jb + 1 < njb)
+        load_b(pr, jb + 1);
+      else if (q + 1 < count)
+        load_b(cur, 0);
+      // register i of lane (li, lk): W(row0 + li, 16 jb + 4 lk + i)
+      dbl4 w = dbl4{0.0, 0.0, 0.0, 0.0};
+      const int o = jb * 16 * kp;
+#pragma unroll
+      for (int s = 0; s < 2 * KB; ++s)
+        if (s < nk) {
+          const dbl2 x = *(const dbl2*)(cp[s & 1] + o + (s >> 1) * 16);
+          w = __builtin_amdgcn_mfma_f64_16x16x4f64(x[0], a[s][0], w, 0, 0, 0);
+          w = __builtin_amdgcn_mfma_f64_16x16x4f64(x[1], a[s][1], w, 0, 0, 0);
+        }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const double wv = pr.alpha * w[i];
+#pragma unroll
+        for (int t = 0; t < NB; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(wv, b[2 * t + (i >> 1)][i & 1], acc[t], 0, 0, 0);
+      }
+    }
+  }
+}
+
+// A pair with an identity partner (any sizes up to PANEL_MAX), C in LDS
+template <int NB>
+__device__ __forceinline__ void panel_identity(const PanelPair& pr, const double* __restrict__ arena, const double* cl,
+                                               int kp, int m, int n, int row0, int li, int lk, dbl4 (&acc)[NB]) {
+  if (pr.a < 0 && pr.b < 0) {  // V += alpha C
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = row0 + lk + 4 * i, col = 16 * t + li;
+        if (row < m && col < n) acc[t][i] += pr.alpha * cl[panel_at(col, row, kp)];
+      }
+  } else if (pr.a < 0) {  // V += alpha C B': W(row0 + li, k) = alpha C(row0 + li, k)
+    const __amdgpu_buffer_rsrc_t r = block_rsrc(arena + pr.b, (int64_t)n * pr.k2);
+    const int ks = (pr.trans & 2) ? 1 : n, cs = (pr.trans & 2) ? pr.k2 : 1;
+    for (int k0 = 0; k0 < pr.k2; k0 += 4) {
+      const int k = k0 + lk;
+      const double wv = k < pr.k2 && row0 + li < m ? pr.alpha * cl[panel_at(k, row0 + li, kp)] : 0.0;
+#pragma unroll
+      for (int t = 0; t < NB; ++t) {
+        const int col = 16 * t + li;
+        const double b = bload(r, k < pr.k2 && col < n ? (uint32_t)(k * ks + col * cs) * 8u : OOB);
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(wv, b, acc[t], 0, 0, 0);
+      }
+    }
+  } else {  // V += alpha op(A) C
+    const __amdgpu_buffer_rsrc_t r = block_rsrc(arena + pr.a, (int64_t)m * pr.k1);
+    const int ks = (pr.trans & 1) ? m : 1, rs = (pr.trans & 1) ? 1 : pr.k1;
+    for (int k0 = 0; k0 < pr.k1; k0 += 4) {
+      const int k = k0 + lk;
+      const double a = pr.alpha * bload(r, k < pr.k1 && row0 + li < m ? (uint32_t)((row0 + li) * rs + k * ks) * 8u : OOB);
+#pragma unroll
+      for (int t = 0; t < NB; ++t) {
+        const int col = 16 * t + li;
+        const double x = k < pr.k1 && col < n ? cl[panel_at(col, k, kp)] : 0.0;
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x, acc[t], 0, 0, 0);
+      }
+    }
+  }
+}
+
+// One work unit's rows: four wavefronts at most, one 16-row panel each
+// (TileRef: item = segment, pad = panels of a workgroup, tm = which of them).
+template <int KB, int NB>
+__device__ __forceinline__ void panel_unit(const Seg& sg, const bsg_vblock_t& vb, const PanelPair* __restrict__ prs,
+                                           const double* __restrict__ arena, const double* __restrict__ c,
+                                           double* __restrict__ v, double* __restrict__ part, double* cl, int row0,
+                                           bool active) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  dbl4 acc[NB];  // register i of lane (li, lk): V(row0 + lk + 4 i, 16 t + li)
+#pragma unroll
+  for (int t = 0; t < NB; ++t) acc[t] = dbl4{0.0, 0.0, 0.0, 0.0};
+  for (int q = 0; q < sg.count;) {
+    const PanelPair p0 = prs[sg.first + q];
+    const int k1 = p0.k1, k2 = p0.k2, kp = (k1 + 15) & ~15, np = (k2 + 15) & ~15;
+    // C^T into LDS, zeros up to whole 16s
+    __syncthreads();
+    {
+      const __amdgpu_buffer_rsrc_t r = block_rsrc(c + p0.c, (int64_t)k1 * k2);
+      for (int e = threadIdx.x; e < kp * np; e += 256) {
+        const int k = e / np, col = e - k * np;
+        cl[panel_at(col, k, kp)] = bload(r, k < k1 && col < k2 ? (uint32_t)(k * k2 + col) * 8u : OOB);
+      }
+    }
+    // the run of pairs on this C block: identity partners first (the planner's order)
+    int e = q;
+    while (e < sg.count) {
+      const PanelPair& p = prs[sg.first + e];
+      if (p.c != p0.c || p.k1 != k1 || p.k2 != k2) break;
+      ++e;
+    }
+    __syncthreads();
+    if (active) {
+      while (q < e) {
+        const PanelPair pr = prs[sg.first + q];
+        if (pr.a >= 0 && pr.b >= 0) break;
+        panel_identity<NB>(pr, arena, cl, kp, vb.m, vb.n, row0, li, lk, acc);
+        ++q;
+      }
+      if (q < e) panel_run<KB, NB>(prs + sg.first + q, e - q, arena, cl, kp, vb.m, vb.n, k1, k2, row0, li, lk, acc);
+    }
+    q = e;
+  }
+  if (!active) return;
+  const bool direct = sg.p_off < 0;
+  double* out = direct ? v + vb.v_off : part + sg.p_off;
+#pragma unroll
+  for (int t = 0; t < NB; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = row0 + lk + 4 * i, col = 16 * t + li;
+      if (row < vb.m && col < vb.n) {
+        double* o = out + row * vb.n + col;
+        *o = direct ? *o + acc[t][i] : acc[t][i];
+      }
+    }
+}
+
+// KB: 16-deep groups of k1 the registers hold, also the largest V column
+// group count and C^T size: 3 (up to 48, three waves per SIMD) or 5 (up to
+// 80, two).
+template <int KB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KB <= 3 ? 3 : 2))) void k_panel(
+    const bsg_vblock_t* __restrict__ vbs, const PanelPair* __restrict__ prs, const Seg* __restrict__ segs,
+    const TileRef* __restrict__ tiles, int ntiles, const double* __restrict__ arena, const double* __restrict__ c,
+    double* __restrict__ v, double* __restrict__ part, RootSet rs) {
+  __shared__ __attribute__((aligned(16))) double cl[256 * KB * KB];
+  int tile;
+  const int root = root_of(blockIdx.x, rs.n, tile);
+  if (tile >= ntiles) return;
+  const TileRef tr = tiles[tile];
+  if (tr.item < 0) return;  // padding of the XCD-interleaved order
+  const Seg sg = segs[tr.item];
+  const bsg_vblock_t vb = vbs[sg.vb];
+  c += root * rs.wstride;
+  v += root * rs.wstride;
+  part += root * rs.pstride;
+  // a wavefront's panel turns with the workgroup, so that workgroups with
+  // fewer than four panels load all SIMDs alike; a wave without one only
+  // helps with C
+  const int w = (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + blockIdx.x / 8) & 3;
+  const int row0 = 16 * (tr.tm * tr.pad + w);
+  const bool active = w < tr.pad && row0 < vb.m;
+  const int nb = (vb.n + 15) >> 4;
+  if (nb <= 1)
+    panel_unit<KB, 1>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+  else if (nb == 2)
+    panel_unit<KB, 2>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+  else if (KB <= 3 || nb == 3)
+    panel_unit<KB, 3>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+  else if constexpr (KB > 3) {
+    if (nb == 4)
+      panel_unit<KB, 4>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+    else
+      panel_unit<KB, 5>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+  }
+}

@@ -20,9 +20,11 @@
 
 #include <algorithm>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <thread>
 #include <tuple>
+#include <type_traits>
 #include <unordered_map>
 #include <cstdio>
 #include <cstring>
@@ -54,11 +56,12 @@ struct TileRef {
 
 // Several right-hand sides (roots) in one launch: root r reads c + r
 // wstride, accumulates into v + r wstride, keeps its partial tiles at part +
-// r pstride and its BF16 C slices at cslices + r cstride.
+// r pstride, its BF16 C slices at cslices + r cstride and its W scratch at
+// tstride times r.
 struct RootSet {
   int32_t n;
   int32_t pad;
-  int64_t wstride, pstride, cstride;
+  int64_t wstride, pstride, cstride, tstride;
 };
 // Workgroup L of a launch over rs.n roots -> (tile t, root): the roots of one
 // tile are dispatched next to each other, eight workgroups apart, so tile t
@@ -1173,6 +1176,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
 
 
+#include "gemm_f64.h"
+#include "panel_f64.h"
+
 // Tile geometry of the grouped kernels for an m x n V block: waves WR x WC
 // (WR WC = 4), NR 16-row blocks per wave (TM = 16 NR WR <= 64 rows), a W
 // chunk of JC = 16 PB WC columns and a V tile of JV = 16 NV WC columns.
@@ -1231,8 +1237,11 @@ inline Geom make_geom_w8(int nv) {
 struct TileRule {
   int32_t m_lo, m_hi, n_lo, n_hi, fp64, split;
 };
-std::vector<TileRule> g_tile_rules;
-unsigned g_tile_version = 0;  // bumped by bsg_set_tile_table (pick_geom's cache key)
+struct RuleSet {
+  std::vector<TileRule> rules;
+  unsigned version = 0;  // pick_geom's cache key
+};
+std::shared_ptr<const RuleSet> g_tile_rules = std::make_shared<RuleSet>();
 std::vector<Geom> geom_candidates(int max_nv) {
   std::vector<Geom> cand;
   for (int lwr = 0; lwr <= 2; ++lwr)
@@ -1241,29 +1250,29 @@ std::vector<Geom> geom_candidates(int max_nv) {
   cand.push_back(make_geom_w8(max_nv >= 6 ? 6 : 4));
   return cand;
 }
-Geom pick_geom_uncached(int m, int n, int max_nv);
+Geom pick_geom_uncached(const RuleSet& rs, int m, int n, int max_nv);
 // pick_geom per V block shape, remembered per thread (plans repeat shapes)
-inline Geom pick_geom(int m, int n, int max_nv) {
+inline Geom pick_geom(const RuleSet& rs, int m, int n, int max_nv) {
   thread_local std::unordered_map<uint64_t, Geom> cache;
   thread_local unsigned version = ~0u;
-  if (version != g_tile_version) {
+  if (version != rs.version) {
     cache.clear();
-    version = g_tile_version;
+    version = rs.version;
   }
   const uint64_t key = ((uint64_t)(uint32_t)m << 33) | ((uint64_t)(uint32_t)n << 1) | (max_nv >= 6 ? 1u : 0u);
   auto f = cache.find(key);
   if (f != cache.end()) return f->second;
-  const Geom g = pick_geom_uncached(m, n, max_nv);
+  const Geom g = pick_geom_uncached(rs, m, n, max_nv);
   cache.emplace(key, g);
   return g;
 }
-Geom pick_geom_uncached(int m, int n, int max_nv) {
+Geom pick_geom_uncached(const RuleSet& rs, int m, int n, int max_nv) {
   // typical contraction depth: the block's own dimensions
   const long k = std::max(m, n);
   // the two candidate lists, built once (pick_geom runs per V block)
   static const std::vector<Geom> cand_fp64 = geom_candidates(6), cand_split = geom_candidates(4);
   const std::vector<Geom>& cand = max_nv >= 6 ? cand_fp64 : cand_split;
-  for (const TileRule& r : g_tile_rules)
+  for (const TileRule& r : rs.rules)
     if (m >= r.m_lo && m <= r.m_hi && n >= r.n_lo && n <= r.n_hi) {
       const int idx = max_nv >= 6 ? r.fp64 : r.split;
       if (idx >= 0 && idx < (int)cand.size() && cand[idx].tm <= GTM) return cand[idx];
@@ -1301,11 +1310,11 @@ inline int wave_candidate() {
   static const int n = (int)geom_candidates(6).size();
   return n;
 }
-inline bool wave_block(int m, int n) {
-  if (std::max(m, n) <= 32) return false;  // the small-block kernel's
-  for (const TileRule& r : g_tile_rules)
-    if (m >= r.m_lo && m <= r.m_hi && n >= r.n_lo && n <= r.n_hi) return r.fp64 == wave_candidate();
-  return false;
+// FP64 candidate the tile table names for an m x n V block (-1: none)
+inline int fp64_rule(const RuleSet& rs, int m, int n) {
+  for (const TileRule& r : rs.rules)
+    if (m >= r.m_lo && m <= r.m_hi && n >= r.n_lo && n <= r.n_hi) return r.fp64;
+  return -1;
 }
 // MFMA instructions of one pair in a per-wave tile plus a latency allowance
 // (segment cost)
@@ -1315,6 +1324,27 @@ inline long wave_cost(int n, const bsg_pair_t& pr) {
   if (pr.a_off < 0) return (pr.b_off < 0 ? 0 : njb * 4 * nnb) + 24;
   return (pr.b_off < 0 ? nnb * nk1 : njb * (nk1 + 4 * nnb)) + 24;
 }
+typedef GemmTile<2, 2, 2, 2, 4> GemmT;
+// MFMA instructions per wavefront of one pair in a panel plus a latency
+// allowance
+inline long panel_cost(int n, int k1, int k2, bool a, bool b) {
+  const long nb = (n + 15) / 16;
+  if (!a && !b) return 8;
+  if (!a || !b) return ((b ? k2 : k1) + 3) / 4 * nb + 24;
+  return (k2 + 15) / 16 * (2L * ((k1 + 7) / 8) + 4 * nb) + 8;
+}
+inline long panel_cost(int n, const bsg_pair_t& pr) { return panel_cost(n, pr.k1, pr.k2, pr.a_off >= 0, pr.b_off >= 0); }
+inline long panel_cost(int n, const PanelPair& pr) { return panel_cost(n, pr.k1, pr.k2, pr.a >= 0, pr.b >= 0); }
+// The same of one pair in a V tile of the large blocks' products (16-deep
+// chunks) plus its share of a chunk's overhead
+inline long gemm_cost(const bsg_pair_t& pr) {
+  if (pr.a_off < 0 && pr.b_off < 0) return 0;
+  return ((pr.b_off < 0 ? pr.k1 : pr.k2) + GKC - 1) / GKC * 16 + 4;
+}
+// W scratch of the large blocks' rounds, in doubles: one round up to
+// W_ONE_ROUND, else an even number of rounds of at most W_HALF each; roots
+// share a launch while W_ROOTS holds all of them
+constexpr int64_t W_ONE_ROUND = 1 << 21, W_HALF = 1 << 26, W_ROOTS = 1 << 29, W_KEEP = 1 << 27;
 // MFMA instructions per wavefront of one pair in a tile (segment cost)
 inline long pair_cost(const Geom& g, int n, const bsg_pair_t& pr) {
   auto cdiv = [](long a, long b) { return (a + b - 1) / b; };
@@ -1613,8 +1643,20 @@ double* scratch_address(int device) {
 }  // namespace
 
 // ---------------------------------------------------------------- context and plan
+// W scratch of the large blocks' products.  A context's applications run one
+// after the other (its single stream), so its plans share one buffer: plans
+// and their captured graphs keep the buffer they were made with, the context
+// keeps the latest one up to W_KEEP doubles for the next superblock's plan,
+// and the last holder frees it.
+struct WScratch {
+  double* ptr = nullptr;
+  int64_t doubles = 0;
+  ~WScratch() { (void)hipFree(ptr); }  // waits for the device
+};
+
 struct bsg_context {
   int device = 0;
+  std::shared_ptr<WScratch> wscratch;
   hipStream_t stream = nullptr;
   // second stream (default priority) on which the small-block kernel runs
   // beside the grouped kernel; fork/join events tie it to `stream`
@@ -1634,35 +1676,65 @@ struct bsg_context {
   bool abs_leased = false;
 };
 
+// One round of the large blocks' products: the W tiles, then the V tiles
+// that read them.  Rounds alternate between the context stream and the side
+// stream, each with its own half of the W scratch, so that one round's last
+// tiles run beside the next round's first.
+struct GemmRound {
+  TileRef *d_w = nullptr, *d_v = nullptr;  // W tiles, V tiles
+  int n_w = 0, n_v = 0;
+};
+
+// Launch lists of one precision mode of a chunk
+struct ModeLists {
+  bool ready = false;
+  void* d_blob = nullptr;        // one device allocation holding the arrays below
+  Seg* d_seg = nullptr;
+  TileRef* d_g[NCLS] = {};       // grouped-kernel tiles per kernel class (split: basic, 256 wide, 512 wide)
+  int n_g[NCLS] = {};
+  int4* d_s[2] = {};             // FP64 small-block units, 4 per workgroup (SB = 2, SB = 1)
+  int n_s[2] = {};
+  TileRef* d_w[2] = {};          // FP64 per-wave tiles (16 x 32, 16 x 64), 4 per workgroup (item -1: none), a multiple of 32
+  int n_w[2] = {};
+  TileRef* d_p[2] = {};          // FP64 panels (KB = 3, 5) and their pairs
+  int n_p[2] = {};
+  PanelPair* d_pp = nullptr;
+  GemmUnit* d_gu = nullptr;      // FP64 product tiles, by round
+  GemmSeg* d_gs = nullptr;
+  GemmAdd* d_ga = nullptr;
+  std::vector<GemmRound> rounds;
+  RedItem* d_red = nullptr;
+  int n_red = 0;
+  int64_t part_doubles = 0;
+};
+
 struct PlanChunk {
   bsg_vblock_t* d_vb = nullptr;
   bsg_pair_t* d_pr = nullptr;
-  void* d_blob = nullptr;  // one device allocation holding the arrays below (not d_ps)
-  PairS* d_ps = nullptr;  // slice offsets of the grouped kernel's pairs (split precision, built lazily)
-  // host copies for the slice recipes: pairs in device order, the V block of
-  // each grouped-kernel pair (-1: small-block kernel), the V blocks
-  std::vector<bsg_pair_t> h_perm;
-  std::vector<int> h_vbi;
+  void* d_blob = nullptr;  // the allocation of both
+  PairS* d_ps = nullptr;   // slice offsets of the pairs (split precision, built lazily)
+  // host copies for the launch lists: V blocks, pairs in device order (V
+  // block i's at h_base[i], its first h_fast[i] the small-block or per-wave
+  // kernel's)
+  std::unique_ptr<bsg_pair_t[]> h_perm;
+  int64_t n_pairs = 0;
   std::vector<bsg_vblock_t> h_vb;
-  Seg* d_seg = nullptr;
-  TileRef* d_g[NCLS] = {};  // FP64 grouped-kernel tiles per kernel class
-  int n_g[NCLS] = {};
-  TileRef* d_gbf[3] = {};  // split-precision tiles (basic, 256 wide, 512 wide)
-  int n_gbf[3] = {};
-  int4* d_s[2] = {nullptr, nullptr};  // FP64 small-block units, 4 per workgroup (SB = 2, SB = 1)
-  int n_s[2] = {0, 0};
-  TileRef* d_w[2] = {};  // FP64 per-wave tiles (16 x 32, 16 x 64), 4 per workgroup (item -1: none), a multiple of 32
-  int n_w[2] = {};
-  RedItem* d_red[2] = {nullptr, nullptr};  // after the FP64 / the split-precision kernels
-  int n_red[2] = {0, 0};
+  std::vector<int32_t> h_base, h_fast;
+  ModeLists ml[2];  // FP64, split (made by the first bsg_plan_split_arena)
 };
 
 struct bsg_plan {
   bsg_context* ctx = nullptr;
   std::vector<PlanChunk> chunks;
-  double* part = nullptr;    // partial tiles of `batch` roots, part_doubles apart
-  int64_t part_doubles = 0;  // partial tiles of split V blocks per root (largest chunk)
+  // by precision mode: partial tiles of V blocks in several units, of `batch`
+  // roots, part_doubles (the largest chunk's) apart
+  double* part[2] = {};
+  int64_t part_doubles[2] = {};
+  std::shared_ptr<const RuleSet> rules;  // the tile table when the plan was created
   int32_t batch = 1;         // roots per launch (bsg_plan_set_batch)
+  std::shared_ptr<WScratch> wscratch;  // of the large blocks' rounds, wroots roots w_doubles apart
+  int64_t w_doubles = 0;
+  int32_t wroots = 1;        // roots per launch of the rounds
   bool cs_ready = false;     // d_cs holds C slices for `batch` roots
   bool slices_built = false; // slice recipes and pair slice offsets (first bsg_plan_split_arena)
   bool abs_from_ctx = false; // d_abs is the context's lent buffer
@@ -1747,6 +1819,7 @@ int bsg_free(bsg_context* ctx) {
   if (!ctx) return BSG_OK;
   HIPCHK(hipSetDevice(ctx->device));
   HIPCHK(hipStreamSynchronize(ctx->stream));
+  ctx->wscratch.reset();
   HIPCHK(hipFree(ctx->red));
   if (ctx->copy_list) HIPCHK(hipFree(ctx->copy_list));
   HIPCHK(hipStreamSynchronize(ctx->side));
@@ -1820,6 +1893,507 @@ int bsg_memset_zero(bsg_context* ctx, void* dst, size_t bytes) {
   return BSG_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// Contiguous ranges of a chunk's V blocks with about equal pair counts, one
+// per host thread; work(t, first, last) runs on them.  The V blocks are
+// independent: the lists made per range are concatenated in V block order,
+// so a plan does not depend on the number of threads.
+template <class F>
+int over_vblocks(const bsg_vblock_t* vbs, int n_vb, int64_t n_pairs, F&& work) {
+  int nth = (int)std::min<long>(std::max(1u, std::thread::hardware_concurrency()), 16);
+  // starting a thread costs about as much as planning a few thousand pairs
+  nth = (int)std::max<int64_t>(1, std::min<int64_t>({nth, n_pairs / 6000, n_vb}));
+  std::vector<int> bounds(nth + 1, n_vb);
+  bounds[0] = 0;
+  int64_t acc = 0, tot = 0;
+  for (int i = 0; i < n_vb; ++i) tot += std::max(0, vbs[i].count) + 1;
+  int t = 1;
+  for (int i = 0; i < n_vb && t < nth; ++i) {
+    acc += std::max(0, vbs[i].count) + 1;
+    if (acc * nth >= tot * t) bounds[t++] = i + 1;
+  }
+  std::vector<std::thread> th;
+  for (int t = 1; t < nth; ++t) th.emplace_back([&, t] { work(t, bounds[t], bounds[t + 1]); });
+  work(0, bounds[0], bounds[1]);
+  for (auto& x : th) x.join();
+  return nth;
+}
+constexpr int MAX_PLAN_THREADS = 16;
+
+// the context's W scratch if it holds n doubles, else a new one (null: no memory)
+std::shared_ptr<WScratch> w_scratch(bsg_context* ctx, int64_t n) {
+  if (ctx->wscratch && ctx->wscratch->doubles >= n) return ctx->wscratch;
+  auto w = std::make_shared<WScratch>();
+  if (hipMalloc(&w->ptr, sizeof(double) * n) != hipSuccess) return nullptr;
+  w->doubles = n;
+  if (n <= W_KEEP) ctx->wscratch = w;
+  return w;
+}
+
+// Device arrays of one upload: parts gathered in a host buffer (256-byte
+// aligned), sent with one allocation and one copy, their pointers set then.
+struct Blob {
+  std::vector<std::pair<void**, size_t>> parts;
+  std::vector<char> data;
+  void add(void** d, const void* h, size_t bytes) {
+    if (bytes == 0) return;
+    const size_t off = (data.size() + 255) & ~(size_t)255;
+    data.resize(off + bytes);
+    std::memcpy(data.data() + off, h, bytes);
+    parts.push_back({d, off});
+  }
+  template <class T, class P>
+  void add(P** d, const std::vector<T>& h) {
+    add((void**)d, h.data(), sizeof(T) * h.size());
+  }
+  // false: no memory (nothing is left allocated)
+  bool send(void** blob) {
+    if (data.empty()) return true;
+    char* d = nullptr;
+    if (hipMalloc((void**)&d, data.size()) != hipSuccess ||
+        hipMemcpy(d, data.data(), data.size(), hipMemcpyHostToDevice) != hipSuccess) {
+      (void)hipFree(d);
+      return false;
+    }
+    *blob = d;
+    for (auto& x : parts) *x.first = d + x.second;
+    return true;
+  }
+};
+
+// kernels a work unit runs on
+enum UnitKind : char { UK_GROUPED = 0, UK_SMALL = 1, UK_WAVE = 2, UK_GEMM = 3, UK_PANEL3 = 4, UK_PANEL5 = 5 };
+
+// MFMAs per wavefront of a work unit before its pair list is split
+constexpr long SEG_COST = 2048, SEG_COST_SMALL = 1024;
+
+inline bool small_block(const bsg_vblock_t& vb) { return std::max(vb.m, vb.n) <= 32; }
+// whether the small-block kernel takes a pair of a small block
+inline bool small_pair(const bsg_pair_t& pr) {
+  return (pr.a_off >= 0 && pr.k1 <= 32 && pr.k2 <= 32) || (pr.a_off < 0 && pr.b_off < 0);
+}
+
+// The large blocks' products: segments of the V units (bunits: indices into
+// segs, whose pairs are gq's) and of the W tiles they read, in rounds of about
+// equal W size.
+void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, const std::vector<int>& bunits,
+                   const std::vector<int>& gq, const std::vector<Seg>& segs) {
+  const bsg_pair_t* perm = pc.h_perm.get();
+  std::vector<GemmUnit> gu;
+  std::vector<GemmSeg> gs;
+  std::vector<GemmAdd> ga;
+  int64_t wtot = 0;
+  auto w_size = [&](const bsg_vblock_t& vb, const bsg_pair_t& pr) {
+    return pr.a_off >= 0 && pr.b_off >= 0 ? (((int64_t)vb.m * pr.k2 + 1) & ~(int64_t)1) : 0;
+  };
+  for (int bu : bunits) {
+      const Seg& sg = segs[bu];
+      for (int q = 0; q < sg.count; ++q) wtot += w_size(pc.h_vb[sg.vb], perm[gq[sg.first + q]]);
+  }
+  // an even number of rounds once W is large enough to be worth two
+  int64_t nround = 1;
+  if (wtot > W_ONE_ROUND) nround = 2 * ((wtot + W_HALF * 2 - 1) / (W_HALF * 2));
+  const int64_t target = (wtot + nround - 1) / std::max<int64_t>(1, nround);
+  ml.rounds.reserve(nround + 2);
+  std::vector<GUnit> uw, uv;
+  int64_t wused = 0, wneed[2] = {};
+  std::vector<std::pair<std::vector<TileRef>, std::vector<TileRef>>> rt;  // W tiles, V tiles
+  auto close_round = [&]() {
+    if (uv.empty()) return;
+    int64_t& need = wneed[rt.size() & 1];
+    need = std::max(need, wused);
+    rt.push_back({xcd_order(uw), xcd_order(uv)});
+    uw.clear();
+    uv.clear();
+    wused = 0;
+  };
+  for (int bu : bunits) {
+    const Seg& sg = segs[bu];
+    const bsg_vblock_t& vb = pc.h_vb[sg.vb];
+    GemmUnit un{};
+    un.out = sg.p_off < 0 ? vb.v_off : sg.p_off;
+    un.kind = sg.p_off < 0 ? GU_V : GU_PART;
+    un.m = vb.m;
+    un.n = vb.n;
+    un.alpha = 1.0;
+    un.add_first = (int32_t)ga.size();
+    std::vector<GemmSeg> mine;
+    long vcost = 0;
+    for (int q = 0; q < sg.count; ++q) {
+      const bsg_pair_t& pr = perm[gq[sg.first + q]];
+      if (pr.a_off < 0 && pr.b_off < 0) {
+        ga.push_back({pr.c_off, pr.alpha});
+        continue;
+      }
+      GemmSeg x{};
+      if (pr.a_off < 0) {  // V += alpha C B'
+        x = GemmSeg{pr.c_off, pr.b_off, pr.alpha, pr.k2, (SP_C << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0)};
+      } else if (pr.b_off < 0) {  // V += alpha op(A) C
+        x = GemmSeg{pr.a_off, pr.c_off, pr.alpha * pr.alpha_a, pr.k1, (SP_C << SEG_RSPACE) | (pr.a_trans ? SEG_LT : 0)};
+      } else {
+        GemmUnit w{};  // W = alpha op(A) C (m x k2)
+        w.out = wused;  // the half's offset is added below
+        w.kind = GU_W;
+        w.m = vb.m;
+        w.n = pr.k2;
+        w.first = (int32_t)gs.size();
+        w.count = 1;
+        w.alpha = pr.alpha * pr.alpha_a;
+        gs.push_back(GemmSeg{pr.a_off, pr.c_off, 1.0, pr.k1,
+                             (SP_C << SEG_RSPACE) | (pr.a_trans ? SEG_LT : 0)});
+        GUnit t;
+        t.cost = (pr.k1 + GKC - 1) / GKC + 4;
+        t.seg = (int)gu.size();
+        t.ntm = (w.m + GemmT::TM - 1) / GemmT::TM;
+        t.ntn = (w.n + GemmT::TN - 1) / GemmT::TN;
+        w.pad = (int32_t)(rt.size() & 1);
+        gu.push_back(w);
+        uw.push_back(t);
+        x = GemmSeg{wused, pr.b_off, 1.0, pr.k2, (SP_W << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0) |
+                                                     (int32_t)((rt.size() & 1) << SEG_HALF)};
+        wused += w_size(vb, pr);
+      }
+      vcost += gemm_cost(pr);
+      mine.push_back(x);
+    }
+    un.add_count = (int32_t)ga.size() - un.add_first;
+    un.first = (int32_t)gs.size();
+    un.count = (int32_t)mine.size();
+    gs.insert(gs.end(), mine.begin(), mine.end());
+    GUnit t;
+    t.cost = vcost;
+    t.seg = (int)gu.size();
+    t.ntm = (un.m + GemmT::TM - 1) / GemmT::TM;
+    t.ntn = (un.n + GemmT::TN - 1) / GemmT::TN;
+    gu.push_back(un);
+    uv.push_back(t);
+    if (wused >= target) close_round();
+  }
+  close_round();
+  // the second half of the scratch follows the first
+  for (GemmUnit& u : gu)
+    if (u.kind == GU_W && u.pad) u.out += wneed[0];
+  for (GemmSeg& x : gs) {
+    if (((x.flags >> SEG_LSPACE) & 3) == SP_W && ((x.flags >> SEG_HALF) & 1)) x.l += wneed[0];
+  }
+  p->w_doubles = std::max(p->w_doubles, wneed[0] + wneed[1]);
+  blob.add(&ml.d_gu, gu);
+  blob.add(&ml.d_gs, gs);
+  blob.add(&ml.d_ga, ga);
+  ml.rounds.resize(rt.size());
+  for (size_t r = 0; r < rt.size(); ++r) {
+    blob.add(&ml.rounds[r].d_w, rt[r].first);
+    blob.add(&ml.rounds[r].d_v, rt[r].second);
+    ml.rounds[r].n_w = (int)rt[r].first.size();
+    ml.rounds[r].n_v = (int)rt[r].second.size();
+  }
+}
+
+// The launch lists of one precision mode: every V block's pairs (in device
+// order: the h_fast first ones are the small-block or per-wave kernel's) are
+// cut into work units of about SEG_COST MFMAs per wave; blocks with several
+// units get partial tiles and an ordered reduction.
+int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
+  ModeLists& ml = pc.ml[split];
+  struct Local {
+    std::vector<GUnit> gunits[NCLS];                 // grouped tiles by kernel class
+    std::vector<std::pair<long, int>> sunits[2];     // (cost, segment) of small-block units (SB = 2, SB = 1)
+    std::vector<int> bunits;                         // large blocks' units (segments)
+    std::vector<GUnit> wunits[2], punits[2];         // per-wave tiles (16 x 32, 16 x 64), panels (KB = 3, 5)
+    std::vector<int> gq;                             // pairs of the large blocks' units (indices into h_perm)
+    std::vector<PanelPair> pp;
+    std::vector<Seg> segs;
+    std::vector<RedItem> reds;
+    int64_t poff = 0;
+  };
+  std::vector<Local> loc(MAX_PLAN_THREADS);
+  const int nvb = (int)pc.h_vb.size();
+  const int nth = over_vblocks(pc.h_vb.data(), nvb, pc.n_pairs, [&](int t, int i0, int i1) {
+    Local& L = loc[t];
+    std::vector<std::pair<int, int>> units;  // (first, count)
+    std::vector<char> ukind;
+    std::vector<int> pan[2], big;
+    for (int i = i0; i < i1; ++i) {
+      const bsg_vblock_t& vb = pc.h_vb[i];
+      const bsg_pair_t* perm = pc.h_perm.get();
+      const int base = pc.h_base[i], nfast = pc.h_fast[i], ntot = vb.count;
+      const bool sm = small_block(vb);
+      const int rule = split ? -1 : fp64_rule(*p->rules, vb.m, vb.n);
+      const bool wave_vb = !split && !sm && rule == wave_candidate();
+      units.clear();
+      ukind.clear();
+      Geom g;
+      auto cost_of = [&](int kind, const bsg_pair_t& pr) -> long {
+        switch (kind) {
+          case UK_SMALL: return small_cost(vb.m, vb.n, pr);
+          case UK_WAVE: return wave_cost(vb.n, pr);
+          case UK_GEMM: return gemm_cost(pr);
+          case UK_PANEL3:
+          case UK_PANEL5: return panel_cost(vb.n, pr);
+          default: return pair_cost(g, vb.n, pr);
+        }
+      };
+      // at(q): the list's q-th pair; first: its index where the units point
+      auto cut = [&](int first, int n, int kind, auto at) {
+        const long lim = kind == UK_SMALL ? SEG_COST_SMALL : SEG_COST;
+        int start = 0;
+        long cost = 0;
+        for (int q = 0; q < n; ++q) {
+          cost += cost_of(kind, at(q));
+          if (cost >= lim || q + 1 == n) {
+            units.push_back({first + start, q + 1 - start});
+            ukind.push_back((char)kind);
+            start = q + 1;
+            cost = 0;
+          }
+        }
+      };
+      auto in_perm = [&](int first) { return [&, first](int q) -> const bsg_pair_t& { return perm[first + q]; }; };
+      const int slow = split && !sm ? 0 : nfast;  // pairs the small-block or per-wave kernel takes
+      if (slow > 0) cut(base, slow, wave_vb ? UK_WAVE : UK_SMALL, in_perm(base));
+      if (slow < ntot) {
+        if (split || wave_vb || (!sm && rule >= 0)) {
+          g = pick_geom(*p->rules, vb.m, vb.n, split ? 4 : 6);
+          cut(base + slow, ntot - slow, UK_GROUPED, in_perm(base + slow));
+        } else {
+          const bool med = std::max(vb.m, vb.n) <= PANEL_MAX;
+          for (auto& x : pan) x.clear();
+          big.clear();
+          for (int q = base + slow; q < base + ntot; ++q) {
+            const int k = std::max(perm[q].k1, perm[q].k2);
+            if (!med || k > PANEL_MAX)
+              big.push_back(q);
+            else
+              pan[k > 48 || vb.n > 48].push_back(q);
+          }
+          for (int k = 0; k < 2; ++k) {
+            if (pan[k].empty()) continue;
+            // by C block, identity partners first, else as given
+            std::stable_sort(pan[k].begin(), pan[k].end(), [&](int x, int y) {
+              const bsg_pair_t &a = perm[x], &b = perm[y];
+              if (a.c_off != b.c_off) return a.c_off < b.c_off;
+              return (a.a_off < 0 || a.b_off < 0) && !(b.a_off < 0 || b.b_off < 0);
+            });
+            const int first = (int)L.pp.size();
+            for (int q : pan[k]) {
+              const bsg_pair_t& x = perm[q];
+              L.pp.push_back(PanelPair{x.a_off, x.c_off, x.b_off, x.a_off < 0 ? x.alpha : x.alpha * x.alpha_a, x.k1, x.k2,
+                                       (x.a_trans ? 1 : 0) | (x.b_trans ? 2 : 0), 0});
+            }
+            cut(first, (int)pan[k].size(), k ? UK_PANEL5 : UK_PANEL3, [&](int q) -> const bsg_pair_t& { return perm[pan[k][q]]; });
+          }
+          if (!big.empty()) {
+            const int first = (int)L.gq.size();
+            L.gq.insert(L.gq.end(), big.begin(), big.end());
+            cut(first, (int)big.size(), UK_GEMM, [&](int q) -> const bsg_pair_t& { return perm[big[q]]; });
+          }
+        }
+      }
+      const int64_t mn = (int64_t)vb.m * vb.n;
+      const int nseg = (int)units.size();
+      const int64_t p0 = L.poff;
+      bool tiny = std::max(vb.m, vb.n) <= 16;  // the block and its small-kernel pairs' C blocks within 16 x 16
+      if (tiny && !wave_vb)
+        for (int q = 0; q < slow; ++q)
+          if (perm[base + q].k1 > 16 || perm[base + q].k2 > 16) {
+            tiny = false;
+            break;
+          }
+      for (int u = 0; u < nseg; ++u) {
+        Seg sg;
+        sg.vb = i;
+        sg.first = units[u].first;
+        sg.count = units[u].second;
+        sg.pad = 0;
+        sg.p_off = nseg == 1 ? -1 : p0 + (int64_t)u * mn;
+        const int si = (int)L.segs.size();
+        L.segs.push_back(sg);
+        const int kind = ukind[u];
+        if (kind == UK_GEMM) {
+          L.bunits.push_back(si);
+          continue;
+        }
+        long ucost = 0;
+        if (kind == UK_PANEL3 || kind == UK_PANEL5)
+          for (int q = 0; q < sg.count; ++q) ucost += panel_cost(vb.n, L.pp[sg.first + q]);
+        else
+          for (int q = 0; q < sg.count; ++q) ucost += cost_of(kind, perm[sg.first + q]);
+        if (kind == UK_SMALL) {
+          L.sunits[tiny ? 1 : 0].push_back({ucost, si});
+          continue;
+        }
+        GUnit gu;
+        gu.cost = ucost;
+        gu.seg = si;
+        if (kind == UK_WAVE) {
+          const int nb = wave_nb(vb.n);
+          gu.ntm = (vb.m + 15) / 16;
+          gu.ntn = (vb.n + 16 * nb - 1) / (16 * nb);
+          L.wunits[nb == 4].push_back(gu);
+        } else if (kind == UK_PANEL3 || kind == UK_PANEL5) {
+          const int np = (vb.m + 15) / 16;
+          gu.ntm = (np + 3) / 4;                    // workgroups
+          gu.code = (np + gu.ntm - 1) / gu.ntm;     // panels of each
+          gu.ntn = 1;
+          L.punits[kind == UK_PANEL5].push_back(gu);
+        } else {
+          gu.ntm = (vb.m + g.tm - 1) / g.tm;
+          gu.ntn = (vb.n + g.jv - 1) / g.jv;
+          gu.code = g.code;
+          L.gunits[g.cls].push_back(gu);
+        }
+      }
+      if (nseg > 1) {
+        for (int64_t e0 = 0; e0 < mn; e0 += 256) {
+          RedItem r;
+          r.v_off = vb.v_off;
+          r.p_off = p0;
+          r.nseg = nseg;
+          r.mn = (int32_t)mn;
+          r.e0 = (int32_t)e0;
+          r.len = (int32_t)std::min<int64_t>(256, mn - e0);
+          L.reds.push_back(r);
+        }
+        L.poff += nseg * mn;
+      }
+    }
+  });
+  // concatenate with the local indices shifted
+  std::vector<GUnit> gunits[NCLS], wunits[2], punits[2];
+  std::vector<std::pair<long, int>> sunits[2];
+  std::vector<int> bunits, gq;
+  std::vector<PanelPair> pp;
+  std::vector<Seg> segs;
+  std::vector<RedItem> reds;
+  int64_t poff = 0;
+  if (nth == 1) {
+    Local& L = loc[0];
+    for (int k = 0; k < NCLS; ++k) gunits[k].swap(L.gunits[k]);
+    for (int k = 0; k < 2; ++k) {
+      wunits[k].swap(L.wunits[k]);
+      punits[k].swap(L.punits[k]);
+      sunits[k].swap(L.sunits[k]);
+    }
+    bunits.swap(L.bunits);
+    gq.swap(L.gq);
+    pp.swap(L.pp);
+    segs.swap(L.segs);
+    reds.swap(L.reds);
+    poff = L.poff;
+  } else {
+    size_t ns = 0, np = 0, nr = 0;
+    for (int t = 0; t < nth; ++t) ns += loc[t].segs.size(), np += loc[t].pp.size(), nr += loc[t].reds.size();
+    segs.reserve(ns);
+    pp.reserve(np);
+    reds.reserve(nr);
+    for (int t = 0; t < nth; ++t) {
+      Local& L = loc[t];
+      const int sb = (int)segs.size(), ppb = (int)pp.size(), gb = (int)gq.size();
+      std::vector<char> kind(L.segs.size(), 0);  // 1: the unit's pairs are in pp, 2: in gq
+      for (int k = 0; k < 2; ++k)
+        for (const GUnit& u : L.punits[k]) kind[u.seg] = 1;
+      for (int s : L.bunits) kind[s] = 2;
+      for (size_t s = 0; s < L.segs.size(); ++s) {
+        Seg sg = L.segs[s];
+        if (kind[s]) sg.first += kind[s] == 1 ? ppb : gb;
+        if (sg.p_off >= 0) sg.p_off += poff;
+        segs.push_back(sg);
+      }
+      auto shift = [&](std::vector<GUnit>& to, const std::vector<GUnit>& from) {
+        for (GUnit u : from) {
+          u.seg += sb;
+          to.push_back(u);
+        }
+      };
+      for (int k = 0; k < NCLS; ++k) shift(gunits[k], L.gunits[k]);
+      for (int k = 0; k < 2; ++k) {
+        shift(wunits[k], L.wunits[k]);
+        shift(punits[k], L.punits[k]);
+        for (auto x : L.sunits[k]) sunits[k].push_back({x.first, x.second + sb});
+      }
+      for (int s : L.bunits) bunits.push_back(s + sb);
+      gq.insert(gq.end(), L.gq.begin(), L.gq.end());
+      pp.insert(pp.end(), L.pp.begin(), L.pp.end());
+      for (RedItem r : L.reds) {
+        r.p_off += poff;
+        reds.push_back(r);
+      }
+      poff += L.poff;
+    }
+  }
+  ml.part_doubles = poff;
+  Blob blob;
+  blob.data.reserve(sizeof(Seg) * segs.size() + sizeof(RedItem) * reds.size() + sizeof(PanelPair) * pp.size() +
+                    8 * segs.size() + (1 << 16));
+  blob.add(&ml.d_seg, segs);
+  blob.add(&ml.d_red, reds);
+  ml.n_red = (int)reds.size();
+  blob.add(&ml.d_pp, pp);
+  // small-block units, costliest first, four per workgroup
+  for (int k = 0; k < 2; ++k) {
+    auto& su = sunits[k];
+    std::sort(su.begin(), su.end(), [](const std::pair<long, int>& x, const std::pair<long, int>& y) {
+      return x.first != y.first ? x.first > y.first : x.second < y.second;
+    });
+    std::vector<int4> sq;
+    sq.reserve(su.size() / 4 + 1);
+    for (size_t i = 0; i < su.size(); i += 4) {
+      int e[4];
+      for (int j = 0; j < 4; ++j) e[j] = i + j < su.size() ? su[i + j].second : -1;
+      sq.push_back(make_int4(e[0], e[1], e[2], e[3]));
+    }
+    blob.add(&ml.d_s[k], sq);
+    ml.n_s[k] = (int)sq.size();
+  }
+  for (int k = 0; k < NCLS; ++k) {
+    const std::vector<TileRef> t = xcd_order(gunits[k]);
+    blob.add(&ml.d_g[k], t);
+    ml.n_g[k] = (int)t.size();
+  }
+  for (int k = 0; k < 2; ++k) {
+    const std::vector<TileRef> t = xcd_order(punits[k]);
+    blob.add(&ml.d_p[k], t);
+    ml.n_p[k] = (int)t.size();
+  }
+  // per-wave tiles of each width: units (costliest first) go to the least
+  // loaded of the 8 XCDs, a unit's tiles in consecutive wave slots of that
+  // XCD's workgroups (they share the unit's C and B' blocks in its L2);
+  // workgroup 8 j + x is XCD x's j-th
+  for (int k = 0; k < 2; ++k) {
+    std::vector<std::pair<long, int>> order;
+    for (int u = 0; u < (int)wunits[k].size(); ++u)
+      order.push_back({wunits[k][u].cost * wunits[k][u].ntm * wunits[k][u].ntn, u});
+    std::sort(order.begin(), order.end(), [](const std::pair<long, int>& x, const std::pair<long, int>& y) {
+      return x.first != y.first ? x.first > y.first : x.second < y.second;
+    });
+    std::vector<TileRef> q[8];
+    long load[8] = {};
+    for (const auto& o : order) {
+      const int x = (int)(std::min_element(load, load + 8) - load);
+      const GUnit& gu = wunits[k][o.second];
+      for (int tm = 0; tm < gu.ntm; ++tm)
+        for (int tn = 0; tn < gu.ntn; ++tn) q[x].push_back(TileRef{gu.seg, tm, tn, 0});
+      load[x] += o.first;
+    }
+    size_t nwg = 0;
+    for (auto& e : q) nwg = std::max(nwg, (e.size() + 3) / 4);
+    std::vector<TileRef> wt(nwg * 32, TileRef{-1, 0, 0, 0});
+    for (int x = 0; x < 8; ++x)
+      for (size_t e = 0; e < q[x].size(); ++e) wt[((e / 4) * 8 + x) * 4 + e % 4] = q[x][e];
+    blob.add(&ml.d_w[k], wt);
+    ml.n_w[k] = (int)wt.size();
+  }
+  if (!bunits.empty()) plan_products(p, pc, ml, blob, bunits, gq, segs);
+  if (!blob.send(&ml.d_blob)) return fail(BSG_ERR_NOMEM, "plan lists");
+  ml.ready = true;
+  return BSG_OK;
+}
+}  // namespace
+
+extern "C" {
+
 int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunks, int64_t wave_size,
                     bsg_plan** plan) {
   if (!ctx || !plan || (n_chunks > 0 && !chunks) || wave_size < 0) return fail(BSG_ERR_ARG, "bsg_plan_create: bad args");
@@ -1827,370 +2401,105 @@ int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunk
   auto* p = new bsg_plan();
   p->ctx = ctx;
   p->wave_size = wave_size;
-  int64_t pmax = 0;
-  const long SEG_COST = 2048;        // MFMAs per wavefront of a work unit before its pair list is split
-  const long SEG_COST_SMALL = 1024;  // the same for the per-wave small-block units
-  const long SEG_COST_WAVE = 2048;   // and for the per-wave tiles
+  p->rules = g_tile_rules;
   auto cleanup = [&](int code, const std::string& m) {
     bsg_plan_destroy(p);
     return fail(code, m);
   };
+  p->chunks.resize(std::max(0, n_chunks));
   for (int ci = 0; ci < n_chunks; ++ci) {
     const bsg_chunk_t& ch = chunks[ci];
-    PlanChunk pc;
-    // The V blocks are independent: contiguous ranges of them (about equal
-    // in pairs) are planned on host threads into local lists with local
-    // indices, which are then concatenated in V block order (the result does
-    // not depend on the number of threads).
-    struct Local {
-      std::vector<GUnit> gunits[NCLS], gunits_bf[3];  // the tiles of each work unit (FP64, split)
-      std::vector<bsg_pair_t> perm;                   // pairs in device order (grouped per V block as given)
-      std::vector<int> h_vbi;
-      std::vector<std::pair<long, int>> sunits[2];  // (cost, segment) of small-block units
-      std::vector<GUnit> wunits[2];                 // per-wave tile units (cost per tile), 16 x 32 and 16 x 64
-      std::vector<Seg> segs;
-      std::vector<RedItem> reds[2];  // ordered reductions after the FP64 / the split-precision kernels
-      int64_t poff = 0, arena_extent = 0;
-      double flops = 0.0, flops1 = 0.0, flops2 = 0.0, flops_split = 0.0;
-      std::string err;
-      std::vector<int> fast, slow;  // per V block, reused
-      std::vector<std::pair<int, int>> units;
-      std::vector<char> ukind;  // per unit: 0 grouped kernel, 1 small-block kernel, 2 per-wave tiles
-    };
-    auto plan_vblock = [&](int i, Local& L) -> bool {
-      std::vector<bsg_pair_t>& perm = L.perm;
-      std::vector<Seg>& segs = L.segs;
-      int64_t& poff = L.poff;
-      auto& fast = L.fast;
-      auto& slow = L.slow;
-      auto& units = L.units;
-      auto& ukind = L.ukind;
-      const auto& vb = ch.vblocks[i];
+    PlanChunk& pc = p->chunks[ci];
+    int64_t np = 0;
+    pc.h_vb.assign(ch.vblocks, ch.vblocks + ch.n_vblocks);
+    pc.h_base.resize(ch.n_vblocks);
+    pc.h_fast.resize(ch.n_vblocks);
+    for (int i = 0; i < ch.n_vblocks; ++i) {
+      const bsg_vblock_t& vb = ch.vblocks[i];
       if (vb.m <= 0 || vb.n <= 0 || vb.v_off < 0 || vb.v_off + (int64_t)vb.m * vb.n > wave_size || vb.first < 0 ||
-          vb.count < 0 || vb.first + vb.count > ch.n_pairs) {
-        L.err = "bsg_plan_create: vblock out of range";
-        return false;
-      }
-      const Geom gm = pick_geom(vb.m, vb.n, 6);     // FP64 tiles
-      const Geom gs = pick_geom(vb.m, vb.n, 4);     // split-precision tiles
-      // small blocks (up to 32 x 32) go to the per-wave kernel, except pairs
-      // whose C block is larger than that (or whose A is the identity and B
-      // is not): those run in the grouped kernel with its K pipeline
-      const bool small_vb = std::max(vb.m, vb.n) <= 32;
-      // medium blocks the tile table puts on per-wave tiles (FP64 only): the
-      // pairs within the per-wave kernel's contraction depth go there
-      const bool wave_vb = !small_vb && wave_block(vb.m, vb.n);
-      // tiny: the block and every small-kernel pair's C block within 16 x 16
-      bool tiny = std::max(vb.m, vb.n) <= 16;
-      fast.clear();  // pair indices (absolute) in term order
-      slow.clear();
-      for (int q = 0; q < vb.count; ++q) {
-        const auto& pr = ch.pairs[vb.first + q];
-        if (pr.k1 <= 0 || pr.k2 <= 0 || pr.c_off < 0 || pr.c_off + (int64_t)pr.k1 * pr.k2 > wave_size ||
-            (pr.a_off < 0 && pr.k1 != vb.m) || (pr.b_off < 0 && pr.k2 != vb.n)) {
-          L.err = "bsg_plan_create: pair out of range";
-          return false;
-        }
-        if (pr.a_off >= 0) L.arena_extent = std::max(L.arena_extent, pr.a_off + (int64_t)vb.m * pr.k1);
-        if (pr.b_off >= 0) L.arena_extent = std::max(L.arena_extent, pr.b_off + (int64_t)vb.n * pr.k2);
-        if (pr.a_off >= 0) {
-          L.flops += 2.0 * vb.m * pr.k1 * pr.k2;
-          L.flops1 += 2.0 * vb.m * pr.k1 * pr.k2;
-        }
-        if (pr.b_off >= 0) {
-          L.flops += 2.0 * vb.m * pr.k2 * vb.n;
-          L.flops2 += 2.0 * vb.m * pr.k2 * vb.n;
-        }
-        const bool f = small_vb ? (pr.a_off >= 0 && pr.k1 <= 32 && pr.k2 <= 32) || (pr.a_off < 0 && pr.b_off < 0)
-                                : wave_vb && (pr.a_off < 0 || pr.k1 <= 4 * wave_ka(wave_nb(vb.n)));
-        (f ? fast : slow).push_back(vb.first + q);
-        if (!f || wave_vb)  // split mode: every pair of a per-wave block runs on BF16 slices
-          L.flops_split += (pr.a_off >= 0 ? 2.0 * vb.m * pr.k1 * pr.k2 : 0.0) +
-                           (pr.b_off >= 0 ? 2.0 * vb.m * pr.k2 * vb.n : 0.0);
-        if (f && small_vb && (pr.k1 > 16 || pr.k2 > 16)) tiny = false;
-      }
-      // the block's pairs in device order: the small-kernel (per-wave
-      // kernel) ones, then the rest
-      const int base = (int)perm.size();
-      for (int x : fast) {
-        perm.push_back(ch.pairs[x]);
-        L.h_vbi.push_back(wave_vb ? i : -1);  // the small-block kernel reads no slices
-      }
-      for (int x : slow) {
-        perm.push_back(ch.pairs[x]);
-        L.h_vbi.push_back(i);
-      }
-      // cut each list into work units of about SEG_COST(_SMALL) MFMAs per
-      // wave.  A block on wide tiles is cut twice: for the FP64 wide tiles
-      // and for the split-precision kernel's basic tiles (mode 1 and 2, each
-      // with its own partial tiles and reduction); other blocks share one
-      // cut (mode 0).  Wide blocks have no small-kernel pairs.
-      const int64_t mn = (int64_t)vb.m * vb.n;
-      // nf: the first nf pairs go to the kernel of kind fk (1 small-block, 2
-      // per-wave tiles), the rest to the grouped kernel on geometry g
-      auto emit = [&](const Geom& g, int mode, int nf, int fk) {
-        units.clear();  // (first, count) in device order
-        ukind.clear();
-        auto cut = [&](int first, int n, int kind) {
-          const long lim = kind == 1 ? SEG_COST_SMALL : (kind == 2 ? SEG_COST_WAVE : SEG_COST);
-          int start = 0;
-          long cost = 0;
-          for (int q = 0; q < n; ++q) {
-            const auto& pr = perm[first + q];
-            cost += kind == 1 ? small_cost(vb.m, vb.n, pr) : (kind == 2 ? wave_cost(vb.n, pr) : pair_cost(g, vb.n, pr));
-            if (cost >= lim && q + 1 < n) {
-              units.push_back({first + start, q + 1 - start});
-              ukind.push_back((char)kind);
-              start = q + 1;
-              cost = 0;
-            }
-          }
-          if (n > start) {
-            units.push_back({first + start, n - start});
-            ukind.push_back((char)kind);
-          }
-        };
-        const int ntot = (int)(fast.size() + slow.size());
-        cut(base, nf, fk);
-        cut(base + nf, ntot - nf, 0);
-        const int nseg = (int)units.size();
-        for (int u = 0; u < nseg; ++u) {
-          Seg sg;
-          sg.vb = i;
-          sg.first = units[u].first;
-          sg.count = units[u].second;
-          sg.pad = 0;
-          sg.p_off = nseg == 1 ? -1 : poff + (int64_t)u * mn;
-          int si = (int)segs.size();
-          segs.push_back(sg);
-          if (ukind[u] == 1) {
-            long sc = 0;
-            for (int q = 0; q < sg.count; ++q) sc += small_cost(vb.m, vb.n, perm[sg.first + q]);
-            L.sunits[tiny ? 1 : 0].push_back({sc, si});
-            continue;
-          }
-          if (ukind[u] == 2) {
-            GUnit gu;
-            gu.cost = 0;
-            for (int q = 0; q < sg.count; ++q) gu.cost += wave_cost(vb.n, perm[sg.first + q]);
-            gu.seg = si;
-            gu.ntm = (vb.m + 15) / 16;
-            const int nb = wave_nb(vb.n);
-            gu.ntn = (vb.n + 16 * nb - 1) / (16 * nb);
-            gu.code = 0;
-            L.wunits[nb == 4].push_back(gu);
-            continue;
-          }
-          long ucost = 0;
-          for (int q = 0; q < sg.count; ++q) ucost += pair_cost(g, vb.n, perm[sg.first + q]);
-          GUnit gu;
-          gu.cost = ucost;
-          gu.seg = si;
-          gu.ntm = (vb.m + g.tm - 1) / g.tm;
-          gu.ntn = (vb.n + g.jv - 1) / g.jv;
-          gu.code = g.code;
-          if (mode != 2) L.gunits[g.cls].push_back(gu);
-          if (mode != 1 && g.cls < 3) L.gunits_bf[g.cls].push_back(gu);
-        }
-        if (nseg > 1) {
-          for (int64_t e0 = 0; e0 < mn; e0 += 256) {
-            RedItem r;
-            r.v_off = vb.v_off;
-            r.p_off = poff;
-            r.nseg = nseg;
-            r.mn = (int32_t)mn;
-            r.e0 = (int32_t)e0;
-            r.len = (int32_t)std::min<int64_t>(256, mn - e0);
-            if (mode != 2) L.reds[0].push_back(r);
-            if (mode != 1) L.reds[1].push_back(r);
-          }
-          poff += nseg * mn;
-        }
-      };
-      const int nfast = (int)fast.size();
-      if (wave_vb) {
-        emit(gm, 1, nfast, 2);
-        emit(gs, 2, 0, 0);
-      } else if (gm.code == gs.code && gm.nv == gs.nv) {
-        emit(gm, 0, nfast, 1);
-      } else {
-        emit(gm, 1, nfast, 1);
-        emit(gs, 2, nfast, 1);
-      }
-      return true;
-    };
-    // ranges of V blocks with about equal pair counts, one per thread
-    int nth = (int)std::min<long>(std::max(1u, std::thread::hardware_concurrency()), 16);
-    if (ch.n_pairs < 20000) nth = 1;
-    nth = std::max(1, std::min(nth, ch.n_vblocks));
-    std::vector<int> bounds(nth + 1, ch.n_vblocks);
-    bounds[0] = 0;
-    {
-      int64_t acc = 0, tot = 0;
-      for (int i = 0; i < ch.n_vblocks; ++i) tot += std::max(0, ch.vblocks[i].count) + 1;
-      int t = 1;
-      for (int i = 0; i < ch.n_vblocks && t < nth; ++i) {
-        acc += std::max(0, ch.vblocks[i].count) + 1;
-        if (acc * nth >= tot * t) bounds[t++] = i + 1;
-      }
+          vb.count < 0 || vb.first + (int64_t)vb.count > ch.n_pairs)
+        return cleanup(BSG_ERR_ARG, "bsg_plan_create: vblock out of range");
+      pc.h_base[i] = (int32_t)np;
+      np += vb.count;
     }
-    std::vector<Local> loc(nth);
-    auto work = [&](int t) {
-      for (int i = bounds[t]; i < bounds[t + 1]; ++i)
-        if (!plan_vblock(i, loc[t])) return;
+    if (np > 0x7fffffff) return cleanup(BSG_ERR_ARG, "bsg_plan_create: too many pairs");
+    pc.n_pairs = np;
+    pc.h_perm.reset(new bsg_pair_t[std::max<int64_t>(1, np)]);
+    // the V blocks' pairs in device order: the small-block (per-wave)
+    // kernel's ones, then the rest
+    struct Local {
+      int64_t arena_extent = 0;
+      double flops = 0.0, flops1 = 0.0, flops2 = 0.0, flops_split = 0.0;
+      bool bad = false;
+      std::vector<bsg_pair_t> rest;
     };
-    if (nth == 1) {
-      work(0);
-    } else {
-      std::vector<std::thread> th;
-      for (int t = 1; t < nth; ++t) th.emplace_back(work, t);
-      work(0);
-      for (auto& x : th) x.join();
-    }
-    for (auto& L : loc)
-      if (!L.err.empty()) return cleanup(BSG_ERR_ARG, L.err);
-    // concatenate with the local indices shifted
-    std::vector<GUnit> gunits[NCLS], gunits_bf[3];
-    std::vector<bsg_pair_t> perm;
-    std::vector<std::pair<long, int>> sunits[2];
-    std::vector<GUnit> wunits[2];
-    std::vector<Seg> segs;
-    std::vector<RedItem> reds[2];
-    int64_t poff = 0;
-    for (auto& L : loc) {
-      const int pb = (int)perm.size(), sb = (int)segs.size();
-      const int64_t ob = poff;
+    std::vector<Local> loc(MAX_PLAN_THREADS);
+    const int nth = over_vblocks(ch.vblocks, ch.n_vblocks, np, [&](int t, int i0, int i1) {
+      Local& L = loc[t];
+      for (int i = i0; i < i1; ++i) {
+        const bsg_vblock_t& vb = ch.vblocks[i];
+        const bool sm = small_block(vb), wave_vb = !sm && fp64_rule(*p->rules, vb.m, vb.n) == wave_candidate();
+        bsg_pair_t* to = pc.h_perm.get() + pc.h_base[i];
+        L.rest.clear();
+        int nf = 0;
+        for (int q = 0; q < vb.count; ++q) {
+          const bsg_pair_t& pr = ch.pairs[vb.first + q];
+          if (pr.k1 <= 0 || pr.k2 <= 0 || pr.c_off < 0 || pr.c_off + (int64_t)pr.k1 * pr.k2 > wave_size ||
+              (pr.a_off < 0 && pr.k1 != vb.m) || (pr.b_off < 0 && pr.k2 != vb.n)) {
+            L.bad = true;
+            return;
+          }
+          double f1 = 0.0, f2 = 0.0;
+          if (pr.a_off >= 0) {
+            L.arena_extent = std::max(L.arena_extent, pr.a_off + (int64_t)vb.m * pr.k1);
+            f1 = 2.0 * vb.m * pr.k1 * pr.k2;
+          }
+          if (pr.b_off >= 0) {
+            L.arena_extent = std::max(L.arena_extent, pr.b_off + (int64_t)vb.n * pr.k2);
+            f2 = 2.0 * vb.m * pr.k2 * vb.n;
+          }
+          L.flops += f1 + f2;
+          L.flops1 += f1;
+          L.flops2 += f2;
+          const bool f = sm ? small_pair(pr) : wave_vb && (pr.a_off < 0 || pr.k1 <= 4 * wave_ka(wave_nb(vb.n)));
+          if (!f || wave_vb) L.flops_split += f1 + f2;  // split mode: every pair of a per-wave block runs on BF16 slices
+          if (f)
+            to[nf++] = pr;
+          else
+            L.rest.push_back(pr);
+        }
+        std::copy(L.rest.begin(), L.rest.end(), to + nf);
+        pc.h_fast[i] = nf;
+      }
+    });
+    for (int t = 0; t < nth; ++t) {
+      const Local& L = loc[t];
+      if (L.bad) return cleanup(BSG_ERR_ARG, "bsg_plan_create: pair out of range");
       p->flops += L.flops;
       p->flops1 += L.flops1;
       p->flops2 += L.flops2;
       p->flops_split += L.flops_split;
       p->arena_extent = std::max(p->arena_extent, L.arena_extent);
-      perm.insert(perm.end(), L.perm.begin(), L.perm.end());
-      pc.h_vbi.insert(pc.h_vbi.end(), L.h_vbi.begin(), L.h_vbi.end());
-      for (Seg sg : L.segs) {
-        sg.first += pb;
-        if (sg.p_off >= 0) sg.p_off += ob;
-        segs.push_back(sg);
-      }
-      for (int k = 0; k < 2; ++k)
-        for (auto x : L.sunits[k]) sunits[k].push_back({x.first, x.second + sb});
-      for (int k = 0; k < 2; ++k)
-        for (GUnit g : L.wunits[k]) {
-          g.seg += sb;
-          wunits[k].push_back(g);
-        }
-      for (int k = 0; k < NCLS; ++k)
-        for (GUnit g : L.gunits[k]) {
-          g.seg += sb;
-          gunits[k].push_back(g);
-        }
-      for (int k = 0; k < 3; ++k)
-        for (GUnit g : L.gunits_bf[k]) {
-          g.seg += sb;
-          gunits_bf[k].push_back(g);
-        }
-      for (int k = 0; k < 2; ++k)
-        for (RedItem r : L.reds[k]) {
-          r.p_off += ob;
-          reds[k].push_back(r);
-        }
-      poff += L.poff;
     }
-    pmax = std::max(pmax, poff);
-    // every array of the chunk goes into one device allocation with one copy
-    // (256-byte aligned parts): one hipMalloc / hipFree per chunk
-    std::vector<std::pair<void**, size_t>> parts;  // (device pointer to set, offset in the blob)
-    std::vector<char> blob;
-    blob.reserve(sizeof(bsg_vblock_t) * ch.n_vblocks + sizeof(bsg_pair_t) * perm.size() + sizeof(Seg) * segs.size() +
-                 sizeof(RedItem) * (reds[0].size() + reds[1].size()) +
-                 sizeof(int4) * (sunits[0].size() + sunits[1].size() + 8) / 4 + (1 << 16));
-    auto up = [&](void** d, const void* h, size_t bytes) {
-      if (bytes == 0) return;
-      const size_t off = (blob.size() + 255) & ~(size_t)255;
-      blob.resize(off + bytes);
-      std::memcpy(blob.data() + off, h, bytes);
-      parts.push_back({d, off});
-    };
-    up((void**)&pc.d_vb, ch.vblocks, sizeof(bsg_vblock_t) * ch.n_vblocks);
-    up((void**)&pc.d_pr, perm.data(), sizeof(bsg_pair_t) * perm.size());
-    up((void**)&pc.d_seg, segs.data(), sizeof(Seg) * segs.size());
-    up((void**)&pc.d_red[0], reds[0].data(), sizeof(RedItem) * reds[0].size());
-    up((void**)&pc.d_red[1], reds[1].data(), sizeof(RedItem) * reds[1].size());
-    std::vector<TileRef> gtiles[NCLS];
-    for (int k = 0; k < NCLS; ++k) gtiles[k] = xcd_order(gunits[k]);
-    std::vector<TileRef> gtiles_bf[3] = {xcd_order(gunits_bf[0]), xcd_order(gunits_bf[1]), xcd_order(gunits_bf[2])};
-    // small-block units, costliest first, four per workgroup
-    std::vector<int4> sq[2];
-    for (int k = 0; k < 2; ++k) {
-      std::sort(sunits[k].begin(), sunits[k].end(), [](const std::pair<long, int>& x, const std::pair<long, int>& y) {
-        return x.first != y.first ? x.first > y.first : x.second < y.second;
-      });
-      for (size_t i = 0; i < sunits[k].size(); i += 4) {
-        int e[4];
-        for (int j = 0; j < 4; ++j) e[j] = i + j < sunits[k].size() ? sunits[k][i + j].second : -1;
-        sq[k].push_back(make_int4(e[0], e[1], e[2], e[3]));
-      }
-      up((void**)&pc.d_s[k], sq[k].data(), sizeof(int4) * sq[k].size());
-      pc.n_s[k] = (int)sq[k].size();
-    }
-    for (int k = 0; k < NCLS; ++k) {
-      up((void**)&pc.d_g[k], gtiles[k].data(), sizeof(TileRef) * gtiles[k].size());
-      pc.n_g[k] = (int)gtiles[k].size();
-    }
-    // per-wave tiles of each width: units (costliest first) go to the least
-    // loaded of the 8 XCDs, a unit's tiles in consecutive wave slots of that
-    // XCD's workgroups (they share the unit's C and B' blocks in its L2);
-    // workgroup 8 j + x is XCD x's j-th
-    for (int k = 0; k < 2; ++k) {
-      std::vector<std::pair<long, int>> order;
-      for (int u = 0; u < (int)wunits[k].size(); ++u)
-        order.push_back({wunits[k][u].cost * wunits[k][u].ntm * wunits[k][u].ntn, u});
-      std::sort(order.begin(), order.end(), [](const std::pair<long, int>& x, const std::pair<long, int>& y) {
-        return x.first != y.first ? x.first > y.first : x.second < y.second;
-      });
-      std::vector<TileRef> q[8];
-      long load[8] = {};
-      for (const auto& o : order) {
-        const int x = (int)(std::min_element(load, load + 8) - load);
-        const GUnit& gu = wunits[k][o.second];
-        for (int tm = 0; tm < gu.ntm; ++tm)
-          for (int tn = 0; tn < gu.ntn; ++tn) q[x].push_back(TileRef{gu.seg, tm, tn, 0});
-        load[x] += o.first;
-      }
-      size_t nwg = 0;
-      for (auto& e : q) nwg = std::max(nwg, (e.size() + 3) / 4);
-      std::vector<TileRef> wt(nwg * 32, TileRef{-1, 0, 0, 0});
-      for (int x = 0; x < 8; ++x)
-        for (size_t e = 0; e < q[x].size(); ++e) wt[((e / 4) * 8 + x) * 4 + e % 4] = q[x][e];
-      up((void**)&pc.d_w[k], wt.data(), sizeof(TileRef) * wt.size());
-      pc.n_w[k] = (int)wt.size();
-    }
-    for (int k = 0; k < 3; ++k) {
-      up((void**)&pc.d_gbf[k], gtiles_bf[k].data(), sizeof(TileRef) * gtiles_bf[k].size());
-      pc.n_gbf[k] = (int)gtiles_bf[k].size();
-    }
-    if (!blob.empty()) {
+    if (np > 0) {
+      const size_t pb = (sizeof(bsg_pair_t) * np + 255) & ~(size_t)255;
       char* d = nullptr;
-      if (hipMalloc((void**)&d, blob.size()) != hipSuccess ||
-          hipMemcpy(d, blob.data(), blob.size(), hipMemcpyHostToDevice) != hipSuccess) {
-        (void)hipFree(d);
-        p->chunks.push_back(std::move(pc));
+      if (hipMalloc((void**)&d, pb + sizeof(bsg_vblock_t) * ch.n_vblocks) != hipSuccess)
         return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: plan arrays");
-      }
       pc.d_blob = d;
-      for (auto& x : parts) *x.first = d + x.second;
+      pc.d_pr = (bsg_pair_t*)d;
+      pc.d_vb = (bsg_vblock_t*)(d + pb);
+      if (hipMemcpy(pc.d_pr, pc.h_perm.get(), sizeof(bsg_pair_t) * np, hipMemcpyHostToDevice) != hipSuccess ||
+          hipMemcpy(pc.d_vb, ch.vblocks, sizeof(bsg_vblock_t) * ch.n_vblocks, hipMemcpyHostToDevice) != hipSuccess)
+        return cleanup(BSG_ERR_HIP, "bsg_plan_create: plan arrays");
     }
-    pc.n_red[0] = (int)reds[0].size();
-    pc.n_red[1] = (int)reds[1].size();
-    pc.h_perm = std::move(perm);
-    pc.h_vb.assign(ch.vblocks, ch.vblocks + ch.n_vblocks);
-    p->chunks.push_back(std::move(pc));
+    if (plan_lists(p, pc, false) != BSG_OK) return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: plan arrays");
   }
-  p->part_doubles = pmax;
-  if (pmax > 0) {
-    hipError_t e = hipMalloc(&p->part, sizeof(double) * pmax * p->batch);
-    if (e != hipSuccess) return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: partial-tile scratch");
-  }
+  for (const PlanChunk& pc : p->chunks) p->part_doubles[0] = std::max(p->part_doubles[0], pc.ml[0].part_doubles);
+  if (p->part_doubles[0] > 0 && hipMalloc(&p->part[0], sizeof(double) * p->part_doubles[0]) != hipSuccess)
+    return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: partial-tile scratch");
+  if (p->w_doubles > 0 && !(p->wscratch = w_scratch(ctx, p->w_doubles)))
+    return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: W scratch");
   *plan = p;
   return BSG_OK;
 }
@@ -2199,10 +2508,11 @@ int bsg_plan_destroy(bsg_plan* p) {
   if (!p) return BSG_OK;
   if (p->ctx) (void)hipStreamSynchronize(p->ctx->stream);
   for (auto& c : p->chunks) {
-    (void)hipFree(c.d_blob);  // every array but the lazily built slice offsets
+    (void)hipFree(c.d_blob);
     (void)hipFree(c.d_ps);
+    for (auto& ml : c.ml) (void)hipFree(ml.d_blob);
   }
-  (void)hipFree(p->part);
+  for (double* x : p->part) (void)hipFree(x);
   (void)hipFree(p->d_ab_items);
   (void)hipFree(p->d_c_items);
   if (p->abs_from_ctx)
@@ -2216,7 +2526,7 @@ int bsg_plan_destroy(bsg_plan* p) {
 }
 
 int64_t bsg_plan_arena_extent(const bsg_plan* p) { return p ? p->arena_extent : 0; }
-int64_t bsg_plan_partial_doubles(const bsg_plan* p) { return p ? p->part_doubles : 0; }
+int64_t bsg_plan_partial_doubles(const bsg_plan* p) { return p ? std::max(p->part_doubles[0], p->part_doubles[1]) : 0; }
 
 }  // extern "C"
 
@@ -2273,9 +2583,15 @@ int build_slices(bsg_plan* p) {
   // superblock are referenced once) and its item list reserved likewise;
   // the C blocks are few (one per wavefunction block)
   size_t n_ab = 0;
+  // f(pair index, V block) for every pair that reads slices: all but the
+  // small-block kernel's
+  auto sliced = [](const PlanChunk& pc, auto f) {
+    for (size_t i = 0; i < pc.h_vb.size(); ++i)
+      for (int64_t j = pc.h_base[i] + (small_block(pc.h_vb[i]) ? pc.h_fast[i] : 0); j < pc.h_base[i] + pc.h_vb[i].count; ++j)
+        f(j, pc.h_vb[i]);
+  };
   for (auto& pc : p->chunks)
-    for (size_t j = 0; j < pc.h_perm.size(); ++j)
-      if (pc.h_vbi[j] >= 0) n_ab += (pc.h_perm[j].a_off >= 0) + (pc.h_perm[j].b_off >= 0);
+    sliced(pc, [&](int64_t j, const bsg_vblock_t&) { n_ab += (pc.h_perm[j].a_off >= 0) + (pc.h_perm[j].b_off >= 0); });
   SliceTable abt(n_ab), ct(0);
   p->ab_items.reserve(n_ab);
   auto slice_of = [&](std::vector<SliceItem>& items, int64_t& elems, int64_t src, int rows, int cols, int trans) {
@@ -2299,17 +2615,15 @@ int build_slices(bsg_plan* p) {
     return ct.get(off, 0, [&] { return slice_of(p->c_items, p->c_elems, off, k2, k1, 1); });
   };
   for (auto& pc : p->chunks) {
-    std::vector<PairS> ps(pc.h_perm.size(), PairS{-1, -1, -1});
-    for (size_t j = 0; j < pc.h_perm.size(); ++j) {
-      if (pc.h_vbi[j] < 0) continue;
-      const bsg_vblock_t& vb = pc.h_vb[pc.h_vbi[j]];
+    std::vector<PairS> ps(pc.n_pairs, PairS{-1, -1, -1});
+    sliced(pc, [&](int64_t j, const bsg_vblock_t& vb) {
       const bsg_pair_t& pr = pc.h_perm[j];
       if (pr.a_off >= 0) {
         ps[j].a = ab_slice(pr.a_off, pr.a_trans, vb.m, pr.k1);  // op(A)(i, p), K = p contiguous
         ps[j].c = c_slice(pr.c_off, pr.k1, pr.k2);
       }
       if (pr.b_off >= 0) ps[j].b = ab_slice(pr.b_off, pr.b_trans ? 0 : 1, vb.n, pr.k2);  // B'(k, col) as [col][k]
-    }
+    });
     if (!ps.empty()) {
       HIPCHK(hipMalloc((void**)&pc.d_ps, sizeof(PairS) * ps.size()));
       HIPCHK(hipMemcpy(pc.d_ps, ps.data(), sizeof(PairS) * ps.size(), hipMemcpyHostToDevice));
@@ -2334,6 +2648,17 @@ int bsg_plan_split_arena(bsg_context* ctx, bsg_plan* p, const double* arena, int
   if (p->ctx != ctx) return fail(BSG_ERR_ARG, "bsg_plan_split_arena: plan belongs to another context");
   if (n < p->arena_extent) return fail(BSG_ERR_ARG, "bsg_plan_split_arena: arena smaller than the plan's extent");
   HIPCHK(hipSetDevice(ctx->device));
+  // FP64-only plans (the rotations, FP64 solves) never pay for the split
+  // lists and slice recipes
+  for (auto& pc : p->chunks) {
+    if (pc.ml[1].ready) continue;
+    const int rc = plan_lists(p, pc, true);
+    if (rc != BSG_OK) return rc;
+    p->part_doubles[1] = std::max(p->part_doubles[1], pc.ml[1].part_doubles);
+  }
+  if (!p->part[1] && p->part_doubles[1] > 0 &&
+      hipMalloc(&p->part[1], sizeof(double) * p->part_doubles[1] * p->batch) != hipSuccess)
+    return fail(BSG_ERR_NOMEM, "bsg_plan_split_arena: partial-tile scratch");
   if (!p->slices_built) {
     const int rc = build_slices(p);
     if (rc != BSG_OK) return rc;
@@ -2383,8 +2708,10 @@ int bsg_set_tile_table(const int32_t* rules, int32_t n) {
       return fail(BSG_ERR_ARG, "bsg_set_tile_table: bad rule");
     t.push_back(r);
   }
-  g_tile_rules = t;
-  ++g_tile_version;
+  auto rs = std::make_shared<RuleSet>();
+  rs->rules = t;
+  rs->version = g_tile_rules->version + 1;
+  g_tile_rules = rs;
   return BSG_OK;
 }
 int bsg_tile_candidates(int32_t precision) {
@@ -2402,17 +2729,32 @@ int bsg_plan_set_batch(bsg_context* ctx, bsg_plan* p, int32_t nroot) {
     HIPCHK(hipGraphExecDestroy(p->graph));
     p->graph = nullptr;
   }
-  if (p->part_doubles > 0) {
-    double* np = nullptr;
-    if (hipMalloc(&np, sizeof(double) * p->part_doubles * nroot) != hipSuccess)
-      return fail(BSG_ERR_NOMEM, "bsg_plan_set_batch: partial-tile scratch");
-    (void)hipFree(p->part);
-    p->part = np;
+  // the rounds of large blocks take as many roots per launch as W_ROOTS
+  // doubles of scratch hold
+  const int32_t wroots =
+      (int32_t)std::max<int64_t>(1, std::min<int64_t>(nroot, W_ROOTS / std::max<int64_t>(1, p->w_doubles)));
+  // every new buffer before any old one goes: a failure leaves the plan as it was
+  double* np[2] = {};
+  std::shared_ptr<WScratch> nw;
+  __bf16* nc = nullptr;
+  const bool cs = p->cs_ready && p->c_elems > 0, wn = p->w_doubles > 0 && wroots != p->wroots;
+  if ((p->part[0] && hipMalloc(&np[0], sizeof(double) * p->part_doubles[0] * nroot) != hipSuccess) ||
+      (p->part[1] && hipMalloc(&np[1], sizeof(double) * p->part_doubles[1] * nroot) != hipSuccess) ||
+      (wn && !(nw = w_scratch(ctx, p->w_doubles * wroots))) ||
+      (cs && hipMalloc((void**)&nc, 2 * p->c_elems * nroot) != hipSuccess)) {
+    for (double* x : np) (void)hipFree(x);
+    return fail(BSG_ERR_NOMEM, "bsg_plan_set_batch: scratch of the roots");
   }
-  if (p->cs_ready && p->c_elems > 0) {
-    __bf16* nc = nullptr;
-    if (hipMalloc((void**)&nc, 2 * p->c_elems * nroot) != hipSuccess)
-      return fail(BSG_ERR_NOMEM, "bsg_plan_set_batch: wavefunction slices");
+  for (int k = 0; k < 2; ++k)
+    if (np[k]) {
+      (void)hipFree(p->part[k]);
+      p->part[k] = np[k];
+    }
+  if (nw) {
+    p->wscratch = nw;
+    p->wroots = wroots;
+  }
+  if (nc) {
     (void)hipFree(p->d_cs);
     p->d_cs = nc;
   }
@@ -2440,82 +2782,114 @@ namespace {
 int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, const double* arena, const double* c,
                   double* v, hipEvent_t* ev, bool split, double* part, const RootSet& rs, long* launches = nullptr) {
   hipStream_t st = ctx->stream;
+  const ModeLists& ml = ch.ml[split];
   auto grid = [&](int n) { return dim3((unsigned)(((n + 7) / 8) * 8 * rs.n)); };
   long nl = 0;
   if (ev) HIPCHK(hipEventRecord(ev[0], st));
   // the side stream runs the small-block kernel and the basic tiles beside
   // the wide tiles on the context stream; they write disjoint V blocks and
   // partial tiles, and the reduction waits for both
-  const int nbasic = split ? ch.n_gbf[0] : ch.n_g[0];
-  const bool side = ch.n_s[0] > 0 || ch.n_s[1] > 0 || nbasic > 0;
+  const int nbasic = ml.n_g[0];
+  const int *ns = ml.n_s;
+  const bool side = ns[0] > 0 || ns[1] > 0 || nbasic > 0 || ml.n_p[0] > 0 || ml.rounds.size() > 1;
+  // round r of the large blocks, in launches of the roots its scratch holds
+  auto round = [&](size_t r, hipStream_t q) {
+    const GemmRound& g = ml.rounds[r];
+    for (int r0 = 0; r0 < rs.n; r0 += p->wroots) {
+      RootSet sub = rs;
+      sub.n = std::min(p->wroots, rs.n - r0);
+      const double* cr = c + r0 * rs.wstride;
+      double *vr = v + r0 * rs.wstride, *pr = part + r0 * rs.pstride;
+      auto tiles = [&](const TileRef* t, int n) {
+        if (n == 0) return;
+        hipLaunchKernelGGL((k_gemm<GemmT>), dim3((unsigned)(((n + 7) / 8) * 8 * sub.n)), dim3(GemmT::NT), 0, q, ml.d_gu,
+                           ml.d_gs, ml.d_ga, t, n, arena, cr, vr, p->wscratch ? p->wscratch->ptr : nullptr, pr, sub);
+        ++nl;
+      };
+      tiles(g.d_w, g.n_w);
+      tiles(g.d_v, g.n_v);
+    }
+  };
   if (side) {
     HIPCHK(hipEventRecord(ctx->fork, st));
     HIPCHK(hipStreamWaitEvent(ctx->side, ctx->fork, 0));
     if (ev) HIPCHK(hipEventRecord(ev[1], ctx->side));
-    if (ch.n_s[0] > 0) {
-      hipLaunchKernelGGL((k_small<2>), grid(ch.n_s[0]), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ch.d_seg, ch.d_s[0],
-                         ch.n_s[0], arena, c, v, part, rs);
+    for (size_t r = 1; r < ml.rounds.size(); r += 2) round(r, ctx->side);
+    if (ml.n_p[0] > 0) {
+      hipLaunchKernelGGL((k_panel<3>), grid(ml.n_p[0]), dim3(256), 0, ctx->side, ch.d_vb, ml.d_pp, ml.d_seg, ml.d_p[0],
+                         ml.n_p[0], arena, c, v, part, rs);
       ++nl;
     }
-    if (ch.n_s[1] > 0) {
-      hipLaunchKernelGGL((k_small<1>), grid(ch.n_s[1]), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ch.d_seg, ch.d_s[1],
-                         ch.n_s[1], arena, c, v, part, rs);
+    if (ns[0] > 0) {
+      hipLaunchKernelGGL((k_small<2>), grid(ns[0]), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ml.d_seg,
+                         ml.d_s[0], ns[0], arena, c, v, part, rs);
+      ++nl;
+    }
+    if (ns[1] > 0) {
+      hipLaunchKernelGGL((k_small<1>), grid(ns[1]), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ml.d_seg,
+                         ml.d_s[1], ns[1], arena, c, v, part, rs);
       ++nl;
     }
     if (nbasic > 0) {
       if (split)
         hipLaunchKernelGGL((k_sigma_bf<2, 2>), grid(nbasic), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ch.d_ps,
-                           ch.d_seg, ch.d_gbf[0], nbasic, p->d_abs, p->d_cs, c, v, part, rs);
+                           ml.d_seg, ml.d_g[0], nbasic, p->d_abs, p->d_cs, c, v, part, rs);
       else
-        hipLaunchKernelGGL((k_sigma<2, 2>), grid(nbasic), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ch.d_seg,
-                           ch.d_g[0], nbasic, arena, c, v, part, rs);
+        hipLaunchKernelGGL((k_sigma<2, 2>), grid(nbasic), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ml.d_seg,
+                           ml.d_g[0], nbasic, arena, c, v, part, rs);
       ++nl;
     }
     if (ev) HIPCHK(hipEventRecord(ev[2], ctx->side));
     HIPCHK(hipEventRecord(ctx->join, ctx->side));
   }
   if (split) {
-    if (ch.n_gbf[2] > 0) {
-      hipLaunchKernelGGL((k_sigma_bf<1, 4, 8>), grid(ch.n_gbf[2]), dim3(512), 0, st, ch.d_vb, ch.d_pr, ch.d_ps,
-                         ch.d_seg, ch.d_gbf[2], ch.n_gbf[2], p->d_abs, p->d_cs, c, v, part, rs);
+    if (ml.n_g[2] > 0) {
+      hipLaunchKernelGGL((k_sigma_bf<1, 4, 8>), grid(ml.n_g[2]), dim3(512), 0, st, ch.d_vb, ch.d_pr, ch.d_ps,
+                         ml.d_seg, ml.d_g[2], ml.n_g[2], p->d_abs, p->d_cs, c, v, part, rs);
       ++nl;
     }
-    if (ch.n_gbf[1] > 0) {
-      hipLaunchKernelGGL((k_sigma_bf<1, 4>), grid(ch.n_gbf[1]), dim3(256), 0, st, ch.d_vb, ch.d_pr, ch.d_ps, ch.d_seg,
-                         ch.d_gbf[1], ch.n_gbf[1], p->d_abs, p->d_cs, c, v, part, rs);
+    if (ml.n_g[1] > 0) {
+      hipLaunchKernelGGL((k_sigma_bf<1, 4>), grid(ml.n_g[1]), dim3(256), 0, st, ch.d_vb, ch.d_pr, ch.d_ps, ml.d_seg,
+                         ml.d_g[1], ml.n_g[1], p->d_abs, p->d_cs, c, v, part, rs);
       ++nl;
     }
   } else {
-    if (ch.n_w[1] > 0) {
-      hipLaunchKernelGGL((k_wave<4>), grid(ch.n_w[1] / 4), dim3(256), 0, st, ch.d_vb, ch.d_pr, ch.d_seg, ch.d_w[1],
-                         ch.n_w[1], arena, c, v, part, rs);
+    for (size_t r = 0; r < ml.rounds.size(); r += 2) round(r, st);
+    if (ml.n_p[1] > 0) {
+      hipLaunchKernelGGL((k_panel<5>), grid(ml.n_p[1]), dim3(256), 0, st, ch.d_vb, ml.d_pp, ml.d_seg, ml.d_p[1],
+                         ml.n_p[1], arena, c, v, part, rs);
       ++nl;
     }
-    if (ch.n_w[0] > 0) {
-      hipLaunchKernelGGL((k_wave<2>), grid(ch.n_w[0] / 4), dim3(256), 0, st, ch.d_vb, ch.d_pr, ch.d_seg, ch.d_w[0],
-                         ch.n_w[0], arena, c, v, part, rs);
+    if (ml.n_w[1] > 0) {
+      hipLaunchKernelGGL((k_wave<4>), grid(ml.n_w[1] / 4), dim3(256), 0, st, ch.d_vb, ch.d_pr, ml.d_seg, ml.d_w[1],
+                         ml.n_w[1], arena, c, v, part, rs);
       ++nl;
     }
-    if (ch.n_g[3] > 0) {
-      hipLaunchKernelGGL((k_sigma<1, 6, PB, 8>), grid(ch.n_g[3]), dim3(512), 0, st, ch.d_vb, ch.d_pr, ch.d_seg,
-                         ch.d_g[3], ch.n_g[3], arena, c, v, part, rs);
+    if (ml.n_w[0] > 0) {
+      hipLaunchKernelGGL((k_wave<2>), grid(ml.n_w[0] / 4), dim3(256), 0, st, ch.d_vb, ch.d_pr, ml.d_seg, ml.d_w[0],
+                         ml.n_w[0], arena, c, v, part, rs);
       ++nl;
     }
-    if (ch.n_g[2] > 0) {
-      hipLaunchKernelGGL((k_sigma<1, 6>), grid(ch.n_g[2]), dim3(256), 0, st, ch.d_vb, ch.d_pr, ch.d_seg, ch.d_g[2],
-                         ch.n_g[2], arena, c, v, part, rs);
+    if (ml.n_g[3] > 0) {
+      hipLaunchKernelGGL((k_sigma<1, 6, PB, 8>), grid(ml.n_g[3]), dim3(512), 0, st, ch.d_vb, ch.d_pr, ml.d_seg,
+                         ml.d_g[3], ml.n_g[3], arena, c, v, part, rs);
       ++nl;
     }
-    if (ch.n_g[1] > 0) {
-      hipLaunchKernelGGL((k_sigma<1, 4>), grid(ch.n_g[1]), dim3(256), 0, st, ch.d_vb, ch.d_pr, ch.d_seg, ch.d_g[1],
-                         ch.n_g[1], arena, c, v, part, rs);
+    if (ml.n_g[2] > 0) {
+      hipLaunchKernelGGL((k_sigma<1, 6>), grid(ml.n_g[2]), dim3(256), 0, st, ch.d_vb, ch.d_pr, ml.d_seg, ml.d_g[2],
+                         ml.n_g[2], arena, c, v, part, rs);
+      ++nl;
+    }
+    if (ml.n_g[1] > 0) {
+      hipLaunchKernelGGL((k_sigma<1, 4>), grid(ml.n_g[1]), dim3(256), 0, st, ch.d_vb, ch.d_pr, ml.d_seg, ml.d_g[1],
+                         ml.n_g[1], arena, c, v, part, rs);
       ++nl;
     }
   }
   if (side) HIPCHK(hipStreamWaitEvent(st, ctx->join, 0));
   if (ev) HIPCHK(hipEventRecord(ev[3], st));
-  if (ch.n_red[split] > 0) {
-    hipLaunchKernelGGL(k_reduce, dim3(ch.n_red[split], rs.n), dim3(256), 0, st, ch.d_red[split], part, v, rs);
+  if (ml.n_red > 0) {
+    hipLaunchKernelGGL(k_reduce, dim3(ml.n_red, rs.n), dim3(256), 0, st, ml.d_red, part, v, rs);
     ++nl;
   }
   if (ev) HIPCHK(hipEventRecord(ev[4], st));
@@ -2527,7 +2901,7 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
 int check_precision(const bsg_plan* p, const double* arena, int32_t precision) {
   if (precision == BSG_FP64) return BSG_OK;
   if (precision != BSG_SPLIT_BF16) return fail(BSG_ERR_ARG, "unknown precision mode");
-  if (p->split_src != arena || !p->slices_built || (p->ab_elems > 0 && !p->d_abs) || (p->c_elems > 0 && !p->d_cs))
+  if (p->split_src != arena || !p->slices_built || (p->part_doubles[1] > 0 && !p->part[1]) || (p->ab_elems > 0 && !p->d_abs) || (p->c_elems > 0 && !p->d_cs))
     return fail(BSG_ERR_ARG, "split precision needs bsg_plan_split_arena on this arena first");
   return BSG_OK;
 }
@@ -2547,8 +2921,9 @@ int sigma_apply_with(bsg_context* ctx, bsg_plan* p, const double* arena, const d
     rs.n = std::min(group, nvec - iv);
     rs.pad = 0;
     rs.wstride = p->wave_size;
-    rs.pstride = p->part_doubles;
+    rs.pstride = p->part_doubles[split];
     rs.cstride = p->c_elems;
+    rs.tstride = p->w_doubles;
     const double* cv = c + (size_t)iv * p->wave_size;
     double* vv = v + (size_t)iv * p->wave_size;
     if (split && !p->c_items.empty()) {
@@ -2571,7 +2946,7 @@ int bsg_sigma_apply(bsg_context* ctx, bsg_plan* p, const double* arena, const do
                     int32_t precision) {
   if (!ctx || !p || !arena || !c || !v || nvec <= 0) return fail(BSG_ERR_ARG, "bsg_sigma_apply: bad args");
   if (p->ctx != ctx) return fail(BSG_ERR_ARG, "bsg_sigma_apply: plan belongs to another context");
-  return sigma_apply_with(ctx, p, arena, c, v, nvec, precision, p->part, p->batch);
+  return sigma_apply_with(ctx, p, arena, c, v, nvec, precision, p->part[precision == BSG_SPLIT_BF16], p->batch);
 }
 
 int bsg_plan_capture(bsg_context* ctx, bsg_plan* p, const double* arena, const double* c, double* v, int32_t nvec,
@@ -2591,7 +2966,7 @@ int bsg_plan_capture(bsg_context* ctx, bsg_plan* p, const double* arena, const d
   // joins through the fork/join events and is captured with it); no memset
   // or allocation is recorded
   HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-  rc = sigma_apply_with(ctx, p, arena, c, v, nvec, precision, p->part, p->batch);
+  rc = sigma_apply_with(ctx, p, arena, c, v, nvec, precision, p->part[precision == BSG_SPLIT_BF16], p->batch);
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(ctx->stream, &g);
   if (rc) {
@@ -2627,13 +3002,13 @@ int bsg_sigma_apply_noalloc(bsg_context* ctx, bsg_plan* p, const double* arena, 
   if (!ctx || !p || !arena || !c || !v || nvec <= 0) return fail(BSG_ERR_ARG, "bsg_sigma_apply_noalloc: bad args");
   if (p->ctx != ctx) return fail(BSG_ERR_ARG, "bsg_sigma_apply_noalloc: plan belongs to another context");
   if (!ctx->scratch) return fail(BSG_ERR_ARG, "bsg_sigma_apply_noalloc: no scratch address for this device");
-  if (p->part_doubles > BSG_NOALLOC_SCRATCH_DOUBLES)
-    return fail(BSG_ERR_ARG, "bsg_sigma_apply_noalloc: the plan needs " + std::to_string(p->part_doubles) +
+  const int64_t need = p->part_doubles[precision == BSG_SPLIT_BF16];
+  if (need > BSG_NOALLOC_SCRATCH_DOUBLES)
+    return fail(BSG_ERR_ARG, "bsg_sigma_apply_noalloc: the plan needs " + std::to_string(need) +
                                  " doubles of partial tiles, more than the " +
                                  std::to_string((long long)BSG_NOALLOC_SCRATCH_DOUBLES) + " of the static scratch");
   // as many roots per launch as the scratch holds partial tiles for
-  const int group = p->part_doubles > 0 ? (int)std::min<int64_t>(p->batch, BSG_NOALLOC_SCRATCH_DOUBLES / p->part_doubles)
-                                        : p->batch;
+  const int group = need > 0 ? (int)std::min<int64_t>(p->batch, BSG_NOALLOC_SCRATCH_DOUBLES / need) : p->batch;
   return sigma_apply_with(ctx, p, arena, c, v, nvec, precision, ctx->scratch, group);
 }
 
@@ -2652,7 +3027,7 @@ int bsg_sigma_profile(bsg_context* ctx, bsg_plan* p, const double* arena, const 
   long disp = 0;
   HIPCHK(hipEventRecord(ev[0], ctx->stream));
   for (int r = 0; r < reps; ++r)
-    if ((rc = sigma_apply_with(ctx, p, arena, c, v, nvec, precision, p->part, p->batch, &disp,
+    if ((rc = sigma_apply_with(ctx, p, arena, c, v, nvec, precision, p->part[precision == BSG_SPLIT_BF16], p->batch, &disp,
                                &ev[1 + (size_t)r * ngroups * nch * per])))
       return rc;
   const size_t q = 1 + (size_t)reps * ngroups * nch * per;
@@ -2668,11 +3043,12 @@ int bsg_sigma_profile(bsg_context* ctx, bsg_plan* p, const double* arena, const 
   size_t k = 1;
   for (int r = 0; r < reps * ngroups; ++r)
     for (auto& ch : p->chunks) {
-      const bool sidek = ch.n_s[0] > 0 || ch.n_s[1] > 0 || (split ? ch.n_gbf[0] : ch.n_g[0]) > 0;
+      const ModeLists& ml = ch.ml[split];
+      const bool sidek = ml.n_s[0] > 0 || ml.n_s[1] > 0 || ml.n_g[0] > 0 || ml.n_p[0] > 0 || ml.rounds.size() > 1;
       // [0] fork to join of all fused kernels, [1] reduction, [2] the side
       // stream's kernels alone
       const int from[3] = {0, 3, 1}, to[3] = {3, 4, 2};
-      const bool present[3] = {true, ch.n_red[split] > 0, sidek};
+      const bool present[3] = {true, ml.n_red > 0, sidek};
       for (int i = 0; i < 3; ++i) {
         if (!present[i]) continue;
         HIPCHK(hipEventElapsedTime(&ms, ev[k + from[i]], ev[k + to[i]]));

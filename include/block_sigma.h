@@ -137,9 +137,10 @@ int bsg_plan_split_arena(bsg_context* ctx, bsg_plan* plan, const double* arena, 
 
 /* Measured tile choices (no counterpart in the reference): n rules of six
  * int32 (m_lo, m_hi, n_lo, n_hi, fp64, split); a V block of m x n inside a
- * rule's ranges gets tile geometry number fp64 (FP64 kernels) or split
- * (split-precision kernels) of the candidate list, -1 leaving the MFMA-count
- * model's choice; the first matching rule applies.  Process-wide, read when
+ * rule's ranges gets tile geometry number fp64 (FP64 grouped kernel) or split
+ * (split-precision kernels) of the candidate list, -1 leaving the default (FP64:
+ * panels for blocks and contraction depths up to 80, product tiles above;
+ * split: the MFMA-count model's geometry); the first matching rule applies.  Process-wide, read when
  * plans are created (n = 0 clears).  bsg_tile_candidates gives the list's
  * length for a precision.  For FP64 its last entry is not a geometry but the
  * per-wave tile kernel (one wavefront per 16 x 32 V tile, 16 x 64 for blocks
@@ -184,15 +185,18 @@ int bsg_plan_capture(bsg_context* ctx, bsg_plan* plan, const double* arena, cons
 int bsg_plan_replay(bsg_context* ctx, bsg_plan* plan);
 
 /* Doubles of partial-tile scratch one application of the plan uses (V blocks
- * whose pair list is cut into several work units; 0 if none). */
+ * whose pair list is cut into several work units; 0 if none): the larger of
+ * the FP64 application's and, once bsg_plan_split_arena has set it up, the
+ * split one's. */
 int64_t bsg_plan_partial_doubles(const bsg_plan* plan);
 
 /* bsg_sigma_apply without any allocation, for callers that cannot call
  * hipMalloc (code under HIP graph capture, tight serving loops, harnesses
  * that forbid it).  No counterpart in the reference.  The partial tiles live
  * in a static device array of BSG_NOALLOC_SCRATCH_DOUBLES doubles (64 MiB),
- * one per GPU, held until the process ends; a plan whose
- * bsg_plan_partial_doubles exceeds it is rejected with BSG_ERR_ARG.  Results
+ * one per GPU, held until the process ends; an application that needs more
+ * partial tiles is rejected with BSG_ERR_ARG.  The W scratch of large blocks
+ * belongs to the plan (made with it) and its context.  Results
  * are bitwise those of bsg_sigma_apply.  Every call on one GPU shares that
  * GPU's array: calls that overlap on one GPU (other contexts' streams, other
  * threads) race and must be serialised by the caller.  The plan itself (and,
