@@ -1399,73 +1399,8 @@ inline std::vector<TileRef> xcd_order(std::vector<GUnit>& units) {
 }
 
 // ---------------------------------------------------------------- vector kernels
-constexpr int RB = 256, RMAXB = 1024;
+#include "vectors.h"
 
-__global__ __launch_bounds__(RB) void k_dot_partial(const double* __restrict__ x, const double* __restrict__ y,
-                                                    int64_t n, double* __restrict__ part) {
-  __shared__ double sh[RB];
-  double s = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB) s += x[i] * y[i];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = RB / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-__global__ __launch_bounds__(RB) void k_sum_partial(const double* __restrict__ part, int np, double* __restrict__ out) {
-  __shared__ double sh[RB];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < np; i += RB) s += part[i];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = RB / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = sh[0];
-}
-__global__ void k_axpy(double a, const double* __restrict__ x, double* __restrict__ y, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    y[i] += a * x[i];
-}
-__global__ void k_scal(double a, double* __restrict__ x, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    x[i] *= a;
-}
-// the same with the scalar in device memory: x *= 1/sqrt(s[0]) (only if
-// s[0] > floor), y += -s[0] x
-__global__ void k_scal_rsqrt_dev(const double* __restrict__ s, double floor, double* __restrict__ x, int64_t n) {
-  const double n2 = s[0];
-  if (!(n2 > floor)) return;
-  const double a = 1.0 / sqrt(n2);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    x[i] *= a;
-}
-// y -= (num[0] / den[0]) x (Olsen's step with both dot products on the device)
-__global__ void k_axpy_ratio_dev(const double* __restrict__ num, const double* __restrict__ den,
-                                 const double* __restrict__ x, double* __restrict__ y, int64_t n) {
-  const double a = -(num[0] / den[0]);
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    y[i] += a * x[i];
-}
-__global__ void k_axpy_neg_dev(const double* __restrict__ s, const double* __restrict__ x, double* __restrict__ y,
-                               int64_t n) {
-  const double a = -s[0];
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    y[i] += a * x[i];
-}
-__global__ void k_precond(double* __restrict__ x, const double* __restrict__ d, double e, double shift, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    double den = e - d[i];
-    if (fabs(den) > 1e-12) x[i] /= (den + shift);
-  }
-}
-__global__ void k_copy(const double* __restrict__ x, double* __restrict__ y, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    y[i] = x[i];
-}
 // one workgroup per chunk of at most COPY_CHUNK doubles
 constexpr int64_t COPY_CHUNK = 16384;
 __global__ __launch_bounds__(256) void k_copy_chunks(const bsg_copy_seg_t* __restrict__ chunks) {
@@ -1506,79 +1441,6 @@ __global__ __launch_bounds__(256) void k_build(const bsg_build_group_t* __restri
   g.dst[(int64_t)r * g.ld + c] += s;
 }
 
-// Gram matrix tile of two vector sets (mx, my <= GMAX vectors of length n,
-// stride ld): per-block partial sums G[i my + j] = sum_x X_i[x] Y_j[x] over
-// the block's chunks, then an ordered sum over blocks (deterministic).
-// Larger sets (up to GRAM_MAX vectors) run as GMAX x GMAX tiles.
-constexpr int GMAX = 32, GCH = 64, GBLK = 256, GRAM_MAX = 128;
-__global__ __launch_bounds__(256) void k_gram_partial(const double* __restrict__ X, const double* __restrict__ Y, int mx,
-                                                      int my, int64_t n, int64_t ld, double* __restrict__ part) {
-  __shared__ double xs[GMAX][GCH + 1], ys[GMAX][GCH + 1];
-  double acc[GMAX * GMAX / 256];
-  const int npair = mx * my;
-#pragma unroll
-  for (int u = 0; u < GMAX * GMAX / 256; ++u) acc[u] = 0.0;
-  for (int64_t x0 = (int64_t)blockIdx.x * GCH; x0 < n; x0 += (int64_t)gridDim.x * GCH) {
-    for (int e = threadIdx.x; e < GMAX * GCH; e += 256) {
-      const int i = e / GCH, x = e % GCH;
-      const bool ok = x0 + x < n;
-      if (i < mx) xs[i][x] = ok ? X[(int64_t)i * ld + x0 + x] : 0.0;
-      if (i < my) ys[i][x] = ok ? Y[(int64_t)i * ld + x0 + x] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < GMAX * GMAX / 256; ++u) {
-      const int pidx = threadIdx.x + 256 * u;
-      if (pidx < npair) {
-        const int i = pidx / my, j = pidx % my;
-        double s = 0.0;
-        for (int x = 0; x < GCH; ++x) s += xs[i][x] * ys[j][x];
-        acc[u] += s;
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int u = 0; u < GMAX * GMAX / 256; ++u) {
-    const int pidx = threadIdx.x + 256 * u;
-    if (pidx < npair) part[(int64_t)blockIdx.x * npair + pidx] = acc[u];
-  }
-}
-// out[(i) ldo + j] = sum over blocks of the tile's partials (i < mx, j < my)
-__global__ __launch_bounds__(256) void k_gram_sum(const double* __restrict__ part, int nblk, int mx, int my,
-                                                  double* __restrict__ out, int ldo) {
-  const int pidx = blockIdx.x * 256 + threadIdx.x;
-  const int npair = mx * my;
-  if (pidx >= npair) return;
-  double s = 0.0;
-  for (int b = 0; b < nblk; ++b) s += part[(int64_t)b * npair + pidx];
-  out[(int64_t)(pidx / my) * ldo + pidx % my] = s;
-}
-// Y_j[x] (+)= sum_{i < m} coef[i ldc + j] X_i[x] for j < mo (m, mo <= GMAX);
-// accumulate = 0 overwrites Y
-__global__ __launch_bounds__(256) void k_lincomb(const double* __restrict__ X, int m, int64_t n, int64_t ld,
-                                                 const double* __restrict__ coef, int ldc, int mo,
-                                                 double* __restrict__ Y, int64_t ldy, int accumulate) {
-  __shared__ double cs[GMAX * GMAX];
-  for (int e = threadIdx.x; e < m * mo; e += 256) cs[e] = coef[(int64_t)(e / mo) * ldc + e % mo];
-  __syncthreads();
-  for (int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x; x < n; x += (int64_t)gridDim.x * 256) {
-    double xv[GMAX];
-#pragma unroll
-    for (int i = 0; i < GMAX; ++i) xv[i] = i < m ? X[(int64_t)i * ld + x] : 0.0;
-    for (int j = 0; j < mo; ++j) {
-      double s = 0.0;
-#pragma unroll
-      for (int i = 0; i < GMAX; ++i)
-        if (i < m) s += xv[i] * cs[i * mo + j];
-      if (accumulate)
-        Y[(int64_t)j * ldy + x] += s;
-      else
-        Y[(int64_t)j * ldy + x] = s;
-    }
-  }
-}
-
 // diag(H) by V block: item i covers elements [e0, e0 + 256) of the block of
 // its term group; every thread sums the group's terms in list order for its
 // element (alpha_t A_ii B_jj, identity partners read as 1).
@@ -1607,6 +1469,8 @@ __global__ __launch_bounds__(256) void k_diag(const bsg_diag_t* __restrict__ ter
   diag[t0.v_off + e] += s;
 }
 
+// workgroups of a reduction over n elements, two per thread at least
+int reduce_grid(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(RMAXB, (n + 2 * RB - 1) / (2 * RB))); }
 int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(2048, (n + 255) / 256)); }
 
 }  // namespace
@@ -1654,6 +1518,8 @@ struct WScratch {
   ~WScratch() { (void)hipFree(ptr); }  // waits for the device
 };
 
+constexpr int COEF_SLOTS = 4;
+
 struct bsg_context {
   int device = 0;
   std::shared_ptr<WScratch> wscratch;
@@ -1662,12 +1528,16 @@ struct bsg_context {
   // beside the grouped kernel; fork/join events tie it to `stream`
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
-  double* red = nullptr;  // RMAXB partials + 4 result slots
-  double* gpart = nullptr;  // Gram partials (GBLK GMAX^2) + result (GRAM_MAX^2) + coefficients (GRAM_MAX^2)
+  double* red = nullptr;  // two sets of two partial lists (RMAXB each)
+  double* gpart = nullptr;  // Gram partials (GBLK GMAX^2) + coefficient slots (GRAM_MAX^2 each)
   bsg_copy_seg_t* copy_list = nullptr;  // chunk list of bsg_copy_segments (grown on demand)
   size_t copy_cap = 0;
-  double* coef_pin = nullptr;    // page-locked staging of bsg_lincomb's coefficients (GRAM_MAX^2)
-  hipEvent_t coef_done = nullptr;  // its last copy to the device
+  // page-locked staging of bsg_lincomb's coefficients, used in turn (GRAM_MAX^2
+  // each), their last copies to the device, and results (GRAM_MAX^2)
+  double* coef_pin = nullptr;
+  hipEvent_t coef_done[COEF_SLOTS] = {};
+  int coef_next = 0;
+  double* res_pin = nullptr;
   double* scratch = nullptr;  // this device's copy of the static scratch (bsg_sigma_apply_noalloc)
   // operator-slice buffer lent to one split-precision plan at a time (grown
   // on demand), so successive superblocks do not allocate and free it
@@ -1775,13 +1645,13 @@ int bsg_init(bsg_context** ctx, int device) {
     delete c;
     return fail(BSG_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
   }
-  e = hipMalloc(&c->red, sizeof(double) * (RMAXB + 4));
+  e = hipMalloc(&c->red, sizeof(double) * 4 * RMAXB);
   if (e != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     delete c;
     return fail(BSG_ERR_NOMEM, "bsg_init: reduction buffer");
   }
-  if (hipMalloc(&c->gpart, sizeof(double) * ((size_t)GBLK * GMAX * GMAX + 2 * GRAM_MAX * GRAM_MAX)) != hipSuccess) {
+  if (hipMalloc(&c->gpart, sizeof(double) * ((size_t)GBLK * GMAX * GMAX + COEF_SLOTS * GRAM_MAX * GRAM_MAX)) != hipSuccess) {
     (void)hipFree(c->red);
     (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1798,13 +1668,20 @@ int bsg_init(bsg_context** ctx, int device) {
   }
   if (hipStreamCreate(&c->side) != hipSuccess || hipEventCreateWithFlags(&c->fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->join, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->coef_done, hipEventDisableTiming) != hipSuccess ||
-      hipHostMalloc((void**)&c->coef_pin, sizeof(double) * GRAM_MAX * GRAM_MAX, hipHostMallocDefault) != hipSuccess) {
+      [&] {
+        for (hipEvent_t& e : c->coef_done)
+          if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return true;
+        return false;
+      }() ||
+      hipHostMalloc((void**)&c->coef_pin, sizeof(double) * COEF_SLOTS * GRAM_MAX * GRAM_MAX, hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void**)&c->res_pin, sizeof(double) * GRAM_MAX * GRAM_MAX, hipHostMallocDefault) != hipSuccess) {
     if (c->side) (void)hipStreamDestroy(c->side);
     if (c->fork) (void)hipEventDestroy(c->fork);
     if (c->join) (void)hipEventDestroy(c->join);
-    if (c->coef_done) (void)hipEventDestroy(c->coef_done);
+    for (hipEvent_t e : c->coef_done)
+      if (e) (void)hipEventDestroy(e);
     if (c->coef_pin) (void)hipHostFree(c->coef_pin);
+    if (c->res_pin) (void)hipHostFree(c->res_pin);
     (void)hipFree(c->gpart);
     (void)hipFree(c->red);
     (void)hipStreamDestroy(c->stream);
@@ -1826,7 +1703,8 @@ int bsg_free(bsg_context* ctx) {
   HIPCHK(hipFree(ctx->gpart));
   if (ctx->abs_buf) HIPCHK(hipFree(ctx->abs_buf));
   HIPCHK(hipHostFree(ctx->coef_pin));
-  HIPCHK(hipEventDestroy(ctx->coef_done));
+  HIPCHK(hipHostFree(ctx->res_pin));
+  for (hipEvent_t e : ctx->coef_done) HIPCHK(hipEventDestroy(e));
   HIPCHK(hipEventDestroy(ctx->fork));
   HIPCHK(hipEventDestroy(ctx->join));
   HIPCHK(hipStreamDestroy(ctx->side));
@@ -3104,35 +2982,32 @@ int bsg_diag_apply(bsg_context* ctx, const bsg_diag_t* terms, int32_t n, const d
 
 int bsg_dot(bsg_context* ctx, const double* x, const double* y, int64_t n, double* result) {
   if (!ctx || !x || !y || !result || n < 0) return fail(BSG_ERR_ARG, "bsg_dot: bad args");
-  int nb = (int)std::max<int64_t>(1, std::min<int64_t>(RMAXB, (n + RB - 1) / RB));
-  hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(RB), 0, ctx->stream, x, y, n, ctx->red);
-  hipLaunchKernelGGL(k_sum_partial, dim3(1), dim3(RB), 0, ctx->stream, ctx->red, nb, ctx->red + RMAXB);
+  const int nb = reduce_grid(n);
+  hipLaunchKernelGGL(k_dot_partial<false>, dim3(nb), dim3(RB), 0, ctx->stream, x, y, (const double*)nullptr, n, ctx->red);
+  hipLaunchKernelGGL(k_sum_partial, dim3(1), dim3(RB), 0, ctx->stream, ctx->red, nb, ctx->res_pin);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(result, ctx->red + RMAXB, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
+  *result = ctx->res_pin[0];
   return BSG_OK;
 }
 int bsg_gs_orthonormalise(bsg_context* ctx, double* r, const double* B, int32_t m, int64_t ld, int64_t n,
                           int32_t normalise) {
   if (!ctx || !r || n < 0 || m < 0 || (m > 0 && (!B || ld < n))) return fail(BSG_ERR_ARG, "bsg_gs_orthonormalise: bad args");
   if (n == 0) return BSG_OK;
-  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(RMAXB, (n + RB - 1) / RB));
-  double* s = ctx->red + RMAXB;
-  auto dot = [&](const double* x, const double* y) {
-    hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(RB), 0, ctx->stream, x, y, n, ctx->red);
-    hipLaunchKernelGGL(k_sum_partial, dim3(1), dim3(RB), 0, ctx->stream, ctx->red, nb, s);
-  };
-  for (int32_t j = 0; j < m; ++j) {
-    const double* bj = B + (int64_t)j * ld;
-    dot(r, r);
-    hipLaunchKernelGGL(k_scal_rsqrt_dev, dim3(grid_for(n)), dim3(256), 0, ctx->stream, s, -1.0, r, n);
-    dot(r, bj);
-    hipLaunchKernelGGL(k_axpy_neg_dev, dim3(grid_for(n)), dim3(256), 0, ctx->stream, s, bj, r, n);
+  const int nb = reduce_grid(n);
+  double *pin = ctx->red, *pout = ctx->red + 2 * RMAXB;
+  if (m > 0) {
+    hipLaunchKernelGGL(k_dot_partial<true>, dim3(nb), dim3(RB), 0, ctx->stream, r, r, B, n, pin);
+    for (int32_t j = 0; j < m; ++j) {
+      const double* bj = B + (int64_t)j * ld;
+      hipLaunchKernelGGL(k_gs_step, dim3(nb), dim3(RB), 0, ctx->stream, r, bj, j + 1 < m ? bj + ld : nullptr, n, pin, nb,
+                         pout);
+      std::swap(pin, pout);
+    }
+  } else if (normalise) {
+    hipLaunchKernelGGL(k_dot_partial<false>, dim3(nb), dim3(RB), 0, ctx->stream, r, r, (const double*)nullptr, n, pin);
   }
-  if (normalise) {
-    dot(r, r);
-    hipLaunchKernelGGL(k_scal_rsqrt_dev, dim3(grid_for(n)), dim3(256), 0, ctx->stream, s, 1e-15, r, n);
-  }
+  if (normalise) hipLaunchKernelGGL(k_scal_rsqrt, dim3(nb), dim3(RB), 0, ctx->stream, pin, nb, 1e-15, r, n);
   HIPCHK(hipGetLastError());
   return BSG_OK;
 }
@@ -3146,41 +3021,61 @@ int bsg_axpy(bsg_context* ctx, double a, const double* x, double* y, int64_t n) 
 int bsg_gram(bsg_context* ctx, const double* X, const double* Y, int32_t m, int64_t n, int64_t ld, double* out) {
   if (!ctx || !X || !Y || !out || m <= 0 || m > GRAM_MAX || n < 0 || ld < n)
     return fail(BSG_ERR_ARG, "bsg_gram: bad args");
-  const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(GBLK, (n + GCH - 1) / GCH));
+  // about four 16-deep steps per wavefront at least
+  const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>(GBLK, (n + 255) / 256));
   double* part = ctx->gpart;
-  double* res = ctx->gpart + (size_t)GBLK * GMAX * GMAX;
-  // GMAX x GMAX tiles in stream order (the partials are reused tile by tile)
+  // GMAX x GMAX tiles in stream order (the partials are reused tile by tile);
+  // the sums go straight to page-locked host memory
   for (int i0 = 0; i0 < m; i0 += GMAX)
     for (int j0 = 0; j0 < m; j0 += GMAX) {
       const int mx = std::min(GMAX, m - i0), my = std::min(GMAX, m - j0);
       hipLaunchKernelGGL(k_gram_partial, dim3(nblk), dim3(256), 0, ctx->stream, X + (int64_t)i0 * ld,
                          Y + (int64_t)j0 * ld, mx, my, n, ld, part);
-      hipLaunchKernelGGL(k_gram_sum, dim3((mx * my + 255) / 256), dim3(256), 0, ctx->stream, part, nblk, mx, my,
-                         res + (int64_t)i0 * m + j0, m);
+      hipLaunchKernelGGL(k_gram_sum, dim3((mx * my + 3) / 4), dim3(256), 0, ctx->stream, part, nblk, mx, my,
+                         ctx->res_pin + (int64_t)i0 * m + j0, m);
     }
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(out, res, sizeof(double) * m * m, hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipStreamSynchronize(ctx->stream));
+  std::memcpy(out, ctx->res_pin, sizeof(double) * m * m);
   return BSG_OK;
 }
 int bsg_lincomb(bsg_context* ctx, const double* X, int32_t m, int64_t n, int64_t ld, const double* coef, int32_t mo,
                 double* Y, int64_t ldy) {
   if (!ctx || !X || !coef || !Y || m <= 0 || m > GRAM_MAX || mo <= 0 || mo > GRAM_MAX || n < 0 || ld < n || ldy < n)
     return fail(BSG_ERR_ARG, "bsg_lincomb: bad args");
-  double* cd = ctx->gpart + (size_t)GBLK * GMAX * GMAX + (size_t)GRAM_MAX * GRAM_MAX;
-  // coefficients through page-locked staging, so the call returns without
-  // waiting for the kernels (the staging is reused once its last copy is done)
-  HIPCHK(hipEventSynchronize(ctx->coef_done));
-  std::memcpy(ctx->coef_pin, coef, sizeof(double) * m * mo);
-  HIPCHK(hipMemcpyAsync(cd, ctx->coef_pin, sizeof(double) * m * mo, hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(hipEventRecord(ctx->coef_done, ctx->stream));
+  // coefficients through page-locked staging slots used in turn, so the call
+  // returns without waiting for the kernels (a slot is reused once its last
+  // copy is done; its device copy is behind that in stream order)
+  const int slot = ctx->coef_next;
+  ctx->coef_next = (slot + 1) % COEF_SLOTS;
+  const size_t at = (size_t)slot * GRAM_MAX * GRAM_MAX;
+  double* cd = ctx->gpart + (size_t)GBLK * GMAX * GMAX + at;
+  HIPCHK(hipEventSynchronize(ctx->coef_done[slot]));
+  for (int32_t i = 0; i < m; ++i)  // transposed: a result's coefficients contiguous
+    for (int32_t j = 0; j < mo; ++j) ctx->coef_pin[at + (size_t)j * m + i] = coef[(size_t)i * mo + j];
+  HIPCHK(hipMemcpyAsync(cd, ctx->coef_pin + at, sizeof(double) * m * mo, hipMemcpyHostToDevice, ctx->stream));
+  HIPCHK(hipEventRecord(ctx->coef_done[slot], ctx->stream));
   // GMAX x GMAX coefficient tiles; the first row tile of each output tile
   // overwrites Y, the others add in order
   for (int j0 = 0; j0 < mo; j0 += GMAX)
-    for (int i0 = 0; i0 < m; i0 += GMAX)
-      hipLaunchKernelGGL(k_lincomb, dim3(grid_for(n)), dim3(256), 0, ctx->stream, X + (int64_t)i0 * ld,
-                         std::min(GMAX, m - i0), n, ld, cd + (int64_t)i0 * mo + j0, mo, std::min(GMAX, mo - j0),
-                         Y + (int64_t)j0 * ldy, ldy, i0 > 0 ? 1 : 0);
+    for (int i0 = 0; i0 < m; i0 += GMAX) {
+      const int mt = std::min(GMAX, m - i0);
+      auto run = [&](auto MB) {
+        hipLaunchKernelGGL(k_lincomb<decltype(MB)::value>, dim3(grid_for((n + 1) / 2)), dim3(256), 0, ctx->stream,
+                           X + (int64_t)i0 * ld, mt, n, ld, cd + (int64_t)j0 * m + i0, m, std::min(GMAX, mo - j0),
+                           Y + (int64_t)j0 * ldy, ldy, i0 > 0 ? 1 : 0);
+      };
+      switch ((mt + 3) / 4) {
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 2: run(std::integral_constant<int, 2>{}); break;
+        case 3: run(std::integral_constant<int, 3>{}); break;
+        case 4: run(std::integral_constant<int, 4>{}); break;
+        case 5: run(std::integral_constant<int, 5>{}); break;
+        case 6: run(std::integral_constant<int, 6>{}); break;
+        case 7: run(std::integral_constant<int, 7>{}); break;
+        default: run(std::integral_constant<int, 8>{}); break;
+      }
+    }
   HIPCHK(hipGetLastError());
   return BSG_OK;
 }
@@ -3273,19 +3168,11 @@ int bsg_olsen_precondition(bsg_context* ctx, double* r, const double* c, const d
                            double* work, int64_t n) {
   if (!ctx || !r || !c || !d || !work || n < 0) return fail(BSG_ERR_ARG, "bsg_olsen_precondition: bad args");
   if (n == 0) return BSG_OK;
-  hipLaunchKernelGGL(k_copy, dim3(grid_for(n)), dim3(256), 0, ctx->stream, c, work, n);
-  int rc;
-  if ((rc = bsg_precondition(ctx, work, d, e, shift, n))) return rc;
-  // the two dot products stay in device memory: no host round trip
-  const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(RMAXB, (n + RB - 1) / RB));
-  double* s = ctx->red + RMAXB;
-  hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(RB), 0, ctx->stream, work, r, n, ctx->red);
-  hipLaunchKernelGGL(k_sum_partial, dim3(1), dim3(RB), 0, ctx->stream, ctx->red, nb, s + 1);
-  hipLaunchKernelGGL(k_dot_partial, dim3(nb), dim3(RB), 0, ctx->stream, c, work, n, ctx->red);
-  hipLaunchKernelGGL(k_sum_partial, dim3(1), dim3(RB), 0, ctx->stream, ctx->red, nb, s + 2);
-  hipLaunchKernelGGL(k_axpy_ratio_dev, dim3(grid_for(n)), dim3(256), 0, ctx->stream, s + 1, s + 2, c, r, n);
+  const int nb = reduce_grid(n);
+  hipLaunchKernelGGL(k_olsen_dots, dim3(nb), dim3(RB), 0, ctx->stream, r, c, d, e, shift, work, n, ctx->red);
+  hipLaunchKernelGGL(k_olsen_step, dim3(nb), dim3(RB), 0, ctx->stream, r, c, d, e, shift, n, ctx->red, nb);
   HIPCHK(hipGetLastError());
-  return bsg_precondition(ctx, r, d, e, shift, n);
+  return BSG_OK;
 }
 
 }  // extern "C"
