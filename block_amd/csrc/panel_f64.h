@@ -32,10 +32,12 @@ __device__ __forceinline__ int panel_at(int col, int k, int kp) {
 
 // One run of pairs with the same C block, k1 <= 16 KB and n <= 16 NB (a whole
 // wavefront: rows row0 .. row0 + 15 of the block)
-template <int KB, int NB>
+// stage() puts C into LDS (between barriers) once the first pair's loads are
+// under way.
+template <int KB, int NB, class F>
 __device__ __forceinline__ void panel_run(const PanelPair* __restrict__ prs, int count,
                                           const double* __restrict__ arena, const double* cl, int kp, int m, int n,
-                                          int k1, int k2, int row0, int li, int lk, dbl4 (&acc)[NB]) {
+                                          int k1, int k2, int row0, int li, int lk, dbl4 (&acc)[NB], F&& stage) {
   const int nk = (k1 + 7) >> 3, njb = (k2 + 15) >> 4;
   // byte offsets in a block, the same for every pair of the run: op(A)
   // (row row0 + li) and B' (column li of a 16-column group)
@@ -86,6 +88,7 @@ __device__ __forceinline__ void panel_run(const PanelPair* __restrict__ prs, int
   PanelPair nxt = prs[count > 1 ? 1 : 0];
   load_a(cur);
   load_b(cur, 0);
+  stage();
   for (int q = 0; q < count; ++q) {
     dbl2 a[2 * KB];
 #pragma unroll
@@ -170,7 +173,7 @@ template <int KB, int NB>
 __device__ __forceinline__ void panel_unit(const Seg& sg, const bsg_vblock_t& vb, const PanelPair* __restrict__ prs,
                                            const double* __restrict__ arena, const double* __restrict__ c,
                                            double* __restrict__ v, double* __restrict__ part, double* cl, int row0,
-                                           bool active) {
+                                           int tid, int nthreads) {
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
   dbl4 acc[NB];  // register i of lane (li, lk): V(row0 + lk + 4 i, 16 t + li)
 #pragma unroll
@@ -178,35 +181,51 @@ __device__ __forceinline__ void panel_unit(const Seg& sg, const bsg_vblock_t& vb
   for (int q = 0; q < sg.count;) {
     const PanelPair p0 = prs[sg.first + q];
     const int k1 = p0.k1, k2 = p0.k2, kp = (k1 + 15) & ~15, np = (k2 + 15) & ~15;
-    // C^T into LDS, zeros up to whole 16s
-    __syncthreads();
-    {
-      const __amdgpu_buffer_rsrc_t r = block_rsrc(c + p0.c, (int64_t)k1 * k2);
-      for (int e = threadIdx.x; e < kp * np; e += 256) {
-        const int k = e / np, col = e - k * np;
-        cl[panel_at(col, k, kp)] = bload(r, k < k1 && col < k2 ? (uint32_t)(k * k2 + col) * 8u : OOB);
-      }
+    // the run of pairs on this C block: [q, f) with an identity partner, then [f, e)
+    int f = q;
+    while (f < sg.count) {
+      const PanelPair& p = prs[sg.first + f];
+      if (p.c != p0.c || p.k1 != k1 || p.k2 != k2 || (p.a >= 0 && p.b >= 0)) break;
+      ++f;
     }
-    // the run of pairs on this C block: identity partners first (the planner's order)
-    int e = q;
+    int e = f;
     while (e < sg.count) {
       const PanelPair& p = prs[sg.first + e];
-      if (p.c != p0.c || p.k1 != k1 || p.k2 != k2) break;
+      if (p.c != p0.c || p.k1 != k1 || p.k2 != k2 || p.a < 0 || p.b < 0) break;
       ++e;
     }
-    __syncthreads();
-    if (active) {
-      while (q < e) {
-        const PanelPair pr = prs[sg.first + q];
-        if (pr.a >= 0 && pr.b >= 0) break;
-        panel_identity<NB>(pr, arena, cl, kp, vb.m, vb.n, row0, li, lk, acc);
-        ++q;
+    // C^T into LDS, zeros up to whole 16s: 8 lanes take 16 columns of a row, a
+    // column group's loads of all rows before their stores
+    auto stage = [&]() __attribute__((always_inline)) {
+      __syncthreads();
+      const __amdgpu_buffer_rsrc_t r = block_rsrc(c + p0.c, (int64_t)k1 * k2);
+      const int col0 = 2 * (tid & 7), kstep = nthreads >> 3;
+      for (int k = tid >> 3; k < kp; k += kstep) {
+        dbl2 x[KB];
+#pragma unroll
+        for (int j = 0; j < KB; ++j) {
+          const int col = 16 * j + col0;
+          if (16 * j < np) x[j] = bload128(r, col < k2 ? (uint32_t)(k * k2 + col) * 8u : OOB, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < KB; ++j) {
+          const int col = 16 * j + col0;
+          if (16 * j < np) {
+            cl[panel_at(col, k, kp)] = x[j][0];
+            cl[panel_at(col + 1, k, kp)] = col + 1 < k2 ? x[j][1] : 0.0;
+          }
+        }
       }
-      if (q < e) panel_run<KB, NB>(prs + sg.first + q, e - q, arena, cl, kp, vb.m, vb.n, k1, k2, row0, li, lk, acc);
-    }
+      __syncthreads();
+      for (; q < f; ++q)
+        panel_identity<NB>(prs[sg.first + q], arena, cl, kp, vb.m, vb.n, row0, li, lk, acc);
+    };
+    if (f < e)
+      panel_run<KB, NB>(prs + sg.first + f, e - f, arena, cl, kp, vb.m, vb.n, k1, k2, row0, li, lk, acc, stage);
+    else
+      stage();
     q = e;
   }
-  if (!active) return;
   const bool direct = sg.p_off < 0;
   double* out = direct ? v + vb.v_off : part + sg.p_off;
 #pragma unroll
@@ -241,22 +260,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KB <= 3 ? 3
   v += root * rs.wstride;
   part += root * rs.pstride;
   // a wavefront's panel turns with the workgroup, so that workgroups with
-  // fewer than four panels load all SIMDs alike; a wave without one only
-  // helps with C
+  // fewer than four panels load all SIMDs alike; a wave without one ends at
+  // once and leaves its registers to another workgroup (barriers count the
+  // waves that are left)
   const int w = (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + blockIdx.x / 8) & 3;
   const int row0 = 16 * (tr.tm * tr.pad + w);
-  const bool active = w < tr.pad && row0 < vb.m;
+  const int np = min(tr.pad, (vb.m + 15) / 16 - tr.tm * tr.pad);  // panels of this workgroup
+  if (w >= np) return;
+  const int tid = 64 * w + (threadIdx.x & 63), nt = 64 * np;
   const int nb = (vb.n + 15) >> 4;
   if (nb <= 1)
-    panel_unit<KB, 1>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+    panel_unit<KB, 1>(sg, vb, prs, arena, c, v, part, cl, row0, tid, nt);
   else if (nb == 2)
-    panel_unit<KB, 2>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+    panel_unit<KB, 2>(sg, vb, prs, arena, c, v, part, cl, row0, tid, nt);
   else if (KB <= 3 || nb == 3)
-    panel_unit<KB, 3>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+    panel_unit<KB, 3>(sg, vb, prs, arena, c, v, part, cl, row0, tid, nt);
   else if constexpr (KB > 3) {
     if (nb == 4)
-      panel_unit<KB, 4>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+      panel_unit<KB, 4>(sg, vb, prs, arena, c, v, part, cl, row0, tid, nt);
     else
-      panel_unit<KB, 5>(sg, vb, prs, arena, c, v, part, cl, row0, active);
+      panel_unit<KB, 5>(sg, vb, prs, arena, c, v, part, cl, row0, tid, nt);
   }
 }
