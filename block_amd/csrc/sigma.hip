@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -1223,6 +1224,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
 #include "gemm_f64.h"
 #include "panel_f64.h"
+#include "gemm_bf.h"
 
 // Tile geometry of the grouped kernels for an m x n V block: waves WR x WC
 // (WR WC = 4), NR 16-row blocks per wave (TM = 16 NR WR <= 64 rows), a W
@@ -1355,12 +1357,14 @@ inline int wave_candidate() {
   static const int n = (int)geom_candidates(6).size();
   return n;
 }
-// FP64 candidate the tile table names for an m x n V block (-1: none)
-inline int fp64_rule(const RuleSet& rs, int m, int n) {
+// candidate the tile table names for an m x n V block (-1: none)
+inline int table_rule(const RuleSet& rs, int m, int n, bool split) {
   for (const TileRule& r : rs.rules)
-    if (m >= r.m_lo && m <= r.m_hi && n >= r.n_lo && n <= r.n_hi) return r.fp64;
+    if (m >= r.m_lo && m <= r.m_hi && n >= r.n_lo && n <= r.n_hi) return split ? r.split : r.fp64;
   return -1;
 }
+// split-precision V blocks up to this on both sides stay on the grouped kernel
+constexpr int SPLIT_GROUPED = 64;
 // MFMA instructions of one pair in a per-wave tile plus a latency allowance
 // (segment cost)
 inline long wave_cost(int n, const bsg_pair_t& pr) {
@@ -1370,6 +1374,14 @@ inline long wave_cost(int n, const bsg_pair_t& pr) {
   return (pr.b_off < 0 ? nnb * nk1 : njb * (nk1 + 4 * nnb)) + 24;
 }
 typedef GemmTile<2, 2, 2, 2, 4> GemmT;
+typedef SplitTile<2, 4, 4, 2, 2> SplitBig;
+typedef SplitTile<2, 2, 2, 2, 3> SplitSmall;
+// 128 x 128 split tiles unless they pad an m x n product to much more than
+// 64 x 64 ones would
+inline int split_shape(int m, int n) {
+  auto area = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t) * t * t; };
+  return 2 * area(128) <= 3 * area(64);
+}
 // MFMA instructions per wavefront of one pair in a panel plus a latency
 // allowance
 inline long panel_cost(int n, int k1, int k2, bool a, bool b) {
@@ -1596,8 +1608,8 @@ struct bsg_context {
 // stream, each with its own half of the W scratch, so that one round's last
 // tiles run beside the next round's first.
 struct GemmRound {
-  TileRef *d_w = nullptr, *d_v = nullptr;  // W tiles, V tiles
-  int n_w = 0, n_v = 0;
+  TileRef *d_w[2] = {}, *d_v[2] = {};  // W tiles, V tiles by tile shape (FP64: the first only)
+  int n_w[2] = {}, n_v[2] = {};
 };
 
 // Launch lists of one precision mode of a chunk
@@ -1635,6 +1647,7 @@ struct PlanChunk {
   int64_t n_pairs = 0;
   std::vector<bsg_vblock_t> h_vb;
   std::vector<int32_t> h_base, h_fast;
+  std::vector<PairS> h_ps;
   ModeLists ml[2];  // FP64, split (made by the first bsg_plan_split_arena)
 };
 
@@ -1647,9 +1660,11 @@ struct bsg_plan {
   int64_t part_doubles[2] = {};
   std::shared_ptr<const RuleSet> rules;  // the tile table when the plan was created
   int32_t batch = 1;         // roots per launch (bsg_plan_set_batch)
-  std::shared_ptr<WScratch> wscratch;  // of the large blocks' rounds, wroots roots w_doubles apart
-  int64_t w_doubles = 0;
-  int32_t wroots = 1;        // roots per launch of the rounds
+  // by precision mode: W scratch of the large blocks' rounds, wroots roots
+  // w_doubles apart
+  std::shared_ptr<WScratch> wscratch[2];
+  int64_t w_doubles[2] = {};
+  int32_t wroots[2] = {1, 1};  // roots per launch of the rounds
   bool cs_ready = false;     // d_cs holds C slices for `batch` roots
   bool slices_built = false; // slice recipes and pair slice offsets (first bsg_plan_split_arena)
   bool abs_from_ctx = false; // d_abs is the context's lent buffer
@@ -1857,6 +1872,10 @@ std::shared_ptr<WScratch> w_scratch(bsg_context* ctx, int64_t n) {
   return w;
 }
 
+int32_t rounds_roots(int64_t w_doubles, int32_t nroot) {
+  return (int32_t)std::max<int64_t>(1, std::min<int64_t>(nroot, W_ROOTS / std::max<int64_t>(1, w_doubles)));
+}
+
 // Device arrays of one upload: parts gathered in a host buffer (256-byte
 // aligned), sent with one allocation and one copy, their pointers set then.
 struct Blob {
@@ -1904,34 +1923,51 @@ inline bool small_pair(const bsg_pair_t& pr) {
 // segs, whose pairs are gq's) and of the W tiles they read, in rounds of about
 // equal W size.
 void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, const std::vector<int>& bunits,
-                   const std::vector<int>& gq, const std::vector<Seg>& segs) {
+                   const std::vector<int>& gq, const std::vector<Seg>& segs, bool split) {
   const bsg_pair_t* perm = pc.h_perm.get();
+  const auto pad8 = [](int k) { return (k + 7) & ~7; };
   std::vector<GemmUnit> gu;
   std::vector<GemmSeg> gs;
-  std::vector<GemmAdd> ga;
+  std::vector<GemmAdd> ga, wadd;
   int64_t wtot = 0;
   auto w_size = [&](const bsg_vblock_t& vb, const bsg_pair_t& pr) {
-    return pr.a_off >= 0 && pr.b_off >= 0 ? (((int64_t)vb.m * pr.k2 + 1) & ~(int64_t)1) : 0;
+    if (pr.b_off < 0 || (pr.a_off < 0 && !split)) return (int64_t)0;
+    const int64_t n = split ? (3 * (int64_t)vb.m * pad8(pr.k2) + 3) / 4 : (int64_t)vb.m * pr.k2;  // doubles
+    return (n + 1) & ~(int64_t)1;
   };
   for (int bu : bunits) {
-      const Seg& sg = segs[bu];
-      for (int q = 0; q < sg.count; ++q) wtot += w_size(pc.h_vb[sg.vb], perm[gq[sg.first + q]]);
+    const Seg& sg = segs[bu];
+    for (int q = 0; q < sg.count; ++q) wtot += w_size(pc.h_vb[sg.vb], perm[gq[sg.first + q]]);
   }
   // an even number of rounds once W is large enough to be worth two
   int64_t nround = 1;
   if (wtot > W_ONE_ROUND) nround = 2 * ((wtot + W_HALF * 2 - 1) / (W_HALF * 2));
   const int64_t target = (wtot + nround - 1) / std::max<int64_t>(1, nround);
   ml.rounds.reserve(nround + 2);
-  std::vector<GUnit> uw, uv;
+  std::vector<GUnit> uw[2], uv[2];
   int64_t wused = 0, wneed[2] = {};
-  std::vector<std::pair<std::vector<TileRef>, std::vector<TileRef>>> rt;  // W tiles, V tiles
+  std::vector<std::array<std::vector<TileRef>, 4>> rt;  // W tiles, V tiles by shape
+  // a unit's tiles into the list of its tile shape
+  auto put = [&](std::vector<GUnit>(&to)[2], const GemmUnit& u, long cost) {
+    const int shape = split ? split_shape(u.m, u.n) : 0;
+    const int edge = split ? (shape ? SplitBig::T : SplitSmall::T) : GemmT::TM;
+    GUnit t;
+    t.cost = cost;
+    t.seg = (int)gu.size();
+    t.ntm = (u.m + edge - 1) / edge;
+    t.ntn = (u.n + edge - 1) / edge;
+    to[shape].push_back(t);
+    gu.push_back(u);
+  };
   auto close_round = [&]() {
-    if (uv.empty()) return;
+    if (uv[0].empty() && uv[1].empty()) return;
     int64_t& need = wneed[rt.size() & 1];
     need = std::max(need, wused);
-    rt.push_back({xcd_order(uw), xcd_order(uv)});
-    uw.clear();
-    uv.clear();
+    rt.push_back({xcd_order(uw[0]), xcd_order(uw[1]), xcd_order(uv[0]), xcd_order(uv[1])});
+    for (int k = 0; k < 2; ++k) {
+      uw[k].clear();
+      uv[k].clear();
+    }
     wused = 0;
   };
   for (int bu : bunits) {
@@ -1953,7 +1989,36 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
         continue;
       }
       GemmSeg x{};
-      if (pr.a_off < 0) {  // V += alpha C B'
+      const int half = (int)(rt.size() & 1);
+      if (split) {
+        // operands are slices with K padded to 8; op(A) C is formed as W^T, and
+        // an identity A's W = alpha C is split like any other W
+        const PairS& ps = pc.h_ps[gq[sg.first + q]];
+        if (pr.b_off < 0) {
+          x = GemmSeg{ps.a, ps.c, pr.alpha * pr.alpha_a, pad8(pr.k1), BS_C << SEG_RSPACE};
+        } else {
+          GemmUnit w{};
+          w.out = 4 * wused;
+          w.kind = GU_W;
+          w.m = pr.k2;
+          w.n = vb.m;
+          w.pad = half;
+          w.first = (int32_t)gs.size();
+          w.alpha = 1.0;
+          if (pr.a_off >= 0) {
+            w.alpha = pr.alpha * pr.alpha_a;
+            w.count = 1;
+            gs.push_back(GemmSeg{ps.c, ps.a, 1.0, pad8(pr.k1), BS_C << SEG_LSPACE});
+          } else {
+            w.add_first = (int32_t)wadd.size();
+            w.add_count = 1;
+            wadd.push_back({pr.c_off, pr.alpha});
+          }
+          put(uw, w, (pr.k1 + 31) / 32 + 4);
+          x = GemmSeg{4 * wused, ps.b, 1.0, pad8(pr.k2), (BS_W << SEG_LSPACE) | half << SEG_HALF};
+          wused += w_size(vb, pr);
+        }
+      } else if (pr.a_off < 0) {  // V += alpha C B'
         x = GemmSeg{pr.c_off, pr.b_off, pr.alpha, pr.k2, (SP_C << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0)};
       } else if (pr.b_off < 0) {  // V += alpha op(A) C
         x = GemmSeg{pr.a_off, pr.c_off, pr.alpha * pr.alpha_a, pr.k1, (SP_C << SEG_RSPACE) | (pr.a_trans ? SEG_LT : 0)};
@@ -1966,18 +2031,11 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
         w.first = (int32_t)gs.size();
         w.count = 1;
         w.alpha = pr.alpha * pr.alpha_a;
+        w.pad = half;
         gs.push_back(GemmSeg{pr.a_off, pr.c_off, 1.0, pr.k1,
                              (SP_C << SEG_RSPACE) | (pr.a_trans ? SEG_LT : 0)});
-        GUnit t;
-        t.cost = (pr.k1 + GKC - 1) / GKC + 4;
-        t.seg = (int)gu.size();
-        t.ntm = (w.m + GemmT::TM - 1) / GemmT::TM;
-        t.ntn = (w.n + GemmT::TN - 1) / GemmT::TN;
-        w.pad = (int32_t)(rt.size() & 1);
-        gu.push_back(w);
-        uw.push_back(t);
-        x = GemmSeg{wused, pr.b_off, 1.0, pr.k2, (SP_W << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0) |
-                                                     (int32_t)((rt.size() & 1) << SEG_HALF)};
+        put(uw, w, (pr.k1 + GKC - 1) / GKC + 4);
+        x = GemmSeg{wused, pr.b_off, 1.0, pr.k2, (SP_W << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0) | half << SEG_HALF};
         wused += w_size(vb, pr);
       }
       vcost += gemm_cost(pr);
@@ -1987,32 +2045,34 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
     un.first = (int32_t)gs.size();
     un.count = (int32_t)mine.size();
     gs.insert(gs.end(), mine.begin(), mine.end());
-    GUnit t;
-    t.cost = vcost;
-    t.seg = (int)gu.size();
-    t.ntm = (un.m + GemmT::TM - 1) / GemmT::TM;
-    t.ntn = (un.n + GemmT::TN - 1) / GemmT::TN;
-    gu.push_back(un);
-    uv.push_back(t);
+    put(uv, un, vcost);
     if (wused >= target) close_round();
   }
   close_round();
-  // the second half of the scratch follows the first
-  for (GemmUnit& u : gu)
-    if (u.kind == GU_W && u.pad) u.out += wneed[0];
-  for (GemmSeg& x : gs) {
-    if (((x.flags >> SEG_LSPACE) & 3) == SP_W && ((x.flags >> SEG_HALF) & 1)) x.l += wneed[0];
+  // the second half of the scratch follows the first; the W units' own
+  // additions follow the V units'
+  const int64_t second = split ? 4 * wneed[0] : wneed[0];
+  for (GemmUnit& u : gu) {
+    if (u.kind != GU_W) continue;
+    if (u.pad) u.out += second;
+    u.add_first += (int32_t)ga.size();
   }
-  p->w_doubles = std::max(p->w_doubles, wneed[0] + wneed[1]);
+  static_assert((int)SP_W == (int)BS_W, "one test for both precisions");
+  for (GemmSeg& x : gs)
+    if (((x.flags >> SEG_LSPACE) & 3) == SP_W && ((x.flags >> SEG_HALF) & 1)) x.l += second;
+  ga.insert(ga.end(), wadd.begin(), wadd.end());
+  p->w_doubles[split] = std::max(p->w_doubles[split], wneed[0] + wneed[1]);
   blob.add(&ml.d_gu, gu);
   blob.add(&ml.d_gs, gs);
   blob.add(&ml.d_ga, ga);
   ml.rounds.resize(rt.size());
   for (size_t r = 0; r < rt.size(); ++r) {
-    blob.add(&ml.rounds[r].d_w, rt[r].first);
-    blob.add(&ml.rounds[r].d_v, rt[r].second);
-    ml.rounds[r].n_w = (int)rt[r].first.size();
-    ml.rounds[r].n_v = (int)rt[r].second.size();
+    for (int k = 0; k < 2; ++k) {
+      blob.add(&ml.rounds[r].d_w[k], rt[r][k]);
+      blob.add(&ml.rounds[r].d_v[k], rt[r][2 + k]);
+      ml.rounds[r].n_w[k] = (int)rt[r][k].size();
+      ml.rounds[r].n_v[k] = (int)rt[r][2 + k].size();
+    }
   }
 }
 
@@ -2045,7 +2105,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       const bsg_pair_t* perm = pc.h_perm.get();
       const int base = pc.h_base[i], nfast = pc.h_fast[i], ntot = vb.count;
       const bool sm = small_block(vb);
-      const int rule = split ? -1 : fp64_rule(*p->rules, vb.m, vb.n);
+      const int rule = table_rule(*p->rules, vb.m, vb.n, split);
       const bool wave_vb = !split && !sm && rule == wave_candidate();
       units.clear();
       ukind.clear();
@@ -2079,11 +2139,11 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       const int slow = split && !sm ? 0 : nfast;  // pairs the small-block or per-wave kernel takes
       if (slow > 0) cut(base, slow, wave_vb ? UK_WAVE : UK_SMALL, in_perm(base));
       if (slow < ntot) {
-        if (split || wave_vb || (!sm && rule >= 0)) {
+        if (wave_vb || (!sm && rule >= 0) || (split && std::max(vb.m, vb.n) <= SPLIT_GROUPED)) {
           g = pick_geom(*p->rules, vb.m, vb.n, split ? 4 : 6);
           cut(base + slow, ntot - slow, UK_GROUPED, in_perm(base + slow));
         } else {
-          const bool med = std::max(vb.m, vb.n) <= PANEL_MAX;
+          const bool med = !split && std::max(vb.m, vb.n) <= PANEL_MAX;
           for (auto& x : pan) x.clear();
           big.clear();
           for (int q = base + slow; q < base + ntot; ++q) {
@@ -2310,7 +2370,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     blob.add(&ml.d_w[k], wt);
     ml.n_w[k] = (int)wt.size();
   }
-  if (!bunits.empty()) plan_products(p, pc, ml, blob, bunits, gq, segs);
+  if (!bunits.empty()) plan_products(p, pc, ml, blob, bunits, gq, segs, split);
   if (!blob.send(&ml.d_blob)) return fail(BSG_ERR_NOMEM, "plan lists");
   ml.ready = true;
   return BSG_OK;
@@ -2363,7 +2423,7 @@ int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunk
       Local& L = loc[t];
       for (int i = i0; i < i1; ++i) {
         const bsg_vblock_t& vb = ch.vblocks[i];
-        const bool sm = small_block(vb), wave_vb = !sm && fp64_rule(*p->rules, vb.m, vb.n) == wave_candidate();
+        const bool sm = small_block(vb), wave_vb = !sm && table_rule(*p->rules, vb.m, vb.n, false) == wave_candidate();
         bsg_pair_t* to = pc.h_perm.get() + pc.h_base[i];
         L.rest.clear();
         int nf = 0;
@@ -2423,7 +2483,7 @@ int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunk
   for (const PlanChunk& pc : p->chunks) p->part_doubles[0] = std::max(p->part_doubles[0], pc.ml[0].part_doubles);
   if (p->part_doubles[0] > 0 && hipMalloc(&p->part[0], sizeof(double) * p->part_doubles[0]) != hipSuccess)
     return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: partial-tile scratch");
-  if (p->w_doubles > 0 && !(p->wscratch = w_scratch(ctx, p->w_doubles)))
+  if (p->w_doubles[0] > 0 && !(p->wscratch[0] = w_scratch(ctx, p->w_doubles[0])))
     return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: W scratch");
   *plan = p;
   return BSG_OK;
@@ -2542,7 +2602,8 @@ int build_slices(bsg_plan* p) {
     return ct.get(off, 0, [&] { return slice_of(p->c_items, p->c_elems, off, k2, k1, 1); });
   };
   for (auto& pc : p->chunks) {
-    std::vector<PairS> ps(pc.n_pairs, PairS{-1, -1, -1});
+    std::vector<PairS>& ps = pc.h_ps;
+    ps.assign(pc.n_pairs, PairS{-1, -1, -1});
     sliced(pc, [&](int64_t j, const bsg_vblock_t& vb) {
       const bsg_pair_t& pr = pc.h_perm[j];
       if (pr.a_off >= 0) {
@@ -2585,6 +2646,10 @@ int bsg_plan_split_arena(bsg_context* ctx, bsg_plan* p, const double* arena, int
   HIPCHK(hipSetDevice(ctx->device));
   // FP64-only plans (the rotations, FP64 solves) never pay for the split
   // lists and slice recipes
+  if (!p->slices_built) {
+    const int rc = build_slices(p);
+    if (rc != BSG_OK) return rc;
+  }
   for (auto& pc : p->chunks) {
     if (pc.ml[1].ready) continue;
     const int rc = plan_lists(p, pc, true);
@@ -2594,9 +2659,10 @@ int bsg_plan_split_arena(bsg_context* ctx, bsg_plan* p, const double* arena, int
   if (!p->part[1] && p->part_doubles[1] > 0 &&
       hipMalloc(&p->part[1], sizeof(double) * p->part_doubles[1] * p->batch) != hipSuccess)
     return fail(BSG_ERR_NOMEM, "bsg_plan_split_arena: partial-tile scratch");
-  if (!p->slices_built) {
-    const int rc = build_slices(p);
-    if (rc != BSG_OK) return rc;
+  if (!p->wscratch[1] && p->w_doubles[1] > 0) {
+    p->wroots[1] = rounds_roots(p->w_doubles[1], p->batch);
+    if (!(p->wscratch[1] = w_scratch(ctx, p->w_doubles[1] * p->wroots[1])))
+      return fail(BSG_ERR_NOMEM, "bsg_plan_split_arena: W scratch");
   }
   // operator slices for the grouped kernel (the small-block kernel splits
   // in registers), and room for the C slices of one launch's roots
@@ -2667,16 +2733,18 @@ int bsg_plan_set_batch(bsg_context* ctx, bsg_plan* p, int32_t nroot) {
   }
   // the rounds of large blocks take as many roots per launch as W_ROOTS
   // doubles of scratch hold
-  const int32_t wroots =
-      (int32_t)std::max<int64_t>(1, std::min<int64_t>(nroot, W_ROOTS / std::max<int64_t>(1, p->w_doubles)));
+  int32_t wroots[2];
+  for (int k = 0; k < 2; ++k) wroots[k] = rounds_roots(p->w_doubles[k], nroot);
   // every new buffer before any old one goes: a failure leaves the plan as it was
   double* np[2] = {};
-  std::shared_ptr<WScratch> nw;
+  std::shared_ptr<WScratch> nw[2];
   __bf16* nc = nullptr;
-  const bool cs = p->cs_ready && p->c_elems > 0, wn = p->w_doubles > 0 && wroots != p->wroots;
+  const bool cs = p->cs_ready && p->c_elems > 0;
+  auto more_w = [&](int k) { return p->wscratch[k] && wroots[k] != p->wroots[k]; };
   if ((p->part[0] && hipMalloc(&np[0], sizeof(double) * p->part_doubles[0] * nroot) != hipSuccess) ||
       (p->part[1] && hipMalloc(&np[1], sizeof(double) * p->part_doubles[1] * nroot) != hipSuccess) ||
-      (wn && !(nw = w_scratch(ctx, p->w_doubles * wroots))) ||
+      (more_w(0) && !(nw[0] = w_scratch(ctx, p->w_doubles[0] * wroots[0]))) ||
+      (more_w(1) && !(nw[1] = w_scratch(ctx, p->w_doubles[1] * wroots[1]))) ||
       (cs && hipMalloc((void**)&nc, 2 * p->c_elems * nroot) != hipSuccess)) {
     for (double* x : np) (void)hipFree(x);
     return fail(BSG_ERR_NOMEM, "bsg_plan_set_batch: scratch of the roots");
@@ -2686,10 +2754,11 @@ int bsg_plan_set_batch(bsg_context* ctx, bsg_plan* p, int32_t nroot) {
       (void)hipFree(p->part[k]);
       p->part[k] = np[k];
     }
-  if (nw) {
-    p->wscratch = nw;
-    p->wroots = wroots;
-  }
+  for (int k = 0; k < 2; ++k)
+    if (nw[k]) {
+      p->wscratch[k] = nw[k];
+      p->wroots[k] = wroots[k];
+    }
   if (nc) {
     (void)hipFree(p->d_cs);
     p->d_cs = nc;
@@ -2731,16 +2800,28 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
   // round r of the large blocks, in launches of the roots its scratch holds
   auto round = [&](size_t r, hipStream_t q) {
     const GemmRound& g = ml.rounds[r];
-    for (int r0 = 0; r0 < rs.n; r0 += p->wroots) {
+    double* wbuf = p->wscratch[split] ? p->wscratch[split]->ptr : nullptr;
+    for (int r0 = 0; r0 < rs.n; r0 += p->wroots[split]) {
       RootSet sub = rs;
-      sub.n = std::min(p->wroots, rs.n - r0);
+      sub.n = std::min(p->wroots[split], rs.n - r0);
       const double* cr = c + r0 * rs.wstride;
+      const __bf16* csr = p->d_cs + r0 * rs.cstride;
       double *vr = v + r0 * rs.wstride, *pr = part + r0 * rs.pstride;
-      auto tiles = [&](const TileRef* t, int n) {
-        if (n == 0) return;
-        hipLaunchKernelGGL((k_gemm<GemmT>), dim3((unsigned)(((n + 7) / 8) * 8 * sub.n)), dim3(GemmT::NT), 0, q, ml.d_gu,
-                           ml.d_gs, ml.d_ga, t, n, arena, cr, vr, p->wscratch ? p->wscratch->ptr : nullptr, pr, sub);
-        ++nl;
+      auto tiles = [&](TileRef* const(&t)[2], const int(&n)[2]) {
+        for (int k = 1; k >= 0; --k) {
+          if (n[k] == 0) continue;
+          const dim3 blocks((unsigned)(((n[k] + 7) / 8) * 8 * sub.n));
+          if (!split)
+            hipLaunchKernelGGL((k_gemm<GemmT>), blocks, dim3(GemmT::NT), 0, q, ml.d_gu, ml.d_gs, ml.d_ga, t[k], n[k],
+                               arena, cr, vr, wbuf, pr, sub);
+          else if (k == 1)
+            hipLaunchKernelGGL((k_gemm_bf<SplitBig>), blocks, dim3(SplitBig::NT), 0, q, ml.d_gu, ml.d_gs, ml.d_ga, t[k],
+                               n[k], p->d_abs, csr, cr, vr, (__bf16*)wbuf, pr, sub);
+          else
+            hipLaunchKernelGGL((k_gemm_bf<SplitSmall>), blocks, dim3(SplitSmall::NT), 0, q, ml.d_gu, ml.d_gs, ml.d_ga,
+                               t[k], n[k], p->d_abs, csr, cr, vr, (__bf16*)wbuf, pr, sub);
+          ++nl;
+        }
       };
       tiles(g.d_w, g.n_w);
       tiles(g.d_v, g.n_v);
@@ -2778,6 +2859,7 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
     if (ev) HIPCHK(hipEventRecord(ev[2], ctx->side));
     HIPCHK(hipEventRecord(ctx->join, ctx->side));
   }
+  for (size_t r = 0; r < ml.rounds.size(); r += 2) round(r, st);
   if (split) {
     if (ml.n_g[2] > 0) {
       hipLaunchKernelGGL((k_sigma_bf<1, 4, 8>), grid(ml.n_g[2]), dim3(512), 0, st, ch.d_vb, ch.d_pr, ch.d_ps,
@@ -2790,7 +2872,6 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
       ++nl;
     }
   } else {
-    for (size_t r = 0; r < ml.rounds.size(); r += 2) round(r, st);
     if (ml.n_p[1] > 0) {
       hipLaunchKernelGGL((k_panel<5>), grid(ml.n_p[1]), dim3(256), 0, st, ch.d_vb, ml.d_pp, ml.d_seg, ml.d_p[1],
                          ml.n_p[1], arena, c, v, part, rs);
@@ -2837,7 +2918,7 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
 int check_precision(const bsg_plan* p, const double* arena, int32_t precision) {
   if (precision == BSG_FP64) return BSG_OK;
   if (precision != BSG_SPLIT_BF16) return fail(BSG_ERR_ARG, "unknown precision mode");
-  if (p->split_src != arena || !p->slices_built || (p->part_doubles[1] > 0 && !p->part[1]) || (p->ab_elems > 0 && !p->d_abs) || (p->c_elems > 0 && !p->d_cs))
+  if (p->split_src != arena || !p->slices_built || (p->part_doubles[1] > 0 && !p->part[1]) || (p->w_doubles[1] > 0 && !p->wscratch[1]) || (p->ab_elems > 0 && !p->d_abs) || (p->c_elems > 0 && !p->d_cs))
     return fail(BSG_ERR_ARG, "split precision needs bsg_plan_split_arena on this arena first");
   return BSG_OK;
 }
@@ -2859,7 +2940,7 @@ int sigma_apply_with(bsg_context* ctx, bsg_plan* p, const double* arena, const d
     rs.wstride = p->wave_size;
     rs.pstride = p->part_doubles[split];
     rs.cstride = p->c_elems;
-    rs.tstride = p->w_doubles;
+    rs.tstride = p->w_doubles[split];
     const double* cv = c + (size_t)iv * p->wave_size;
     double* vv = v + (size_t)iv * p->wave_size;
     if (split && !p->c_items.empty()) {

@@ -1,4 +1,4 @@
-"""FP64 sigma of hand-made work lists against numpy: V blocks and contraction
+"""Sigma of hand-made work lists, FP64 and split precision, against numpy: V blocks and contraction
 depths at the edges of the kernels' tiles (one row or column more or less than
 a tile, odd depths, depths of one), every storage order of the operator
 blocks, identity partners on either side, several units per V block, several
@@ -23,7 +23,8 @@ class Chunk(ctypes.Structure):
 
 
 for _name, _args in (("bsg_plan_create", [vp, vp, ctypes.c_int32, ctypes.c_int64, ctypes.POINTER(vp)]),
-                     ("bsg_plan_destroy", [vp]), ("bsg_plan_set_batch", [vp, vp, ctypes.c_int32])):
+                     ("bsg_plan_destroy", [vp]), ("bsg_plan_set_batch", [vp, vp, ctypes.c_int32]),
+                     ("bsg_plan_split_arena", [vp, vp, vp, ctypes.c_int64])):
     getattr(lib, _name).argtypes = _args
     getattr(lib, _name).restype = ctypes.c_int
 
@@ -112,9 +113,10 @@ CASES = {
 }
 
 
+@pytest.mark.parametrize("precision", [block_amd.FP64, block_amd.SPLIT_BF16], ids=["fp64", "split"])
 @pytest.mark.parametrize("name", list(CASES))
-def test_products(name):
-    print(f"[gpu] products {name}", flush=True)
+def test_products(name, precision):
+    print(f"[gpu] products {name} precision {precision}", flush=True)
     shapes, depths, repeats = CASES[name]
     rng = np.random.default_rng(sorted(CASES).index(name) + 5)
     vbs, prs, wave, wave_c, arena = work_list(rng, shapes, depths, repeats)
@@ -128,15 +130,17 @@ def test_products(name):
         try:
             da, dc = d.upload(arena), d.upload(c)
             dv = d.zeros(nroot * wave)
+            if precision == block_amd.SPLIT_BF16:
+                check(lib.bsg_plan_split_arena(d.ctx, plan, da, len(arena)))
             for r in range(nroot):  # one root at a time
                 check(lib.bsg_sigma_apply(d.ctx, plan, da, dc.value + 8 * r * wave, dv.value + 8 * r * wave, 1,
-                                          block_amd.FP64))
+                                          precision))
             one = d.download(dv, (nroot, wave))
             check(lib.bsg_plan_set_batch(d.ctx, plan, 2))
             check(lib.bsg_memset_zero(d.ctx, dv, 8 * nroot * wave))
-            check(lib.bsg_sigma_apply(d.ctx, plan, da, dc, dv, nroot, block_amd.FP64))  # 2 + 1
+            check(lib.bsg_sigma_apply(d.ctx, plan, da, dc, dv, nroot, precision))  # 2 + 1
             assert np.array_equal(d.download(dv, (nroot, wave)), one)
-            check(lib.bsg_sigma_apply(d.ctx, plan, da, dc, dv, nroot, block_amd.FP64))  # accumulates
+            check(lib.bsg_sigma_apply(d.ctx, plan, da, dc, dv, nroot, precision))  # accumulates
             twice = d.download(dv, (nroot, wave))
         finally:
             lib.bsg_plan_destroy(plan)
@@ -146,7 +150,13 @@ def test_products(name):
         # each of a value's two nested sums of at most `deep` products rounds
         # once per addition, on both sides of the comparison
         deep = 4 * max(int(prs["k1"].max() + prs["k2"].max()), int(vbs["count"].max()))
+        tol = 2 * deep * eps
+        if precision == block_amd.SPLIT_BF16:
+            # per product of the two: operands rounded to 2^-24, the slice
+            # products left out about 3 x 2^-24, FP32 sums of 6 x 32 terms in a
+            # tree or chain per K group (at most 6 + 32 roundings on its result)
+            tol += 2 * (2 + 3 + 38) * 2.0 ** -24
         err = np.abs(one[r] - ref)
-        assert np.all(err <= 2 * deep * eps * bound), (r, float((err / np.maximum(bound, 1e-300)).max()))
-        assert np.all(np.abs(twice[r] - 2 * ref) <= 4 * deep * eps * bound)
+        assert np.all(err <= tol * bound), (r, float((err / np.maximum(bound, 1e-300)).max()))
+        assert np.all(np.abs(twice[r] - 2 * ref) <= 2 * tol * bound)
         assert np.all(one[r][:wave_c] == 0.0)  # nothing written outside the V blocks
