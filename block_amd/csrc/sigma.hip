@@ -861,175 +861,6 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2))) v
     }
 }
 
-// ---------------------------------------------------------------- FP64 small-block kernel
-// V blocks of at most 32 x 32 (2 x 2 blocks of 16) are latency-bound in the
-// grouped kernel: their pairs are tiny and every pair pays the barriers and
-// memory round trips of a cooperative workgroup.  Here each wavefront owns a
-// whole small V block for one work unit and walks its pairs alone -- no LDS,
-// no barriers -- and a workgroup's 4 waves run 4 unrelated units.  A pair is
-// fused in registers by forming W^T = C^T op(A)^T instead of W: register i of
-// a v_mfma_f64_16x16x4f64 result holds (lane/16 + 4 i, lane%16), i.e. for W^T
-// the element W(lane%16, lane/16 + 4 i), which is exactly the A operand of
-// the second product's K step i.  Identity-B pairs use the direct W = op(A) C
-// orientation, whose result layout matches the V accumulators.
-// Small blocks run in FP64 in both precision modes: their MFMAs are not
-// what bounds them (operand latency is), so BF16 slices would only add the
-// slicing work, and FP64 is exact.
-// SB: 16-blocks per dimension of the V blocks an instantiation takes: SB = 1
-// for blocks (and contraction depths) up to 16, whose few registers leave
-// room for four waves per SIMD to hide the operand latency, SB = 2 for the
-// rest up to 32 x 32 (two waves per SIMD).
-template <int SB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SB == 1 ? 4 : 2))) void k_small(
-    const bsg_vblock_t* __restrict__ vbs, const bsg_pair_t* __restrict__ prs, const Seg* __restrict__ segs,
-    const int4* __restrict__ units, int nunits, const double* __restrict__ arena, const double* __restrict__ c,
-    double* __restrict__ v, double* __restrict__ part, RootSet roots) {
-  constexpr int KF = 4 * SB;  // 4-deep K steps of a dimension <= 16 SB
-  int u;
-  const int root = root_of(blockIdx.x, roots.n, u);
-  if (u >= nunits) return;
-  c += root * roots.wstride;
-  v += root * roots.wstride;
-  part += root * roots.pstride;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int4 un = units[u];
-  const int si = w == 0 ? un.x : (w == 1 ? un.y : (w == 2 ? un.z : un.w));
-  if (si < 0) return;  // no unit for this wave (waves never synchronise here)
-  const Seg sg = segs[si];
-  const bsg_vblock_t vb = vbs[sg.vb];
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  // row of accumulator register i inside its block: lk + 4 i
-  const int nrb = (vb.m + 15) / 16, nnb = (vb.n + 15) / 16;
-  dbl4 accV[SB][SB];
-#pragma unroll
-  for (int r = 0; r < SB; ++r)
-#pragma unroll
-    for (int t = 0; t < SB; ++t) accV[r][t] = dbl4{0.0, 0.0, 0.0, 0.0};
-  // The plan sends here only pairs with k1, k2 <= 16 SB and a non-identity A,
-  // or identity A and B' (the rest of a small block's pairs run in k_sigma).
-  // The next pair's descriptor is requested before this pair's operands, so
-  // its latency hides behind this pair's loads and MFMAs (units hold at
-  // least one pair).
-  bsg_pair_t nxt = prs[sg.first];
-  for (int q = 0; q < sg.count; ++q) {
-    const bsg_pair_t pr = nxt;
-    if (q + 1 < sg.count) nxt = prs[sg.first + q + 1];
-    const __amdgpu_buffer_rsrc_t rC = block_rsrc(c + pr.c_off, (int64_t)pr.k1 * pr.k2);
-    const uint32_t crow = (uint32_t)pr.k2 * 8u;
-    if (pr.a_off < 0) {  // identity A and B': V += alpha C
-#pragma unroll
-      for (int r = 0; r < SB; ++r)
-#pragma unroll
-        for (int t = 0; t < SB; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int row = r * 16 + lk + 4 * i, col = t * 16 + li;
-            const bool ok = row < vb.m && col < vb.n;
-            accV[r][t][i] += pr.alpha * bload(rC, ok ? (uint32_t)(row * pr.k2 + col) * 8u : OOB);
-          }
-      continue;
-    }
-    const __amdgpu_buffer_rsrc_t rA = block_rsrc(arena + pr.a_off, (int64_t)vb.m * pr.k1);
-    // op(A)(row, k) at row * ar + k * ak inside the block; rows past m masked,
-    // k past k1 meets zero C rows (out of the C block's range).  Every operand
-    // of the pair is requested before the first MFMA.
-    const int nk1 = (pr.k1 + 3) / 4;
-    const int ar = pr.a_trans ? 1 : pr.k1, ak = pr.a_trans ? vb.m : 1;
-    const double aw = pr.alpha_a * pr.alpha;
-    double a[SB][KF];  // a[r][s]: op(A)(r*16 + li, 4 s + lk)
-#pragma unroll
-    for (int r = 0; r < SB; ++r) {
-      const uint32_t off = (r < nrb && r * 16 + li < vb.m) ? (uint32_t)((r * 16 + li) * ar + lk * ak) * 8u : OOB;
-#pragma unroll
-      for (int s4 = 0; s4 < KF; ++s4) a[r][s4] = s4 < nk1 ? bload2(rA, off, (uint32_t)(s4 * ak) * 32u) : 0.0;
-    }
-    // C operands: ct[jb][s] = C(4 s + lk, jb*16 + li), zero past k2
-    const int njb = (pr.k2 + 15) / 16;
-    double ct[SB][KF];
-#pragma unroll
-    for (int jb = 0; jb < SB; ++jb) {
-      const int col = jb * 16 + li;
-      const uint32_t coff = (jb < njb && col < pr.k2) ? (uint32_t)(lk * pr.k2 + col) * 8u : OOB;
-#pragma unroll
-      for (int s4 = 0; s4 < KF; ++s4) ct[jb][s4] = (jb < njb && s4 < nk1) ? bload2(rC, coff, (uint32_t)(4 * s4) * crow) : 0.0;
-    }
-    if (pr.b_off < 0) {
-      // identity B': V(:, block t) += alpha alpha_a op(A) C(:, block t) (k2 = n)
-#pragma unroll
-      for (int t = 0; t < SB; ++t) {
-        if (t >= nnb) continue;
-        dbl4 accW[SB][1];
-#pragma unroll
-        for (int r = 0; r < SB; ++r) accW[r][0] = dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int s4 = 0; s4 < KF; ++s4)
-          if (s4 < nk1)
-#pragma unroll
-            for (int r = 0; r < SB; ++r)
-              if (r < nrb) accW[r][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r][s4], ct[t][s4], accW[r][0], 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < SB; ++r)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) accV[r][t][i] += aw * accW[r][0][i];
-      }
-      continue;
-    }
-    const __amdgpu_buffer_rsrc_t rB = block_rsrc(arena + pr.b_off, (int64_t)vb.n * pr.k2);
-    const int ks = pr.b_trans ? 1 : vb.n, cs = pr.b_trans ? pr.k2 : 1;
-    double b[SB][4][SB];  // b[jb][i][t]: B'(jb*16 + 4 i + lk, t*16 + li)
-#pragma unroll
-    for (int t = 0; t < SB; ++t) {
-      const uint32_t boff = (t < nnb && t * 16 + li < vb.n) ? (uint32_t)(lk * ks + (t * 16 + li) * cs) * 8u : OOB;
-#pragma unroll
-      for (int jb = 0; jb < SB; ++jb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          b[jb][i][t] = jb < njb ? bload2(rB, boff, (uint32_t)((jb * 4 + i) * ks) * 32u) : 0.0;
-    }
-#pragma unroll
-    for (int jb = 0; jb < SB; ++jb) {
-      if (jb >= njb) continue;
-      // W^T block row jb: register i of lane (li, lk) is W(li, jb*16 + lk + 4 i)
-      dbl4 accT[SB];
-#pragma unroll
-      for (int r = 0; r < SB; ++r) accT[r] = dbl4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int s4 = 0; s4 < KF; ++s4)
-        if (s4 < nk1)
-#pragma unroll
-          for (int r = 0; r < SB; ++r)
-            if (r < nrb) accT[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(ct[jb][s4], a[r][s4], accT[r], 0, 0, 0);
-      // GEMM 2 over K = jb*16 + 4 i + lk, A operand = register i of accT
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int r = 0; r < SB; ++r)
-#pragma unroll
-          for (int t = 0; t < SB; ++t)
-            if (r < nrb && t < nnb)
-              accV[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(aw * accT[r][i], b[jb][i][t], accV[r][t], 0, 0, 0);
-    }
-  }
-  const bool direct = sg.p_off < 0;
-  double* out = direct ? v + vb.v_off : part + sg.p_off;
-#pragma unroll
-  for (int r = 0; r < SB; ++r)
-#pragma unroll
-    for (int t = 0; t < SB; ++t) {
-      const int col = t * 16 + li;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = r * 16 + lk + 4 * i;
-        if (row < vb.m && col < vb.n) {
-          if (direct)
-            out[(size_t)row * vb.n + col] += accV[r][t][i];
-          else
-            out[(size_t)row * vb.n + col] = accV[r][t][i];
-        }
-      }
-    }
-}
-
 // ---------------------------------------------------------------- FP64 per-wave tiles
 // Medium V blocks are latency-bound in the grouped kernel too: a pair's
 // MFMAs are few next to its operand round trips, and a 4-wave tile runs one
@@ -1224,6 +1055,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 
 #include "gemm_f64.h"
 #include "panel_f64.h"
+#include "small_f64.h"
 #include "gemm_bf.h"
 
 // Tile geometry of the grouped kernels for an m x n V block: waves WR x WC
@@ -1337,14 +1169,12 @@ Geom pick_geom_uncached(const RuleSet& rs, int m, int n, int max_nv) {
   }
   return best;
 }
-// MFMA instructions of one pair in the small-block kernel plus a latency
-// allowance (segment cost; the wave works alone)
-inline long small_cost(int m, int n, const bsg_pair_t& pr) {
-  auto cdiv = [](long a, long b) { return (a + b - 1) / b; };
-  const long nrb = cdiv(m, 16), nnb = cdiv(n, 16), njb = cdiv(pr.k2, 16);
-  const long g1 = pr.a_off < 0 ? 0 : (pr.b_off < 0 ? nnb : njb) * cdiv(pr.k1, 4) * nrb;
-  const long g2 = pr.b_off < 0 ? 0 : njb * 4 * nrb * nnb;
-  return g1 + g2 + 24;
+// MFMA instructions of one pair in the small-block kernel plus an allowance
+// for its loads (segment cost; the wave works alone)
+template <class Pair>  // bsg_pair_t, PanelPair
+inline long small_cost(int m, int n, const Pair& pr) {
+  const long nrb = (m + 15) / 16, nnb = (n + 15) / 16, o = (std::max(pr.k1, pr.k2) + 7) / 8;
+  return 2 * o * ((o + 1) / 2 * nrb + nrb * nnb) + 4;
 }
 // Per-wave tiles: 16 x 32 for V blocks up to 32 columns, 16 x 64 above
 // (wave_nb).  In the FP64 column of the tile table the candidate index after
@@ -1619,13 +1449,13 @@ struct ModeLists {
   Seg* d_seg = nullptr;
   TileRef* d_g[NCLS] = {};       // grouped-kernel tiles per kernel class (split: basic, 256 wide, 512 wide)
   int n_g[NCLS] = {};
-  int4* d_s[2] = {};             // FP64 small-block units, 4 per workgroup (SB = 2, SB = 1)
-  int n_s[2] = {};
+  int32_t* d_s[3] = {};          // FP64 small-block units (up to 16, 24, 32 wide)
+  int n_s[3] = {};
   TileRef* d_w[2] = {};          // FP64 per-wave tiles (16 x 32, 16 x 64), 4 per workgroup (item -1: none), a multiple of 32
   int n_w[2] = {};
-  TileRef* d_p[2] = {};          // FP64 panels (KB = 3, 5) and their pairs
+  TileRef* d_p[2] = {};          // FP64 panels (KB = 3, 5)
   int n_p[2] = {};
-  PanelPair* d_pp = nullptr;
+  PanelPair* d_pp = nullptr;     // pairs of the panels and small blocks
   GemmUnit* d_gu = nullptr;      // FP64 product tiles, by round
   GemmSeg* d_gs = nullptr;
   GemmAdd* d_ga = nullptr;
@@ -1908,10 +1738,12 @@ struct Blob {
 };
 
 // kernels a work unit runs on
-enum UnitKind : char { UK_GROUPED = 0, UK_SMALL = 1, UK_WAVE = 2, UK_GEMM = 3, UK_PANEL3 = 4, UK_PANEL5 = 5 };
+enum UnitKind : char { UK_GROUPED = 0, UK_WAVE = 2, UK_GEMM = 3, UK_PANEL3 = 4, UK_PANEL5 = 5, UK_SMALL = 6 /* + class 0 .. 2 */ };
 
-// MFMAs per wavefront of a work unit before its pair list is split
-constexpr long SEG_COST = 2048, SEG_COST_SMALL = 1024;
+// MFMAs per wavefront of a work unit before its pair list is split (small
+// blocks: by width class; half as much or twice as much in the first two
+// takes 217 and 233 us for 208 on the D2h superblock at M = 250)
+constexpr long SEG_COST = 2048, SEG_COST_SMALL[3] = {256, 768, 1024};
 
 inline bool small_block(const bsg_vblock_t& vb) { return std::max(vb.m, vb.n) <= 32; }
 // whether the small-block kernel takes a pair of a small block
@@ -2084,7 +1916,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
   ModeLists& ml = pc.ml[split];
   struct Local {
     std::vector<GUnit> gunits[NCLS];                 // grouped tiles by kernel class
-    std::vector<std::pair<long, int>> sunits[2];     // (cost, segment) of small-block units (SB = 2, SB = 1)
+    std::vector<std::pair<long, int>> sunits[3];     // (cost, segment) of small-block units (up to 16, 24, 32)
     std::vector<int> bunits;                         // large blocks' units (segments)
     std::vector<GUnit> wunits[2], punits[2];         // per-wave tiles (16 x 32, 16 x 64), panels (KB = 3, 5)
     std::vector<int> gq;                             // pairs of the large blocks' units (indices into h_perm)
@@ -2099,7 +1931,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     Local& L = loc[t];
     std::vector<std::pair<int, int>> units;  // (first, count)
     std::vector<char> ukind;
-    std::vector<int> pan[2], big;
+    std::vector<int> pan[2], big, few[3];
     for (int i = i0; i < i1; ++i) {
       const bsg_vblock_t& vb = pc.h_vb[i];
       const bsg_pair_t* perm = pc.h_perm.get();
@@ -2112,7 +1944,9 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       Geom g;
       auto cost_of = [&](int kind, const bsg_pair_t& pr) -> long {
         switch (kind) {
-          case UK_SMALL: return small_cost(vb.m, vb.n, pr);
+          case UK_SMALL:
+          case UK_SMALL + 1:
+          case UK_SMALL + 2: return small_cost(vb.m, vb.n, pr);
           case UK_WAVE: return wave_cost(vb.n, pr);
           case UK_GEMM: return gemm_cost(pr);
           case UK_PANEL3:
@@ -2122,7 +1956,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       };
       // at(q): the list's q-th pair; first: its index where the units point
       auto cut = [&](int first, int n, int kind, auto at) {
-        const long lim = kind == UK_SMALL ? SEG_COST_SMALL : SEG_COST;
+        const long lim = kind >= UK_SMALL ? SEG_COST_SMALL[kind - UK_SMALL] : SEG_COST;
         int start = 0;
         long cost = 0;
         for (int q = 0; q < n; ++q) {
@@ -2137,7 +1971,38 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       };
       auto in_perm = [&](int first) { return [&, first](int q) -> const bsg_pair_t& { return perm[first + q]; }; };
       const int slow = split && !sm ? 0 : nfast;  // pairs the small-block or per-wave kernel takes
-      if (slow > 0) cut(base, slow, wave_vb ? UK_WAVE : UK_SMALL, in_perm(base));
+      // a list's pairs by C block (identity partners first, else as given) as
+      // the kernels that keep C read them; pad: pairs left in the run on one C
+      // block
+      auto cut_by_c = [&](std::vector<int>& list, int kind) {
+        std::stable_sort(list.begin(), list.end(), [&](int x, int y) {
+          const bsg_pair_t &a = perm[x], &b = perm[y];
+          if (a.c_off != b.c_off) return a.c_off < b.c_off;
+          return (a.a_off < 0 || a.b_off < 0) && !(b.a_off < 0 || b.b_off < 0);
+        });
+        const int first = (int)L.pp.size();
+        for (int q : list) {
+          const bsg_pair_t& x = perm[q];
+          L.pp.push_back(PanelPair{x.a_off, x.c_off, x.b_off, x.a_off < 0 ? x.alpha : x.alpha * x.alpha_a, x.k1, x.k2,
+                                   (x.a_trans ? 1 : 0) | (x.b_trans ? 2 : 0), 1});
+        }
+        for (int q = (int)L.pp.size() - 2; q >= first; --q) {
+          PanelPair &x = L.pp[q], &y = L.pp[q + 1];
+          if (x.c == y.c && x.k1 == y.k1 && x.k2 == y.k2) x.pad = y.pad + 1;
+        }
+        cut(first, (int)list.size(), kind, [&](int q) -> const bsg_pair_t& { return perm[list[q]]; });
+      };
+      if (slow > 0 && wave_vb) cut(base, slow, UK_WAVE, in_perm(base));
+      if (slow > 0 && !wave_vb) {
+        for (auto& x : few) x.clear();
+        for (int q = base; q < base + slow; ++q) {
+          int k = std::max(vb.m, vb.n);
+          if (perm[q].a_off >= 0) k = std::max(k, std::max(perm[q].k1, perm[q].k2));
+          few[k <= 16 ? 0 : (k <= 24 ? 1 : 2)].push_back(q);
+        }
+        for (int k = 0; k < 3; ++k)
+          if (!few[k].empty()) cut_by_c(few[k], UK_SMALL + k);
+      }
       if (slow < ntot) {
         if (wave_vb || (!sm && rule >= 0) || (split && std::max(vb.m, vb.n) <= SPLIT_GROUPED)) {
           g = pick_geom(*p->rules, vb.m, vb.n, split ? 4 : 6);
@@ -2153,22 +2018,8 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
             else
               pan[k > 48 || vb.n > 48].push_back(q);
           }
-          for (int k = 0; k < 2; ++k) {
-            if (pan[k].empty()) continue;
-            // by C block, identity partners first, else as given
-            std::stable_sort(pan[k].begin(), pan[k].end(), [&](int x, int y) {
-              const bsg_pair_t &a = perm[x], &b = perm[y];
-              if (a.c_off != b.c_off) return a.c_off < b.c_off;
-              return (a.a_off < 0 || a.b_off < 0) && !(b.a_off < 0 || b.b_off < 0);
-            });
-            const int first = (int)L.pp.size();
-            for (int q : pan[k]) {
-              const bsg_pair_t& x = perm[q];
-              L.pp.push_back(PanelPair{x.a_off, x.c_off, x.b_off, x.a_off < 0 ? x.alpha : x.alpha * x.alpha_a, x.k1, x.k2,
-                                       (x.a_trans ? 1 : 0) | (x.b_trans ? 2 : 0), 0});
-            }
-            cut(first, (int)pan[k].size(), k ? UK_PANEL5 : UK_PANEL3, [&](int q) -> const bsg_pair_t& { return perm[pan[k][q]]; });
-          }
+          for (int k = 0; k < 2; ++k)
+            if (!pan[k].empty()) cut_by_c(pan[k], k ? UK_PANEL5 : UK_PANEL3);
           if (!big.empty()) {
             const int first = (int)L.gq.size();
             L.gq.insert(L.gq.end(), big.begin(), big.end());
@@ -2179,13 +2030,6 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       const int64_t mn = (int64_t)vb.m * vb.n;
       const int nseg = (int)units.size();
       const int64_t p0 = L.poff;
-      bool tiny = std::max(vb.m, vb.n) <= 16;  // the block and its small-kernel pairs' C blocks within 16 x 16
-      if (tiny && !wave_vb)
-        for (int q = 0; q < slow; ++q)
-          if (perm[base + q].k1 > 16 || perm[base + q].k2 > 16) {
-            tiny = false;
-            break;
-          }
       for (int u = 0; u < nseg; ++u) {
         Seg sg;
         sg.vb = i;
@@ -2203,10 +2047,12 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
         long ucost = 0;
         if (kind == UK_PANEL3 || kind == UK_PANEL5)
           for (int q = 0; q < sg.count; ++q) ucost += panel_cost(vb.n, L.pp[sg.first + q]);
+        else if (kind >= UK_SMALL)
+          for (int q = 0; q < sg.count; ++q) ucost += small_cost(vb.m, vb.n, L.pp[sg.first + q]);
         else
           for (int q = 0; q < sg.count; ++q) ucost += cost_of(kind, perm[sg.first + q]);
-        if (kind == UK_SMALL) {
-          L.sunits[tiny ? 1 : 0].push_back({ucost, si});
+        if (kind >= UK_SMALL) {
+          L.sunits[kind - UK_SMALL].push_back({ucost, si});
           continue;
         }
         GUnit gu;
@@ -2247,7 +2093,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
   });
   // concatenate with the local indices shifted
   std::vector<GUnit> gunits[NCLS], wunits[2], punits[2];
-  std::vector<std::pair<long, int>> sunits[2];
+  std::vector<std::pair<long, int>> sunits[3];
   std::vector<int> bunits, gq;
   std::vector<PanelPair> pp;
   std::vector<Seg> segs;
@@ -2259,8 +2105,8 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     for (int k = 0; k < 2; ++k) {
       wunits[k].swap(L.wunits[k]);
       punits[k].swap(L.punits[k]);
-      sunits[k].swap(L.sunits[k]);
     }
+    for (int k = 0; k < 3; ++k) sunits[k].swap(L.sunits[k]);
     bunits.swap(L.bunits);
     gq.swap(L.gq);
     pp.swap(L.pp);
@@ -2279,6 +2125,8 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       std::vector<char> kind(L.segs.size(), 0);  // 1: the unit's pairs are in pp, 2: in gq
       for (int k = 0; k < 2; ++k)
         for (const GUnit& u : L.punits[k]) kind[u.seg] = 1;
+      for (int k = 0; k < 3; ++k)
+        for (const auto& x : L.sunits[k]) kind[x.second] = 1;
       for (int s : L.bunits) kind[s] = 2;
       for (size_t s = 0; s < L.segs.size(); ++s) {
         Seg sg = L.segs[s];
@@ -2296,8 +2144,9 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       for (int k = 0; k < 2; ++k) {
         shift(wunits[k], L.wunits[k]);
         shift(punits[k], L.punits[k]);
-        for (auto x : L.sunits[k]) sunits[k].push_back({x.first, x.second + sb});
       }
+      for (int k = 0; k < 3; ++k)
+        for (auto x : L.sunits[k]) sunits[k].push_back({x.first, x.second + sb});
       for (int s : L.bunits) bunits.push_back(s + sb);
       gq.insert(gq.end(), L.gq.begin(), L.gq.end());
       pp.insert(pp.end(), L.pp.begin(), L.pp.end());
@@ -2316,19 +2165,15 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
   blob.add(&ml.d_red, reds);
   ml.n_red = (int)reds.size();
   blob.add(&ml.d_pp, pp);
-  // small-block units, costliest first, four per workgroup
-  for (int k = 0; k < 2; ++k) {
+  // small-block units, costliest first
+  for (int k = 0; k < 3; ++k) {
     auto& su = sunits[k];
     std::sort(su.begin(), su.end(), [](const std::pair<long, int>& x, const std::pair<long, int>& y) {
       return x.first != y.first ? x.first > y.first : x.second < y.second;
     });
-    std::vector<int4> sq;
-    sq.reserve(su.size() / 4 + 1);
-    for (size_t i = 0; i < su.size(); i += 4) {
-      int e[4];
-      for (int j = 0; j < 4; ++j) e[j] = i + j < su.size() ? su[i + j].second : -1;
-      sq.push_back(make_int4(e[0], e[1], e[2], e[3]));
-    }
+    std::vector<int32_t> sq;
+    sq.reserve(su.size());
+    for (const auto& x : su) sq.push_back(x.second);
     blob.add(&ml.d_s[k], sq);
     ml.n_s[k] = (int)sq.size();
   }
@@ -2796,7 +2641,7 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
   // partial tiles, and the reduction waits for both
   const int nbasic = ml.n_g[0];
   const int *ns = ml.n_s;
-  const bool side = ns[0] > 0 || ns[1] > 0 || nbasic > 0 || ml.n_p[0] > 0 || ml.rounds.size() > 1;
+  const bool side = ns[1] > 0 || ns[2] > 0 || nbasic > 0 || ml.n_p[0] > 0 || ml.rounds.size() > 1;
   // round r of the large blocks, in launches of the roots its scratch holds
   auto round = [&](size_t r, hipStream_t q) {
     const GemmRound& g = ml.rounds[r];
@@ -2837,14 +2682,14 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
                          ml.n_p[0], arena, c, v, part, rs);
       ++nl;
     }
-    if (ns[0] > 0) {
-      hipLaunchKernelGGL((k_small<2>), grid(ns[0]), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ml.d_seg,
-                         ml.d_s[0], ns[0], arena, c, v, part, rs);
+    if (ns[2] > 0) {
+      hipLaunchKernelGGL((k_small<4>), grid(ns[2]), dim3(64), 0, ctx->side, ch.d_vb, ml.d_pp, ml.d_seg, ml.d_s[2],
+                         ns[2], arena, c, v, part, rs);
       ++nl;
     }
     if (ns[1] > 0) {
-      hipLaunchKernelGGL((k_small<1>), grid(ns[1]), dim3(256), 0, ctx->side, ch.d_vb, ch.d_pr, ml.d_seg,
-                         ml.d_s[1], ns[1], arena, c, v, part, rs);
+      hipLaunchKernelGGL((k_small<3>), grid(ns[1]), dim3(64), 0, ctx->side, ch.d_vb, ml.d_pp, ml.d_seg, ml.d_s[1],
+                         ns[1], arena, c, v, part, rs);
       ++nl;
     }
     if (nbasic > 0) {
@@ -2858,6 +2703,11 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
     }
     if (ev) HIPCHK(hipEventRecord(ev[2], ctx->side));
     HIPCHK(hipEventRecord(ctx->join, ctx->side));
+  }
+  if (ns[0] > 0) {
+    hipLaunchKernelGGL((k_small<2>), grid(ns[0]), dim3(64), 0, st, ch.d_vb, ml.d_pp, ml.d_seg, ml.d_s[0], ns[0],
+                       arena, c, v, part, rs);
+    ++nl;
   }
   for (size_t r = 0; r < ml.rounds.size(); r += 2) round(r, st);
   if (split) {

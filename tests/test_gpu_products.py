@@ -108,6 +108,10 @@ CASES = {
     "mixed": ([(81, 16), (40, 81), (33, 95), (64, 40)], [(81, 3), (7, 82), (96, 81), (30, 40)], 2),
     # 64-wide tiles: exact, one less, one more, depths of odd and even length
     "large": ([(127, 129), (128, 64), (97, 193), (191, 82)], [(1, 1), (2, 15), (16, 17), (129, 31), (100, 130)], 2),
+    # small-block kernel: each of its width and depth classes (8s and 16s, one
+    # less, one more), runs on one C block longer than its operand sets
+    "width32": ([(1, 1), (8, 7), (16, 16), (17, 3), (9, 24), (24, 24), (25, 8), (32, 31)],
+                [(1, 1), (8, 8), (9, 2), (3, 16), (17, 24), (24, 23), (25, 8), (31, 32)], 3),
     # many pairs per V block: several units, reduced in order
     "units": ([(90, 100), (50, 60), (20, 24)], [(61, 67), (24, 24)], 60),
 }
