@@ -1233,6 +1233,10 @@ inline int split_shape(int m, int n) {
   auto area = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t) * t * t; };
   return 2 * area(128) <= 3 * area(64);
 }
+// ... in superblocks that fill the chip with such tiles: at 11,000 W tiles of
+// 128 (C1, peak dimension 250) the smaller shape alone takes 1.28 ms for 1.40
+// with both, at 22,000 2.91 for 2.71 (C1, 313), at 55,000 2.71 for 2.62
+constexpr int64_t SPLIT_WIDE = 1 << 14;
 // MFMA instructions per wavefront of one pair in a panel plus a latency
 // allowance
 inline long panel_cost(int n, int k1, int k2, bool a, bool b) {
@@ -1252,7 +1256,7 @@ inline long gemm_cost(const bsg_pair_t& pr) {
 // W scratch of the large blocks' rounds, in doubles: one round up to
 // W_ONE_ROUND, else an even number of rounds of at most W_HALF each; roots
 // share a launch while W_ROOTS holds all of them
-constexpr int64_t W_ONE_ROUND = 1 << 21, W_HALF = 1 << 26, W_ROOTS = 1 << 29, W_KEEP = 1 << 27;
+constexpr int64_t W_ONE_ROUND = 1 << 23, W_HALF = 1 << 26, W_ROOTS = 1 << 29, W_KEEP = 1 << 27;
 // MFMA instructions per wavefront of one pair in a tile (segment cost)
 inline long pair_cost(const Geom& g, int n, const bsg_pair_t& pr) {
   auto cdiv = [](long a, long b) { return (a + b - 1) / b; };
@@ -1795,10 +1799,17 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
     const int64_t n = split ? (3 * (int64_t)vb.m * pad8(pr.k2) + 3) / 4 : (int64_t)vb.m * pr.k2;  // doubles
     return (n + 1) & ~(int64_t)1;
   };
+  int64_t wide_tiles = 0;  // W tiles of the larger shape
   for (int bu : bunits) {
     const Seg& sg = segs[bu];
-    for (int q = 0; q < sg.count; ++q) wtot += w_size(pc.h_vb[sg.vb], perm[gq[sg.first + q]]);
+    const bsg_vblock_t& vb = pc.h_vb[sg.vb];
+    for (int q = 0; q < sg.count; ++q) {
+      const bsg_pair_t& pr = perm[gq[sg.first + q]];
+      wtot += w_size(vb, pr);
+      if (split) wide_tiles += ((vb.m + SplitBig::T - 1) / SplitBig::T) * (int64_t)((pr.k2 + SplitBig::T - 1) / SplitBig::T);
+    }
   }
+  const bool wide = wide_tiles >= SPLIT_WIDE;
   // an even number of rounds once W is large enough to be worth two
   int64_t nround = 1;
   if (wtot > W_ONE_ROUND) nround = 2 * ((wtot + W_HALF * 2 - 1) / (W_HALF * 2));
@@ -1809,7 +1820,7 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
   std::vector<std::array<std::vector<TileRef>, 4>> rt;  // W tiles, V tiles by shape
   // a unit's tiles into the list of its tile shape
   auto put = [&](std::vector<GUnit>(&to)[2], const GemmUnit& u, long cost) {
-    const int shape = split ? split_shape(u.m, u.n) : 0;
+    const int shape = wide ? split_shape(u.m, u.n) : 0;
     const int edge = split ? (shape ? SplitBig::T : SplitSmall::T) : GemmT::TM;
     GUnit t;
     t.cost = cost;
@@ -1985,7 +1996,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       };
       // at(q): the list's q-th pair; first: its index where the units point
       auto cut = [&](int first, int n, int kind, auto at) {
-        const long lim = kind == UK_GEMM ? SEG_COST : std::min(fill, kind >= UK_SMALL ? SEG_COST_SMALL[kind - UK_SMALL] : SEG_COST);
+        const long lim = std::min(kind == UK_GEMM ? fill / 2 : fill, kind >= UK_SMALL ? SEG_COST_SMALL[kind - UK_SMALL] : SEG_COST);
         int start = 0;
         long cost = 0;
         for (int q = 0; q < n; ++q) {
