@@ -8,32 +8,40 @@
 // it holds its rows of op(A) in registers, forms W^T = C^T op(A)^T 16 W columns
 // at a time (C^T from LDS), and the result registers are at once the A operand
 // of the product with B'.  What a wavefront streams per pair is op(A)'s rows
-// and B'; both are requested a step ahead (op(A) a pair, B' 16 rows) in a
-// second register set.  The waves of a workgroup (the 16-row panels of one
+// and B'.  Each has one register set, requested as soon as the product that
+// reads it is done and while the other product runs, which leaves room for
+// three waves per SIMD.  The waves of a workgroup (the 16-row panels of one
 // V block) meet only where the C block changes.
 //
-// K order: a 16-byte load takes two K of an operand whose K is contiguous,
-// so K step (s, e) of lane lk is 8 s + 2 lk + e in op(A) C, and W column
-// 4 lk + i of a 16-column group in W B' (the C^T rows are permuted for that).
+// K order: step (s, e) of lane lk is 8 s + 2 lk + e in both products, so that
+// a 16-byte load takes two K of an operand whose K is contiguous (the C^T rows
+// are permuted, so that W columns come out in that order).
+//
+// Bound by the MFMA chains of too few wavefronts: C's 51 KB of LDS and 168
+// registers allow ten to twelve per CU, blocks of 65 to 80 rows fill 7.5.  36
+// orbitals, D2h, M = 1000 (330,000 pairs, blocks up to 79): 4.25 ms per
+// application on the grouped and per-wave tiles, 2.3 with this kernel on two
+// register sets of each operand and two waves per SIMD, 1.96 so.  Measured and
+// not kept: five panels to a workgroup (2.68), a launch of its own for C up to
+// 64 x 64 with the LDS for it (2.22 to 2.31 where one launch took 2.22).
 struct PanelPair {
   int64_t a, c, b;       // offsets; a, b < 0: identity
   double alpha;
   int32_t k1, k2, trans, pad;  // trans: bit 0 op(A) stored k1 x m, bit 1 B' stored n x k2
 };
 
+constexpr int WAIT_VM0 = 0x0f70;  // s_waitcnt: no vector load under way
 constexpr int PANEL_MAX = 80;  // rows, columns and contraction depths the kernel takes
 // LDS place of C(k, col): 16-byte pairs of K, the eight pairs of 16 K in an
-// order that lets 8 lanes (columns 0, 4, 8, 12, 1, 5, 9, 13 or those two on)
-// meet every bank once
+// order that lets the lanes of 8 successive columns meet every bank once
 __device__ __forceinline__ int panel_at(int col, int k, int kp) {
-  const int f = ((col >> 2) & 3) | ((col & 1) << 2);
+  const int f = col & 7;
   return col * kp + (k & ~15) + ((((k >> 1) ^ f) & 7) << 1) + (k & 1);
 }
 
 // One run of pairs with the same C block, k1 <= 16 KB and n <= 16 NB (a whole
-// wavefront: rows row0 .. row0 + 15 of the block)
-// stage() puts C into LDS (between barriers) once the first pair's loads are
-// under way.
+// wavefront: rows row0 .. row0 + 15 of the block).  stage() puts C into LDS
+// (between barriers) once the first pair's loads are under way.
 template <int KB, int NB, class F>
 __device__ __forceinline__ void panel_run(const PanelPair* __restrict__ prs, int count,
                                           const double* __restrict__ arena, const double* cl, int kp, int m, int n,
@@ -43,45 +51,41 @@ __device__ __forceinline__ void panel_run(const PanelPair* __restrict__ prs, int
   // (row row0 + li) and B' (column li of a 16-column group)
   const uint32_t oa0 = (uint32_t)((row0 + li) * k1 + 2 * lk) * 8u;   // m x k1, K contiguous
   const uint32_t oa1 = (uint32_t)(2 * lk * m + row0 + li) * 8u;      // k1 x m
-  const uint32_t ob0 = (uint32_t)(4 * lk * n + li) * 8u;             // k2 x n
-  const uint32_t ob1 = (uint32_t)(li * k2 + 4 * lk) * 8u;            // n x k2, K contiguous
+  const uint32_t ob0 = (uint32_t)(2 * lk * n + li) * 8u;             // k2 x n
+  const uint32_t ob1 = (uint32_t)(li * k2 + 2 * lk) * 8u;            // n x k2, K contiguous
   const double* cp[2];  // this lane's C^T row of a 16-column group (permuted), K pairs lk and 4 + lk
   {
-    const int col = 4 * (li & 3) + (li >> 2);
+    const int col = 8 * (li >> 3) + 2 * (li & 3) + ((li >> 2) & 1);
     cp[0] = cl + panel_at(col, 2 * lk, kp);
     cp[1] = cl + panel_at(col, 8 + 2 * lk, kp);
   }
-  dbl2 an[2 * KB], bn[2 * NB];
+  dbl2 a[2 * KB];
+  dbl2 b[2][NB];
   auto load_a = [&](const PanelPair& p) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t r = block_rsrc(arena + p.a, (int64_t)m * k1);
-    if (p.trans & 1) {
+    const bool ta = p.trans & 1;
+    const uint32_t oa = ta ? oa1 : oa0, ak = ta ? 8u * m : 8u;
 #pragma unroll
-      for (int s = 0; s < 2 * KB; ++s)
-        if (s < nk) {
-          an[s][0] = bload2(r, oa1, (uint32_t)(8 * s * m) * 8u);
-          an[s][1] = bload2(r, oa1, (uint32_t)(8 * s * m + m) * 8u);
-        }
-    } else {
-#pragma unroll
-      for (int s = 0; s < 2 * KB; ++s)
-        if (s < nk) an[s] = bload128(r, oa0, 64u * s);
-    }
+    for (int s = 0; s < 2 * KB; ++s)
+      if (s < nk) {
+        a[s][0] = bload2(r, oa, (uint32_t)(8 * s) * ak);
+        a[s][1] = bload2(r, oa, (uint32_t)(8 * s + 1) * ak);
+      }
   };
   auto load_b = [&](const PanelPair& p, int jb) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t r = block_rsrc(arena + p.b, (int64_t)n * k2);
     if (p.trans & 2) {
 #pragma unroll
-      for (int t = 0; t < NB; ++t) {
-        const uint32_t o = ob1 + (uint32_t)(t * k2) * 128u;
-        bn[2 * t] = bload128(r, o, 128u * jb);
-        bn[2 * t + 1] = bload128(r, o + 16u, 128u * jb);
-      }
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int t = 0; t < NB; ++t) b[i][t] = bload128(r, ob1, (uint32_t)(16 * jb + 8 * i) * 8u + (uint32_t)(t * k2) * 128u);
     } else {
-      const uint32_t s0 = (uint32_t)(jb * n) * 128u;
 #pragma unroll
-      for (int t = 0; t < NB; ++t)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) bn[2 * t + (i >> 1)][i & 1] = bload2(r, ob0 + 128u * t, s0 + (uint32_t)(i * n) * 8u);
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+          for (int t = 0; t < NB; ++t) b[i][t][e] = bload2(r, ob0, (uint32_t)((16 * jb + 8 * i + e) * n) * 8u + 128u * t);
     }
   };
   PanelPair cur = prs[0];
@@ -89,40 +93,49 @@ __device__ __forceinline__ void panel_run(const PanelPair* __restrict__ prs, int
   load_a(cur);
   load_b(cur, 0);
   stage();
-  for (int q = 0; q < count; ++q) {
-    dbl2 a[2 * KB];
+  // register i of lane (li, lk): W(row0 + li, 16 jb + 8 (i >> 1) + 2 lk + (i & 1))
+  auto first = [&](int jb) __attribute__((always_inline)) {
+    dbl4 w = dbl4{0.0, 0.0, 0.0, 0.0};
+    const int o = jb * 16 * kp;
 #pragma unroll
-    for (int s = 0; s < 2 * KB; ++s) a[s] = an[s];
-    const PanelPair pr = cur;
+    for (int s = 0; s < 2 * KB; ++s)
+      if (s < nk) {
+        const dbl2 x = *(const dbl2*)(cp[s & 1] + o + (s >> 1) * 16);
+        w = __builtin_amdgcn_mfma_f64_16x16x4f64(x[0], a[s][0], w, 0, 0, 0);
+        w = __builtin_amdgcn_mfma_f64_16x16x4f64(x[1], a[s][1], w, 0, 0, 0);
+      }
+    return w;
+  };
+  auto second = [&](dbl4 w, double alpha, int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const double wv = alpha * w[2 * i + e];
+#pragma unroll
+      for (int t = 0; t < NB; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(wv, b[i][t][e], acc[t], 0, 0, 0);
+    }
+  };
+  const bool half = ((k2 - 1) & 15) < 8;  // the last 16 W columns' upper half is empty
+  for (int q = 0; q < count; ++q) {
+    const double alpha = cur.alpha;
+    for (int jb = 0; jb + 1 < njb; ++jb) {
+      const dbl4 w = first(jb);
+      __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+      second(w, alpha, 0);
+      second(w, alpha, 1);
+      load_b(cur, jb + 1);
+    }
+    const dbl4 w = first(njb - 1);
     cur = nxt;
     if (q + 2 < count) nxt = prs[q + 2];
+    // explicit waits for B', then for op(A): both were requested a product
+    // earlier, and without them the compiler, which cannot count the loads of
+    // a storage order it does not know, waits for the newest ones too
+    __builtin_amdgcn_s_waitcnt(WAIT_VM0);
     if (q + 1 < count) load_a(cur);
-    for (int jb = 0; jb < njb; ++jb) {
-      dbl2 b[2 * NB];
-#pragma unroll
-      for (int t = 0; t < 2 * NB; ++t) b[t] = bn[t];
-      if (jb + 1 < njb)
-        load_b(pr, jb + 1);
-      else if (q + 1 < count)
-        load_b(cur, 0);
-      // register i of lane (li, lk): W(row0 + li, 16 jb + 4 lk + i)
-      dbl4 w = dbl4{0.0, 0.0, 0.0, 0.0};
-      const int o = jb * 16 * kp;
-#pragma unroll
-      for (int s = 0; s < 2 * KB; ++s)
-        if (s < nk) {
-          const dbl2 x = *(const dbl2*)(cp[s & 1] + o + (s >> 1) * 16);
-          w = __builtin_amdgcn_mfma_f64_16x16x4f64(x[0], a[s][0], w, 0, 0, 0);
-          w = __builtin_amdgcn_mfma_f64_16x16x4f64(x[1], a[s][1], w, 0, 0, 0);
-        }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const double wv = pr.alpha * w[i];
-#pragma unroll
-        for (int t = 0; t < NB; ++t)
-          acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(wv, b[2 * t + (i >> 1)][i & 1], acc[t], 0, 0, 0);
-      }
-    }
+    second(w, alpha, 0);
+    if (!half) second(w, alpha, 1);
+    __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+    if (q + 1 < count) load_b(cur, 0);
   }
 }
 
@@ -241,10 +254,9 @@ __device__ __forceinline__ void panel_unit(const Seg& sg, const bsg_vblock_t& vb
 }
 
 // KB: 16-deep groups of k1 the registers hold, also the largest V column
-// group count and C^T size: 3 (up to 48, three waves per SIMD) or 5 (up to
-// 80, two).
+// group count and C^T size: 3 (up to 48) or 5 (up to 80).
 template <int KB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KB <= 3 ? 3 : 2))) void k_panel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_panel(
     const bsg_vblock_t* __restrict__ vbs, const PanelPair* __restrict__ prs, const Seg* __restrict__ segs,
     const TileRef* __restrict__ tiles, int ntiles, const double* __restrict__ arena, const double* __restrict__ c,
     double* __restrict__ v, double* __restrict__ part, RootSet rs) {

@@ -2142,6 +2142,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
           const int np = (vb.m + 15) / 16;
           gu.ntm = (np + 3) / 4;                    // workgroups
           gu.code = (np + gu.ntm - 1) / gu.ntm;     // panels of each
+          gu.cost = ucost * np / gu.ntm;            // of its wavefronts that have a panel
           gu.ntn = 1;
           L.punits[kind == UK_PANEL5].push_back(gu);
         } else {
