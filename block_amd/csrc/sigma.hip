@@ -1269,6 +1269,27 @@ inline long pair_cost(const Geom& g, int n, const bsg_pair_t& pr) {
   return g1 + g2 + 16 * nch;
 }
 
+// (cost, index) pairs, given by ascending index, to descending cost: counted
+// into place where the costs are few (a rotation's tens of thousands of
+// one-pair units; comparing them took a third of its plan's time)
+inline void costliest_first(std::vector<std::pair<long, int>>& v) {
+  constexpr long MOST = 1 << 16;
+  long top = 0;
+  for (const auto& x : v) top = std::max(top, x.first);
+  if (v.size() < 512 || top >= MOST) {
+    std::sort(v.begin(), v.end(), [](const std::pair<long, int>& a, const std::pair<long, int>& b) {
+      return a.first != b.first ? a.first > b.first : a.second < b.second;
+    });
+    return;
+  }
+  std::vector<int32_t> at(top + 2, 0);
+  for (const auto& x : v) ++at[top - x.first + 1];
+  for (long k = 1; k <= top + 1; ++k) at[k] += at[k - 1];
+  std::vector<std::pair<long, int>> to(v.size());
+  for (const auto& x : v) to[at[top - x.first]++] = x;
+  v.swap(to);
+}
+
 // Launch order of the grouped kernel's tiles.  Workgroup i runs on XCD
 // i mod 8, each XCD with its own L2: the tiles of one work unit share their
 // C and B' blocks, so a unit's tiles go to one XCD, units are spread over
@@ -1286,9 +1307,7 @@ inline std::vector<TileRef> xcd_order(std::vector<GUnit>& units) {
   // (work, index) pairs sorted by work descending, index ascending on ties
   std::vector<std::pair<long, int>> ord(units.size());
   for (size_t i = 0; i < ord.size(); ++i) ord[i] = {units[i].cost * units[i].ntiles(), (int)i};
-  std::sort(ord.begin(), ord.end(), [](const std::pair<long, int>& a, const std::pair<long, int>& b) {
-    return a.first != b.first ? a.first > b.first : a.second < b.second;
-  });
+  costliest_first(ord);
   std::vector<std::vector<TileRef>> q(NXCD);
   for (auto& v : q) v.reserve(units.size() / NXCD + 16);
   long load[NXCD] = {};
@@ -2047,7 +2066,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       // the kernels that keep C read them; pad: pairs left in the run on one C
       // block
       auto cut_by_c = [&](std::vector<int>& list, int kind) {
-        std::stable_sort(list.begin(), list.end(), [&](int x, int y) {
+        if (list.size() > 1) std::stable_sort(list.begin(), list.end(), [&](int x, int y) {
           const bsg_pair_t &a = perm[x], &b = perm[y];
           if (a.c_off != b.c_off) return a.c_off < b.c_off;
           return (a.a_off < 0 || a.b_off < 0) && !(b.a_off < 0 || b.b_off < 0);
@@ -2244,9 +2263,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
   // small-block units, costliest first
   for (int k = 0; k < 3; ++k) {
     auto& su = sunits[k];
-    std::sort(su.begin(), su.end(), [](const std::pair<long, int>& x, const std::pair<long, int>& y) {
-      return x.first != y.first ? x.first > y.first : x.second < y.second;
-    });
+    costliest_first(su);
     std::vector<int32_t> sq;
     sq.reserve(su.size());
     for (const auto& x : su) sq.push_back(x.second);
@@ -2271,9 +2288,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     std::vector<std::pair<long, int>> order;
     for (int u = 0; u < (int)wunits[k].size(); ++u)
       order.push_back({wunits[k][u].cost * wunits[k][u].ntm * wunits[k][u].ntn, u});
-    std::sort(order.begin(), order.end(), [](const std::pair<long, int>& x, const std::pair<long, int>& y) {
-      return x.first != y.first ? x.first > y.first : x.second < y.second;
-    });
+    costliest_first(order);
     std::vector<TileRef> q[8];
     long load[8] = {};
     for (const auto& o : order) {
