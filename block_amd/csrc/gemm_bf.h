@@ -11,6 +11,8 @@
 // Bound by L2 and LDS traffic: a slice element is 6 bytes for 32 / 6 of the
 // FP64 kernel's product rate, so the tile is as large as the registers of two
 // waves per SIMD hold (128 x 128: 12 TB/s at full rate, half of a 64 x 64's).
+// 24 orbitals, C1, M = 500: 4.90 ms per application on 16-row tiles that read
+// every slice fragment for 16 rows, 2.70 so.
 
 // spaces of a segment's operands
 enum : int32_t { BS_OPER = 0, BS_W = 1, BS_C = 2 };

@@ -7,6 +7,13 @@
 // wavefront) and walks a list of segments, out += alpha L_s R_s, as one
 // contraction: one segment for W, the unit's run of pairs for V.  A pair with
 // an identity partner is a single segment of the second kind.
+//
+// Bound by the FP64 matrix pipes (62% of the rate their instruction reaches by
+// itself; the rest is VALU work beside them and tile edges).  24 orbitals, C1,
+// M = 500 (169 GFLOP): 6.19 ms per application on 16-row tiles that kept W on
+// chip and read C and B' per 16 rows, 3.94 so (43 TFLOP/s); 30 orbitals, M =
+// 800, four roots: 114.4 -> 69.7 ms.  At the time of 4.59 ms, 128 x 64 tiles
+// of four wavefronts took 5.57, five waves per SIMD instead of four 5.81.
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 __device__ inline dbl2 bload128(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
   return __builtin_bit_cast(dbl2, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
@@ -40,8 +47,7 @@ struct GemmUnit {
 constexpr int GKC = 16;      // K depth of a staged chunk
 // LDS layout of a chunk: 16 doubles per row, the eight 16-byte pairs of K of
 // row r in the order (pair ^ (r & 7)): 8 lanes reading the same pair of 8 rows,
-// or writing the 8 pairs of one row, meet every bank once without padding
-// (a padded 128 x 64 tile would leave a third workgroup no room).
+// or writing the 8 pairs of one row, meet every bank once without padding.
 __device__ __forceinline__ int chunk_at(int row, int k) { return row * GKC + ((((k >> 1) ^ row) & 7) << 1) + (k & 1); }
 
 // One operand of a segment as a thread stages it: 64 rows of the operand x 16

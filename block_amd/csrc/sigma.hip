@@ -4,17 +4,17 @@
 // of operatorfunctions.C:485-537), grouped by the V block they update:
 //   W = alpha_a op(A) C        (first GEMM, operatorfunctions.C:512-516)
 //   V += alpha W op(B)^T       (second GEMM, operatorfunctions.C:530)
-// k_sigma fuses both: a workgroup owns one V tile and walks a slice of that
-// block's pair list in order; for every pair it builds W in LDS chunk by
-// chunk (MFMA over the A.C contraction) and immediately contracts it with
-// B into the V accumulator, so W never travels to HBM.  Tile classes: basic
-// tiles (up to 64 rows, 4 wavefronts of 32 x 32 or 16 x 64), and wide
-// 16-row tiles of 256, 384 (4 wavefronts) or 768 columns (8 wavefronts in
-// one row), so a wide V block forms each W column once per row panel;
-// v_mfma_f64_16x16x4f64 throughout.  k_sigma_bf is the same on pre-split
-// BF16 slices (v_mfma_f32_16x16x32_bf16, 256- and 512-wide tiles), k_small
-// gives V blocks up to 32 x 32 one wavefront each.  Long pair lists are cut
-// into work units whose partial tiles k_reduce adds in list order, so V is
+// By the size of the V block and of a pair's depths:
+//   up to 32: k_small (small_f64.h), a wavefront per work unit, W in registers;
+//   up to 80, FP64: k_panel (panel_f64.h), 16 rows per wavefront, C in LDS;
+//   33 to 64, split precision: k_sigma_bf, a workgroup per V tile that forms W
+//   in LDS chunks from pre-split BF16 slices (v_mfma_f32_16x16x32_bf16) and
+//   contracts each with B' at once;
+//   larger: k_gemm (gemm_f64.h) and k_gemm_bf (gemm_bf.h), the two products as
+//   LDS tiles of their own, W in scratch.
+// k_sigma (k_sigma_bf's FP64 counterpart) and k_wave (one 16-row tile per
+// wavefront) run where a tile-table rule names them.  Long pair lists are cut
+// into work units whose partial tiles k_reduce adds in a fixed order, so V is
 // reduced without atomics and bitwise reproducibly.
 #include <hip/hip_runtime.h>
 
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void k_reduce(const RedItem* __restrict__ item
 }
 
 // ---------------------------------------------------------------- FP64 grouped kernel
-// One launch covers every V block.  A workgroup of 4 wavefronts owns a V
+// Runs by tile-table rule.  A workgroup of 4 wavefronts owns a V
 // panel tile: rows [row0, row0 + TM) and one column group of width JC (the
 // whole block when n <= JC), with the waves arranged WR x WC (WR WC = 4),
 // each wave owning NR 16-row blocks and PB = 2 16-wide column blocks (wc,
