@@ -4,13 +4,13 @@
 // Every pair of a V block that reads the same C block needs the same C
 // operands, so the planner orders a block's pairs by C block and a workgroup
 // keeps C in LDS (transposed, zero-padded to 16s) while it walks them.  A
-// wavefront owns 16 rows of the V block (all its columns, up to 80): per pair
+// wavefront owns 16 rows of the V block (all its columns, up to 96): per pair
 // it holds its rows of op(A) in registers, forms W^T = C^T op(A)^T 16 W columns
 // at a time (C^T from LDS), and the result registers are at once the A operand
 // of the product with B'.  What a wavefront streams per pair is op(A)'s rows
 // and B'.  Each has one register set, requested as soon as the product that
 // reads it is done and while the other product runs, which leaves room for
-// three waves per SIMD.  The waves of a workgroup (the 16-row panels of one
+// three waves per SIMD up to 80.  The waves of a workgroup (the 16-row panels of one
 // V block) meet only where the C block changes.
 //
 // K order: step (s, e) of lane lk is 8 s + 2 lk + e in both products, so that
@@ -31,7 +31,7 @@ struct PanelPair {
 };
 
 constexpr int WAIT_VM0 = 0x0f70;  // s_waitcnt: no vector load under way
-constexpr int PANEL_MAX = 80;  // rows, columns and contraction depths the kernel takes
+constexpr int PANEL_MAX = 96;  // rows, columns and contraction depths the kernel takes
 // LDS place of C(k, col): 16-byte pairs of K, the eight pairs of 16 K in an
 // order that lets the lanes of 8 successive columns meet every bank once
 __device__ __forceinline__ int panel_at(int col, int k, int kp) {
@@ -254,9 +254,13 @@ __device__ __forceinline__ void panel_unit(const Seg& sg, const bsg_vblock_t& vb
 }
 
 // KB: 16-deep groups of k1 the registers hold, also the largest V column
-// group count and C^T size: 3 (up to 48) or 5 (up to 80).
+// group count and C^T size: 3 (up to 48), 5 (up to 80) or 6 (up to 96, two
+// waves per SIMD and two workgroups per CU: on blocks of 81 to 96 still faster
+// than 64 x 64 product tiles, which pad them to 128: 24 orbitals, D2h, peak
+// dimension 90 1.77 -> 1.44 ms, 100 2.70 -> 1.98; 112 would leave one
+// workgroup per CU).
 template <int KB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_panel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KB <= 5 ? 3 : 2))) void k_panel(
     const bsg_vblock_t* __restrict__ vbs, const PanelPair* __restrict__ prs, const Seg* __restrict__ segs,
     const TileRef* __restrict__ tiles, int ntiles, const double* __restrict__ arena, const double* __restrict__ c,
     double* __restrict__ v, double* __restrict__ part, RootSet rs) {
@@ -290,7 +294,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   else if constexpr (KB > 3) {
     if (nb == 4)
       panel_unit<KB, 4>(sg, vb, prs, arena, c, v, part, cl, row0, tid, nt);
-    else
+    else if (KB <= 5 || nb == 5)
       panel_unit<KB, 5>(sg, vb, prs, arena, c, v, part, cl, row0, tid, nt);
+    else if constexpr (KB > 5)
+      panel_unit<KB, 6>(sg, vb, prs, arena, c, v, part, cl, row0, tid, nt);
   }
 }

@@ -6,7 +6,7 @@
 //   V += alpha W op(B)^T       (second GEMM, operatorfunctions.C:530)
 // By the size of the V block and of a pair's depths:
 //   up to 32: k_small (small_f64.h), a wavefront per work unit, W in registers;
-//   up to 80, FP64: k_panel (panel_f64.h), 16 rows per wavefront, C in LDS;
+//   up to 96, FP64: k_panel (panel_f64.h), 16 rows per wavefront, C in LDS;
 //   33 to 64, split precision: k_sigma_bf, a workgroup per V tile that forms W
 //   in LDS chunks from pre-split BF16 slices (v_mfma_f32_16x16x32_bf16) and
 //   contracts each with B' at once;
@@ -1529,8 +1529,8 @@ struct ModeLists {
   int n_s[3] = {};
   TileRef* d_w[2] = {};          // FP64 per-wave tiles (16 x 32, 16 x 64), 4 per workgroup (item -1: none), a multiple of 32
   int n_w[2] = {};
-  TileRef* d_p[2] = {};          // FP64 panels (KB = 3, 5)
-  int n_p[2] = {};
+  TileRef* d_p[3] = {};          // FP64 panels (KB = 3, 5, 6)
+  int n_p[3] = {};
   PanelPair* d_pp = nullptr;     // pairs of the panels and small blocks
   GemmUnit* d_gu = nullptr;      // FP64 product tiles, by round
   GemmSeg* d_gs = nullptr;
@@ -1815,7 +1815,7 @@ struct Blob {
 };
 
 // kernels a work unit runs on
-enum UnitKind : char { UK_GROUPED = 0, UK_WAVE = 2, UK_GEMM = 3, UK_PANEL3 = 4, UK_PANEL5 = 5, UK_SMALL = 6 /* + class 0 .. 2 */ };
+enum UnitKind : char { UK_GROUPED = 0, UK_WAVE = 2, UK_GEMM = 3, UK_PANEL = 4 /* + class 0 .. 2 */, UK_SMALL = 7 /* + class 0 .. 2 */ };
 
 // MFMAs per wavefront of a work unit before its pair list is split (small
 // blocks: by width class; half as much or twice as much in the first two
@@ -2008,7 +2008,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     std::vector<GUnit> gunits[NCLS];                 // grouped tiles by kernel class
     std::vector<std::pair<long, int>> sunits[3];     // (cost, segment) of small-block units (up to 16, 24, 32)
     std::vector<int> bunits;                         // large blocks' units (segments)
-    std::vector<GUnit> wunits[2], punits[2];         // per-wave tiles (16 x 32, 16 x 64), panels (KB = 3, 5)
+    std::vector<GUnit> wunits[2], punits[3];         // per-wave tiles (16 x 32, 16 x 64), panels (KB = 3, 5, 6)
     std::vector<int> gq;                             // pairs of the large blocks' units (indices into h_perm)
     std::vector<PanelPair> pp;
     std::vector<Seg> segs;
@@ -2018,11 +2018,17 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
   std::vector<Local> loc(MAX_PLAN_THREADS);
   const long fill = std::max(SEG_COST_MIN, (long)(pc.flops / (2048.0 * UNITS_MIN)));
   const int nvb = (int)pc.h_vb.size();
+  // the widest panels wait for each other's few workgroups beside blocks much
+  // larger than they are (C1, peak dimension 313: 4.05 ms for 3.94 with product
+  // tiles from 81 on; 120: 437 us for 466)
+  int widest = 0;
+  for (const bsg_vblock_t& vb : pc.h_vb) widest = std::max(widest, std::max(vb.m, vb.n));
+  const int panel_max = widest <= 2 * PANEL_MAX ? PANEL_MAX : 80;
   const int nth = over_vblocks(pc.h_vb.data(), nvb, pc.n_pairs, [&](int t, int i0, int i1) {
     Local& L = loc[t];
     std::vector<std::pair<int, int>> units;  // (first, count)
     std::vector<char> ukind;
-    std::vector<int> pan[2], big, few[3];
+    std::vector<int> pan[3], big, few[3];
     for (int i = i0; i < i1; ++i) {
       const bsg_vblock_t& vb = pc.h_vb[i];
       const bsg_pair_t* perm = pc.h_perm.get();
@@ -2040,8 +2046,9 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
           case UK_SMALL + 2: return small_cost(vb.m, vb.n, pr);
           case UK_WAVE: return wave_cost(vb.n, pr);
           case UK_GEMM: return gemm_cost(pr);
-          case UK_PANEL3:
-          case UK_PANEL5: return panel_cost(vb.n, pr);
+          case UK_PANEL:
+          case UK_PANEL + 1:
+          case UK_PANEL + 2: return panel_cost(vb.n, pr);
           default: return pair_cost(g, vb.n, pr);
         }
       };
@@ -2101,19 +2108,19 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
           g = pick_geom(*p->rules, vb.m, vb.n, split ? 4 : 6);
           cut(base + slow, ntot - slow, UK_GROUPED, in_perm(base + slow));
         } else {
-          const bool med = !split && std::max(vb.m, vb.n) <= PANEL_MAX;
+          const bool med = !split && std::max(vb.m, vb.n) <= panel_max;
           for (auto& x : pan) x.clear();
           big.clear();
           for (int q = base + slow; q < base + ntot; ++q) {
             if (few_pair(q)) continue;
             const int k = std::max(perm[q].k1, perm[q].k2);
-            if (!med || k > PANEL_MAX)
+            if (!med || k > panel_max)
               big.push_back(q);
             else
-              pan[k > 48 || vb.n > 48].push_back(q);
+              pan[std::max(k, vb.n) <= 48 ? 0 : (std::max(k, vb.n) <= 80 ? 1 : 2)].push_back(q);
           }
-          for (int k = 0; k < 2; ++k)
-            if (!pan[k].empty()) cut_by_c(pan[k], k ? UK_PANEL5 : UK_PANEL3);
+          for (int k = 0; k < 3; ++k)
+            if (!pan[k].empty()) cut_by_c(pan[k], UK_PANEL + k);
           if (!big.empty()) {
             const int first = (int)L.gq.size();
             L.gq.insert(L.gq.end(), big.begin(), big.end());
@@ -2139,7 +2146,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
           continue;
         }
         long ucost = 0;
-        if (kind == UK_PANEL3 || kind == UK_PANEL5)
+        if (kind >= UK_PANEL && kind < UK_SMALL)
           for (int q = 0; q < sg.count; ++q) ucost += panel_cost(vb.n, L.pp[sg.first + q]);
         else if (kind >= UK_SMALL)
           for (int q = 0; q < sg.count; ++q) ucost += small_cost(vb.m, vb.n, L.pp[sg.first + q]);
@@ -2157,13 +2164,13 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
           gu.ntm = (vb.m + 15) / 16;
           gu.ntn = (vb.n + 16 * nb - 1) / (16 * nb);
           L.wunits[nb == 4].push_back(gu);
-        } else if (kind == UK_PANEL3 || kind == UK_PANEL5) {
+        } else if (kind >= UK_PANEL && kind < UK_SMALL) {
           const int np = (vb.m + 15) / 16;
           gu.ntm = (np + 3) / 4;                    // workgroups
           gu.code = (np + gu.ntm - 1) / gu.ntm;     // panels of each
           gu.cost = ucost * np / gu.ntm;            // of its wavefronts that have a panel
           gu.ntn = 1;
-          L.punits[kind == UK_PANEL5].push_back(gu);
+          L.punits[kind - UK_PANEL].push_back(gu);
         } else {
           gu.ntm = (vb.m + g.tm - 1) / g.tm;
           gu.ntn = (vb.n + g.jv - 1) / g.jv;
@@ -2187,7 +2194,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     }
   });
   // concatenate with the local indices shifted
-  std::vector<GUnit> gunits[NCLS], wunits[2], punits[2];
+  std::vector<GUnit> gunits[NCLS], wunits[2], punits[3];
   std::vector<std::pair<long, int>> sunits[3];
   std::vector<int> bunits, gq;
   std::vector<PanelPair> pp;
@@ -2199,9 +2206,11 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     for (int k = 0; k < NCLS; ++k) gunits[k].swap(L.gunits[k]);
     for (int k = 0; k < 2; ++k) {
       wunits[k].swap(L.wunits[k]);
-      punits[k].swap(L.punits[k]);
     }
-    for (int k = 0; k < 3; ++k) sunits[k].swap(L.sunits[k]);
+    for (int k = 0; k < 3; ++k) {
+      punits[k].swap(L.punits[k]);
+      sunits[k].swap(L.sunits[k]);
+    }
     bunits.swap(L.bunits);
     gq.swap(L.gq);
     pp.swap(L.pp);
@@ -2218,10 +2227,10 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       Local& L = loc[t];
       const int sb = (int)segs.size(), ppb = (int)pp.size(), gb = (int)gq.size();
       std::vector<char> kind(L.segs.size(), 0);  // 1: the unit's pairs are in pp, 2: in gq
-      for (int k = 0; k < 2; ++k)
+      for (int k = 0; k < 3; ++k) {
         for (const GUnit& u : L.punits[k]) kind[u.seg] = 1;
-      for (int k = 0; k < 3; ++k)
         for (const auto& x : L.sunits[k]) kind[x.second] = 1;
+      }
       for (int s : L.bunits) kind[s] = 2;
       for (size_t s = 0; s < L.segs.size(); ++s) {
         Seg sg = L.segs[s];
@@ -2238,10 +2247,11 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       for (int k = 0; k < NCLS; ++k) shift(gunits[k], L.gunits[k]);
       for (int k = 0; k < 2; ++k) {
         shift(wunits[k], L.wunits[k]);
-        shift(punits[k], L.punits[k]);
       }
-      for (int k = 0; k < 3; ++k)
+      for (int k = 0; k < 3; ++k) {
+        shift(punits[k], L.punits[k]);
         for (auto x : L.sunits[k]) sunits[k].push_back({x.first, x.second + sb});
+      }
       for (int s : L.bunits) bunits.push_back(s + sb);
       gq.insert(gq.end(), L.gq.begin(), L.gq.end());
       pp.insert(pp.end(), L.pp.begin(), L.pp.end());
@@ -2275,7 +2285,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     blob.add(&ml.d_g[k], t);
     ml.n_g[k] = (int)t.size();
   }
-  for (int k = 0; k < 2; ++k) {
+  for (int k = 0; k < 3; ++k) {
     const std::vector<TileRef> t = xcd_order(punits[k]);
     blob.add(&ml.d_p[k], t);
     ml.n_p[k] = (int)t.size();
@@ -2814,6 +2824,11 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
       ++nl;
     }
   } else {
+    if (ml.n_p[2] > 0) {
+      hipLaunchKernelGGL((k_panel<6>), grid(ml.n_p[2]), dim3(256), 0, st, ch.d_vb, ml.d_pp, ml.d_seg, ml.d_p[2],
+                         ml.n_p[2], arena, c, v, part, rs);
+      ++nl;
+    }
     if (ml.n_p[1] > 0) {
       hipLaunchKernelGGL((k_panel<5>), grid(ml.n_p[1]), dim3(256), 0, st, ch.d_vb, ml.d_pp, ml.d_seg, ml.d_p[1],
                          ml.n_p[1], arena, c, v, part, rs);

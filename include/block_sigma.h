@@ -139,7 +139,7 @@ int bsg_plan_split_arena(bsg_context* ctx, bsg_plan* plan, const double* arena, 
  * int32 (m_lo, m_hi, n_lo, n_hi, fp64, split); a V block of m x n inside a
  * rule's ranges gets tile geometry number fp64 (FP64 grouped kernel) or split
  * (split-precision kernels) of the candidate list, -1 leaving the default (FP64:
- * panels for blocks and contraction depths up to 80, product tiles above;
+ * panels for blocks and contraction depths up to 96 (80 in superblocks with a block past 192), product tiles above;
  * split: the MFMA-count model's geometry up to 64, product tiles above); the first matching rule applies.  Process-wide, read when
  * plans are created (n = 0 clears).  bsg_tile_candidates gives the list's
  * length for a precision.  For FP64 its last entry is not a geometry but the
