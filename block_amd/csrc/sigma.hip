@@ -2468,7 +2468,7 @@ namespace {
 // open-addressing tables (no allocation per entry), grown by doubling at
 // half load so that their size follows the distinct blocks, not the pairs:
 // keys of the operator blocks (offset, orientation, rows, cols) and of the
-// C blocks (offset)
+// C blocks (offset, rows, cols)
 struct SliceTable {
   struct E {
     int64_t off, key, val;  // off < 0: empty
@@ -2545,8 +2545,9 @@ int build_slices(bsg_plan* p) {
     return abt.get(off, key, [&] { return slice_of(p->ab_items, p->ab_elems, off, rows, cols, trans); });
   };
   auto c_slice = [&](int64_t off, int k1, int k2) {
-    // C^T: (j, p) = C[p k2 + j]
-    return ct.get(off, 0, [&] { return slice_of(p->c_items, p->c_elems, off, k2, k1, 1); });
+    // C^T: (j, p) = C[p k2 + j]; pairs may read one offset as different shapes
+    const int64_t key = ((int64_t)k1 << 32) | k2;
+    return ct.get(off, key, [&] { return slice_of(p->c_items, p->c_elems, off, k2, k1, 1); });
   };
   for (auto& pc : p->chunks) {
     std::vector<PairS>& ps = pc.h_ps;

@@ -1,0 +1,83 @@
+"""Work lists whose pairs or sizes take the plan's less common routes, through
+the C-ABI, against numpy."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import block_amd
+from capi import Device, check, lib, vp
+from test_gpu_products import PAIR, VBLOCK, Chunk, reference
+
+pytestmark = pytest.mark.gpu
+
+BOTH = pytest.mark.parametrize("precision", [block_amd.FP64, block_amd.SPLIT_BF16], ids=["fp64", "split"])
+
+
+class Plan:
+    """A plan of one chunk and its operator arena on the device."""
+
+    def __init__(self, d, vbs, prs, wave, arena, split=False):
+        self.d, self.wave, self.h = d, wave, vp()
+        chunk = Chunk(vbs.ctypes.data, len(vbs), prs.ctypes.data, len(prs))
+        check(lib.bsg_plan_create(d.ctx, ctypes.byref(chunk), 1, wave, ctypes.byref(self.h)))
+        self.arena, self.n = d.upload(arena), len(arena)
+        if split:
+            self.split()
+
+    def split(self):
+        check(lib.bsg_plan_split_arena(self.d.ctx, self.h, self.arena, self.n))
+
+    def apply(self, c, precision, call=lib.bsg_sigma_apply):
+        """H c for the rows of c in one call."""
+        c = np.atleast_2d(c)
+        dc, dv = self.d.upload(c), self.d.zeros(c.size)
+        check(call(self.d.ctx, self.h, self.arena, dc, dv, len(c), precision))
+        return self.d.download(dv, c.shape)
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *a):
+        lib.bsg_plan_destroy(self.h)
+
+
+def tolerance(vbs, prs, precision):
+    """Per sum of absolute products: each of a value's two nested sums of at
+    most `deep` products rounds once per addition, on both sides of the
+    comparison; split: operands rounded to 2^-24, the slice products left out
+    about 3 x 2^-24, FP32 sums of 6 x 32 terms per K group (at most 6 + 32
+    roundings), in each of the two products."""
+    deep = 4 * max(int(prs["k1"].max() + prs["k2"].max()), int(vbs["count"].max()))
+    tol = 2 * deep * np.finfo(float).eps
+    return tol + 2 * (2 + 3 + 38) * 2.0 ** -24 if precision == block_amd.SPLIT_BF16 else tol
+
+
+def agree(got, vbs, prs, c, arena, wave, precision):
+    ref, bound = reference(vbs, prs, c, arena, wave)
+    err = np.abs(got - ref)
+    assert np.all(err <= tolerance(vbs, prs, precision) * bound), float((err / np.maximum(bound, 1e-300)).max())
+
+
+@BOTH
+@pytest.mark.parametrize("m,n", [(90, 100), (40, 50), (20, 24)])
+def test_one_c_offset_as_different_shapes(m, n, precision):
+    """Pairs that read the same C offset as blocks of different shapes (of the
+    same and of different sizes)."""
+    print(f"[gpu] one C offset, {m} x {n}, precision {precision}", flush=True)
+    rng = np.random.default_rng(m)
+    depths = [(66, 70), (70, 66), (3, 100), (100, 3), (17, 17), (m, 40), (40, n)]
+    size = max(k1 * k2 for k1, k2 in depths)
+    prs, arena = [], 0
+    for k1, k2 in depths:
+        a, b = (-1 if k1 == m else arena), (-1 if k2 == n else arena + m * k1)
+        arena += m * k1 + k2 * n
+        prs.append((a, 0, b, k1, k2, int(rng.integers(2)), int(rng.integers(2)), 1.0, rng.uniform(0.5, 1.5)))
+    prs = np.array(prs, dtype=PAIR)
+    vbs = np.array([(size, m, n, 0, len(prs))], dtype=VBLOCK)
+    wave = size + m * n
+    ops = rng.standard_normal(arena)
+    c = np.zeros(wave)
+    c[:size] = rng.standard_normal(size)
+    with Device() as d, Plan(d, vbs, prs, wave, ops, precision == block_amd.SPLIT_BF16) as p:
+        agree(p.apply(c, precision)[0], vbs, prs, c, ops, wave, precision)
