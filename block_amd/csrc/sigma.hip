@@ -1539,6 +1539,8 @@ struct ModeLists {
   RedItem* d_red = nullptr;
   int n_red = 0;
   int64_t part_doubles = 0;
+  // whether an application launches anything on the side stream
+  bool side() const { return n_s[1] > 0 || n_s[2] > 0 || n_g[0] > 0 || n_p[0] > 0 || rounds.size() > 1; }
 };
 
 struct PlanChunk {
@@ -2744,7 +2746,7 @@ int enqueue_chunk(bsg_context* ctx, const bsg_plan* p, const PlanChunk& ch, cons
   // partial tiles, and the reduction waits for both
   const int nbasic = ml.n_g[0];
   const int *ns = ml.n_s;
-  const bool side = ns[1] > 0 || ns[2] > 0 || nbasic > 0 || ml.n_p[0] > 0 || ml.rounds.size() > 1;
+  const bool side = ml.side();
   // round r of the large blocks, in launches of the roots its scratch holds
   auto round = [&](size_t r, hipStream_t q) {
     const GemmRound& g = ml.rounds[r];
@@ -2998,7 +3000,13 @@ int bsg_sigma_profile(bsg_context* ctx, bsg_plan* p, const double* arena, const 
   const size_t nch = p->chunks.size();
   const int ngroups = (nvec + p->batch - 1) / p->batch;
   constexpr size_t per = 5;  // events per chunk launch (enqueue_chunk)
-  std::vector<hipEvent_t> ev((size_t)reps * ngroups * nch * per + 2);
+  struct Events : std::vector<hipEvent_t> {
+    using std::vector<hipEvent_t>::vector;
+    ~Events() {
+      for (hipEvent_t e : *this)
+        if (e) (void)hipEventDestroy(e);
+    }
+  } ev((size_t)reps * ngroups * nch * per + 2, nullptr);
   for (auto& e : ev) HIPCHK(hipEventCreate(&e));
   long disp = 0;
   HIPCHK(hipEventRecord(ev[0], ctx->stream));
@@ -3020,11 +3028,10 @@ int bsg_sigma_profile(bsg_context* ctx, bsg_plan* p, const double* arena, const 
   for (int r = 0; r < reps * ngroups; ++r)
     for (auto& ch : p->chunks) {
       const ModeLists& ml = ch.ml[split];
-      const bool sidek = ml.n_s[0] > 0 || ml.n_s[1] > 0 || ml.n_g[0] > 0 || ml.n_p[0] > 0 || ml.rounds.size() > 1;
       // [0] fork to join of all fused kernels, [1] reduction, [2] the side
       // stream's kernels alone
       const int from[3] = {0, 3, 1}, to[3] = {3, 4, 2};
-      const bool present[3] = {true, ml.n_red > 0, sidek};
+      const bool present[3] = {true, ml.n_red > 0, ml.side()};
       for (int i = 0; i < 3; ++i) {
         if (!present[i]) continue;
         HIPCHK(hipEventElapsedTime(&ms, ev[k + from[i]], ev[k + to[i]]));
@@ -3034,7 +3041,6 @@ int bsg_sigma_profile(bsg_context* ctx, bsg_plan* p, const double* arena, const 
     }
   // kernel dispatches of all applications (every kernel launch counted)
   launches[0] = disp;
-  for (auto& e : ev) HIPCHK(hipEventDestroy(e));
   return BSG_OK;
 }
 

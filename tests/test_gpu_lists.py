@@ -7,9 +7,11 @@ import pytest
 
 import block_amd
 from capi import Device, check, lib, vp
-from test_gpu_products import PAIR, VBLOCK, Chunk, reference
+from test_gpu_products import PAIR, VBLOCK, Chunk, reference, work_list
 
 pytestmark = pytest.mark.gpu
+lib.bsg_sigma_profile.restype = ctypes.c_int
+lib.bsg_sigma_profile.argtypes = [vp, vp, vp, vp, vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32] + [vp] * 3
 
 BOTH = pytest.mark.parametrize("precision", [block_amd.FP64, block_amd.SPLIT_BF16], ids=["fp64", "split"])
 
@@ -34,6 +36,14 @@ class Plan:
         dc, dv = self.d.upload(c), self.d.zeros(c.size)
         check(call(self.d.ctx, self.h, self.arena, dc, dv, len(c), precision))
         return self.d.download(dv, c.shape)
+
+    def profile(self, c, precision, reps=2):
+        """(wall ms, kernel ms, kernel launches of one application)"""
+        dc, dv = self.d.upload(c), self.d.zeros(c.size)
+        wall, ms, n = ctypes.c_double(), (ctypes.c_double * 3)(), (ctypes.c_long * 3)()
+        check(lib.bsg_sigma_profile(self.d.ctx, self.h, self.arena, dc, dv, 1, reps, precision, ctypes.byref(wall),
+                                    ms, n))
+        return wall.value, list(ms), n[0] // reps
 
     def __enter__(self):
         return self
@@ -81,3 +91,28 @@ def test_one_c_offset_as_different_shapes(m, n, precision):
     c[:size] = rng.standard_normal(size)
     with Device() as d, Plan(d, vbs, prs, wave, ops, precision == block_amd.SPLIT_BF16) as p:
         agree(p.apply(c, precision)[0], vbs, prs, c, ops, wave, precision)
+
+
+@BOTH
+@pytest.mark.parametrize("sides,depths,side", [
+    ([(16, 9), (3, 16)], [(16, 5), (8, 16)], False),    # nothing beside the main stream
+    ([(32, 25), (26, 32)], [(30, 5), (8, 27)], True),   # the widest small blocks alone
+    ([(16, 9), (70, 66)], [(16, 5), (70, 66)], None),   # with blocks of another kernel
+], ids=["to16", "to32", "mixed"])
+def test_profile(sides, depths, side, precision):
+    """The timing helper times every list; the side stream's time is there
+    exactly if the list has kernels that run there (both identity partners are
+    left out: split precision runs an identity A on another kernel)."""
+    print(f"[gpu] profile {sides} precision {precision}", flush=True)
+    rng = np.random.default_rng(3)
+    vbs, prs, wave, _, arena = work_list(rng, sides, depths, 2)
+    keep = (prs["a_off"] >= 0) & (prs["b_off"] >= 0)
+    for vb in vbs:
+        vb["count"] = keep[vb["first"]:vb["first"] + vb["count"]].sum()
+    prs = prs[keep]
+    vbs["first"] = np.concatenate([[0], np.cumsum(vbs["count"])[:-1]])
+    with Device() as d, Plan(d, vbs, prs, wave, arena, precision == block_amd.SPLIT_BF16) as p:
+        wall, ms, launches = p.profile(rng.standard_normal(wave), precision)
+    assert wall > 0.0 and ms[0] > 0.0 and launches >= 1
+    if side is not None:
+        assert (ms[2] > 0.0) == side
