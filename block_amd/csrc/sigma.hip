@@ -1866,7 +1866,8 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
   // an even number of rounds once W is large enough to be worth two
   int64_t nround = 1;
   if (wtot > W_ONE_ROUND) nround = 2 * ((wtot + W_HALF * 2 - 1) / (W_HALF * 2));
-  const int64_t target = (wtot + nround - 1) / std::max<int64_t>(1, nround);
+  // (no pair with a W: one round)
+  const int64_t target = std::max<int64_t>(1, (wtot + nround - 1) / nround);
   ml.rounds.reserve(nround + 2);
   std::vector<GUnit> uw[2], uv[2];
   int64_t wused = 0, wneed[2] = {};

@@ -116,3 +116,29 @@ def test_profile(sides, depths, side, precision):
     assert wall > 0.0 and ms[0] > 0.0 and launches >= 1
     if side is not None:
         assert (ms[2] > 0.0) == side
+
+
+@BOTH
+def test_large_blocks_without_w(precision):
+    """Large blocks whose pairs all have an identity partner and need no W:
+    their product tiles are one launch, not one per block."""
+    print(f"[gpu] large blocks without W, precision {precision}", flush=True)
+    rng = np.random.default_rng(4)
+    m, n, nb = 98, 103, 24
+    prs, arena = [], 0
+    for i in range(nb):
+        c = i * m * n
+        prs += [(arena, c, -1, m, n, i & 1, 0, -1.0, 0.75), (-1, c, -1, m, n, 0, 0, 1.0, 1.5)]
+        arena += m * m
+        if precision == block_amd.FP64:  # (split precision slices an identity A's W)
+            prs.append((-1, c, arena, m, n, 0, i & 1, 1.0, -0.5))
+            arena += n * n
+    prs, per, size = np.array(prs, dtype=PAIR), len(prs) // nb, nb * m * n
+    vbs = np.array([(size + i * m * n, m, n, per * i, per) for i in range(nb)], dtype=VBLOCK)
+    ops, c = rng.standard_normal(arena), np.zeros(2 * size)
+    c[:size] = rng.standard_normal(size)
+    with Device() as d, Plan(d, vbs, prs, 2 * size, ops, precision == block_amd.SPLIT_BF16) as p:
+        agree(p.apply(c, precision)[0], vbs, prs, c, ops, 2 * size, precision)
+        launches = p.profile(c, precision)[2]
+    # the products, split: the wavefunction's slices; units past one per block: their reduction
+    assert launches <= 3
