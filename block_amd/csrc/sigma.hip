@@ -1254,7 +1254,8 @@ inline long gemm_cost(const bsg_pair_t& pr) {
   return ((pr.b_off < 0 ? pr.k1 : pr.k2) + GKC - 1) / GKC * 16 + 4;
 }
 // W scratch of the large blocks' rounds, in doubles: one round up to
-// W_ONE_ROUND, else an even number of rounds of at most W_HALF each; roots
+// W_ONE_ROUND, else an even number of rounds of at most W_HALF each (W_HALF / 2
+// and one unit's W where that is more: blocks of some 20,000 rows); roots
 // share a launch while W_ROOTS holds all of them
 constexpr int64_t W_ONE_ROUND = 1 << 23, W_HALF = 1 << 26, W_ROOTS = 1 << 29, W_KEEP = 1 << 27;
 // MFMA instructions per wavefront of one pair in a tile (segment cost)
@@ -1846,7 +1847,7 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
   std::vector<GemmUnit> gu;
   std::vector<GemmSeg> gs;
   std::vector<GemmAdd> ga, wadd;
-  int64_t wtot = 0;
+  int64_t wtot = 0, wunit = 0;  // doubles of W: all units, the largest
   auto w_size = [&](const bsg_vblock_t& vb, const bsg_pair_t& pr) {
     if (pr.b_off < 0 || (pr.a_off < 0 && !split)) return (int64_t)0;
     const int64_t n = split ? (3 * (int64_t)vb.m * pad8(pr.k2) + 3) / 4 : (int64_t)vb.m * pr.k2;  // doubles
@@ -1856,16 +1857,22 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
   for (int bu : bunits) {
     const Seg& sg = segs[bu];
     const bsg_vblock_t& vb = pc.h_vb[sg.vb];
+    int64_t wu = 0;
     for (int q = 0; q < sg.count; ++q) {
       const bsg_pair_t& pr = perm[gq[sg.first + q]];
-      wtot += w_size(vb, pr);
+      wu += w_size(vb, pr);
       if (split) wide_tiles += ((vb.m + SplitBig::T - 1) / SplitBig::T) * (int64_t)((pr.k2 + SplitBig::T - 1) / SplitBig::T);
     }
+    wtot += wu;
+    wunit = std::max(wunit, wu);
   }
   const bool wide = wide_tiles >= SPLIT_WIDE;
   // an even number of rounds once W is large enough to be worth two
+  // (a round is closed by the unit that fills it, which may take it past the
+  // target by almost that unit's W)
+  const int64_t room = std::max(W_HALF / 2, W_HALF - wunit);
   int64_t nround = 1;
-  if (wtot > W_ONE_ROUND) nround = 2 * ((wtot + W_HALF * 2 - 1) / (W_HALF * 2));
+  if (wtot > W_ONE_ROUND) nround = 2 * ((wtot + room * 2 - 1) / (room * 2));
   // (no pair with a W: one round)
   const int64_t target = std::max<int64_t>(1, (wtot + nround - 1) / nround);
   ml.rounds.reserve(nround + 2);

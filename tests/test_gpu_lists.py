@@ -37,11 +37,11 @@ class Plan:
         check(call(self.d.ctx, self.h, self.arena, dc, dv, len(c), precision))
         return self.d.download(dv, c.shape)
 
-    def profile(self, c, precision, reps=2):
+    def profile(self, c, precision, reps=2, nvec=1):
         """(wall ms, kernel ms, kernel launches of one application)"""
         dc, dv = self.d.upload(c), self.d.zeros(c.size)
         wall, ms, n = ctypes.c_double(), (ctypes.c_double * 3)(), (ctypes.c_long * 3)()
-        check(lib.bsg_sigma_profile(self.d.ctx, self.h, self.arena, dc, dv, 1, reps, precision, ctypes.byref(wall),
+        check(lib.bsg_sigma_profile(self.d.ctx, self.h, self.arena, dc, dv, nvec, reps, precision, ctypes.byref(wall),
                                     ms, n))
         return wall.value, list(ms), n[0] // reps
 
@@ -142,3 +142,97 @@ def test_large_blocks_without_w(precision):
         launches = p.profile(c, precision)[2]
     # the products, split: the wavefunction's slices; units past one per block: their reduction
     assert launches <= 3
+
+
+class Products:
+    """V blocks of one shape with `count` pairs each, all pairs reading a few
+    operators (in both storage orders) and C blocks, so that numpy sums long
+    lists quickly."""
+
+    def __init__(self, rng, m, n, depths, count, blocks=1, reuse=3):
+        self.m, self.n = m, n
+        self.blocks, self.wave, arena, self.ops = [], 0, [], 0
+
+        def operator(rows, cols):
+            x, off = rng.standard_normal((rows, cols)), self.ops
+            arena.extend([x.ravel(), x.T.ravel()])
+            self.ops += 2 * x.size
+            return x, (off, off + x.size)
+
+        sets = []
+        for k1, k2 in depths:
+            cs = []
+            for _ in range(reuse):
+                cs.append(self.wave)
+                self.wave += k1 * k2
+            sets.append((k1, k2, [operator(m, k1) for _ in range(reuse)], cs, [operator(k2, n) for _ in range(reuse)]))
+        self.csize, self.terms, prs, vbs = self.wave, [], [], []
+        for _ in range(blocks):
+            first = len(prs)
+            mine = {}
+            for q in range(count):
+                s = q % len(sets)
+                k1, k2, a, c, b = sets[s]
+                i, j, l = rng.integers(reuse, size=3)
+                ta, tb = int(rng.integers(2)), int(rng.integers(2))
+                al = float(rng.uniform(0.5, 1.5) * rng.choice([-1.0, 1.0]))
+                prs.append((a[i][1][ta], c[j], b[l][1][tb], k1, k2, ta, tb, -1.0, al))
+                x = mine.setdefault((s, i, j, l), [0.0, 0.0])
+                x[0] -= al
+                x[1] += abs(al)
+            self.terms.append((self.wave, mine))
+            vbs.append((self.wave, m, n, first, count))
+            self.wave += m * n
+        self.sets, self.arena = sets, np.concatenate(arena)
+        self.vbs, self.prs = np.array(vbs, dtype=VBLOCK), np.array(prs, dtype=PAIR)
+
+    def vectors(self, rng, nroot):
+        c = np.zeros((nroot, self.wave))
+        c[:, :self.csize] = rng.standard_normal((nroot, self.csize))
+        return c
+
+    def agree(self, got, c, precision):
+        tol = tolerance(self.vbs, self.prs, precision)
+        assert np.all(got[:self.csize] == 0.0)
+        half = {}
+        for s, (k1, k2, a, cs, _) in enumerate(self.sets):
+            for j, o in enumerate(cs):
+                x = c[o:o + k1 * k2].reshape(k1, k2)
+                for i, (y, _) in enumerate(a):
+                    half[s, i, j] = y @ x, np.abs(y) @ np.abs(x)
+        for off, mine in self.terms:
+            w = {}
+            for (s, i, j, l), (f, g) in mine.items():
+                x, y = half[s, i, j]
+                z = w.setdefault((s, l), [np.zeros_like(x), np.zeros_like(x)])
+                z[0] += f * x
+                z[1] += g * y
+            v = sum(z[0] @ self.sets[s][4][l][0] for (s, l), z in w.items())
+            bound = sum(z[1] @ np.abs(self.sets[s][4][l][0]) for (s, l), z in w.items())
+            err = np.abs(got[off:off + v.size].reshape(v.shape) - v)
+            assert np.all(err <= tol * bound), float((err / bound).max())
+
+
+def test_rounds_stay_within_the_scratch():
+    """Product tiles in four rounds of almost half the W scratch each, whose
+    last unit does not fit: the rounds stay within it, so that four roots
+    still share each launch, and six roots take a second set of launches."""
+    print("[gpu] rounds of product tiles within the W scratch", flush=True)
+    rng = np.random.default_rng(5)
+    # 16 pairs of 128,000 doubles of W are a unit; four rounds of 2^26 doubles hold 2097 pairs
+    x = Products(rng, 1000, 101, [(99, 128)], 2096)
+    c = x.vectors(rng, 6)
+    with Device() as d, Plan(d, x.vbs, x.prs, x.wave, x.arena) as p:
+        one = np.concatenate([p.apply(v, block_amd.FP64) for v in c])
+        single = p.profile(c[0], block_amd.FP64)[2]
+        check(lib.bsg_plan_set_batch(d.ctx, p.h, 4))
+        four = p.profile(c[:4], block_amd.FP64, nvec=4)[2]
+        assert np.array_equal(p.apply(c[:4], block_amd.FP64), one[:4])
+        check(lib.bsg_plan_set_batch(d.ctx, p.h, 6))
+        six = p.profile(c, block_amd.FP64, nvec=6)[2]
+        assert np.array_equal(p.apply(c, block_amd.FP64), one)
+    for v, w in zip(one, c):
+        x.agree(v, w, block_amd.FP64)
+    print(f"[gpu] launches: one root {single}, four {four}, six {six}", flush=True)
+    assert four == single
+    assert single < six <= 2 * single
