@@ -1257,7 +1257,7 @@ inline long gemm_cost(const bsg_pair_t& pr) {
 // W_ONE_ROUND, else an even number of rounds of at most W_HALF each (W_HALF / 2
 // and one unit's W where that is more: blocks of some 20,000 rows); roots
 // share a launch while W_ROOTS holds all of them
-constexpr int64_t W_ONE_ROUND = 1 << 23, W_HALF = 1 << 26, W_ROOTS = 1 << 29, W_KEEP = 1 << 27;
+constexpr int64_t W_ONE_ROUND = 1 << 23, W_HALF = 1 << 26, W_ROOTS = 1 << 29;
 // MFMA instructions per wavefront of one pair in a tile (segment cost)
 inline long pair_cost(const Geom& g, int n, const bsg_pair_t& pr) {
   auto cdiv = [](long a, long b) { return (a + b - 1) / b; };
@@ -1474,8 +1474,11 @@ double* scratch_address(int device) {
 // W scratch of the large blocks' products.  A context's applications run one
 // after the other (its single stream), so its plans share one buffer: plans
 // and their captured graphs keep the buffer they were made with, the context
-// keeps the latest one up to W_KEEP doubles for the next superblock's plan,
-// and the last holder frees it.
+// keeps the latest one up to W_ROOTS doubles for the next superblock's plan
+// (until bsg_free), and the last holder frees it.  Sizes are whole powers of
+// two up to there, so that a sweep's growing superblocks replace it a few times
+// only: memory is cleared when it is given back, and freeing the 4 GB of four
+// roots with every plan took 40 to 300 ms.
 struct WScratch {
   double* ptr = nullptr;
   int64_t doubles = 0;
@@ -1775,10 +1778,16 @@ constexpr int MAX_PLAN_THREADS = 16;
 // the context's W scratch if it holds n doubles, else a new one (null: no memory)
 std::shared_ptr<WScratch> w_scratch(bsg_context* ctx, int64_t n) {
   if (ctx->wscratch && ctx->wscratch->doubles >= n) return ctx->wscratch;
+  const bool keep = n <= W_ROOTS;
+  if (keep) {
+    int64_t p = 1;
+    while (p < n) p <<= 1;
+    n = p;
+  }
   auto w = std::make_shared<WScratch>();
   if (hipMalloc(&w->ptr, sizeof(double) * n) != hipSuccess) return nullptr;
   w->doubles = n;
-  if (n <= W_KEEP) ctx->wscratch = w;
+  if (keep) ctx->wscratch = w;
   return w;
 }
 

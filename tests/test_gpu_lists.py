@@ -4,6 +4,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 import block_amd
 from capi import Device, check, lib, vp
@@ -236,3 +237,35 @@ def test_rounds_stay_within_the_scratch():
     print(f"[gpu] launches: one root {single}, four {four}, six {six}", flush=True)
     assert four == single
     assert single < six <= 2 * single
+
+
+def test_w_scratch_is_kept_for_the_next_plan():
+    """Four roots' W scratch (1 to 4 GB) stays with the context when its plan
+    goes, serves the next plan, smaller or as large, and is given back with the
+    context."""
+    print("[gpu] W scratch kept", flush=True)
+    rng = np.random.default_rng(6)
+    x = Products(rng, 1000, 101, [(99, 128)], 600)
+    c = x.vectors(rng, 4)
+    gb = 1 << 30
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info(0)[0]
+
+    with Device() as d, Plan(d, x.vbs, x.prs, x.wave, x.arena) as p:  # what the library holds until the process ends
+        p.apply(c[0], block_amd.FP64)
+    start = free()
+    with Device() as d:
+        got = []
+        for i in range(3):
+            with Plan(d, x.vbs, x.prs, x.wave, x.arena) as p:
+                before = free()
+                check(lib.bsg_plan_set_batch(d.ctx, p.h, 4))
+                assert i == 0 or before - free() < gb // 4
+                got.append(p.apply(c, block_amd.FP64))
+            assert gb < start - free() < 5 * gb
+        assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    assert start - free() < gb // 4
+    for v, w in zip(got[0], c):
+        x.agree(v, w, block_amd.FP64)
