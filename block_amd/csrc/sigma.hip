@@ -1472,7 +1472,8 @@ double* scratch_address(int device) {
 
 // ---------------------------------------------------------------- context and plan
 // W scratch of the large blocks' products.  A context's applications run one
-// after the other (its single stream), so its plans share one buffer: plans
+// after the other (its single stream; bsg_context::apply keeps the launches of
+// calls from several threads apart), so its plans share one buffer: plans
 // and their captured graphs keep the buffer they were made with, the context
 // keeps the latest one up to W_ROOTS doubles for the next superblock's plan
 // (until bsg_free), and the last holder frees it.  Sizes are whole powers of
@@ -1489,6 +1490,8 @@ constexpr int COEF_SLOTS = 4;
 
 struct bsg_context {
   int device = 0;
+  std::mutex apply;                    // held while an application is enqueued or captured
+  std::mutex wmu;                      // of wscratch
   std::shared_ptr<WScratch> wscratch;
   hipStream_t stream = nullptr;
   // second stream (default priority) on which the small-block kernel runs
@@ -1777,6 +1780,7 @@ constexpr int MAX_PLAN_THREADS = 16;
 
 // the context's W scratch if it holds n doubles, else a new one (null: no memory)
 std::shared_ptr<WScratch> w_scratch(bsg_context* ctx, int64_t n) {
+  std::lock_guard<std::mutex> lk(ctx->wmu);
   if (ctx->wscratch && ctx->wscratch->doubles >= n) return ctx->wscratch;
   const bool keep = n <= W_ROOTS;
   if (keep) {
@@ -2941,6 +2945,7 @@ int bsg_sigma_apply(bsg_context* ctx, bsg_plan* p, const double* arena, const do
                     int32_t precision) {
   if (!ctx || !p || !arena || !c || !v || nvec <= 0) return fail(BSG_ERR_ARG, "bsg_sigma_apply: bad args");
   if (p->ctx != ctx) return fail(BSG_ERR_ARG, "bsg_sigma_apply: plan belongs to another context");
+  std::lock_guard<std::mutex> lk(ctx->apply);
   return sigma_apply_with(ctx, p, arena, c, v, nvec, precision, p->part[precision == BSG_SPLIT_BF16], p->batch);
 }
 
@@ -2948,6 +2953,7 @@ int bsg_plan_capture(bsg_context* ctx, bsg_plan* p, const double* arena, const d
                      int32_t precision) {
   if (!ctx || !p || !arena || !c || !v || nvec <= 0) return fail(BSG_ERR_ARG, "bsg_plan_capture: bad args");
   if (p->ctx != ctx) return fail(BSG_ERR_ARG, "bsg_plan_capture: plan belongs to another context");
+  std::lock_guard<std::mutex> lk(ctx->apply);
   int rc = check_precision(p, arena, precision);
   if (rc) return rc;
   HIPCHK(hipSetDevice(ctx->device));
@@ -2988,6 +2994,7 @@ int bsg_plan_replay(bsg_context* ctx, bsg_plan* p) {
   // the slices the split kernels read must still be those of the captured arena
   int rc = check_precision(p, p->g_arena, p->g_precision);
   if (rc) return rc;
+  std::lock_guard<std::mutex> lk(ctx->apply);  // not between the launches of another thread's application
   HIPCHK(hipGraphLaunch(p->graph, ctx->stream));
   return BSG_OK;
 }
@@ -2996,6 +3003,7 @@ int bsg_sigma_apply_noalloc(bsg_context* ctx, bsg_plan* p, const double* arena, 
                             int32_t nvec, int32_t precision) {
   if (!ctx || !p || !arena || !c || !v || nvec <= 0) return fail(BSG_ERR_ARG, "bsg_sigma_apply_noalloc: bad args");
   if (p->ctx != ctx) return fail(BSG_ERR_ARG, "bsg_sigma_apply_noalloc: plan belongs to another context");
+  std::lock_guard<std::mutex> lk(ctx->apply);
   if (!ctx->scratch) return fail(BSG_ERR_ARG, "bsg_sigma_apply_noalloc: no scratch address for this device");
   const int64_t need = p->part_doubles[precision == BSG_SPLIT_BF16];
   if (need > BSG_NOALLOC_SCRATCH_DOUBLES)
@@ -3026,6 +3034,7 @@ int bsg_sigma_profile(bsg_context* ctx, bsg_plan* p, const double* arena, const 
   } ev((size_t)reps * ngroups * nch * per + 2, nullptr);
   for (auto& e : ev) HIPCHK(hipEventCreate(&e));
   long disp = 0;
+  std::lock_guard<std::mutex> lk(ctx->apply);
   HIPCHK(hipEventRecord(ev[0], ctx->stream));
   for (int r = 0; r < reps; ++r)
     if ((rc = sigma_apply_with(ctx, p, arena, c, v, nvec, precision, p->part[precision == BSG_SPLIT_BF16], p->batch, &disp,

@@ -1,6 +1,7 @@
 """Work lists whose pairs or sizes take the plan's less common routes, through
 the C-ABI, against numpy."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -269,3 +270,37 @@ def test_w_scratch_is_kept_for_the_next_plan():
     assert start - free() < gb // 4
     for v, w in zip(got[0], c):
         x.agree(v, w, block_amd.FP64)
+
+
+@BOTH
+def test_two_threads_apply_two_plans_of_one_context(precision):
+    """Applications of two plans from two threads, whose large blocks share
+    the context's W scratch, each in order and as alone."""
+    print(f"[gpu] two threads, one context, precision {precision}", flush=True)
+    rng = np.random.default_rng(8)
+    xs = [Products(rng, 130, 101, [(99, 128)], 40, blocks=6), Products(rng, 97, 140, [(120, 103)], 40, blocks=6)]
+    cs = [x.vectors(rng, 1) for x in xs]
+    reps = 40
+    with Device() as d:
+        plans = [Plan(d, x.vbs, x.prs, x.wave, x.arena, precision == block_amd.SPLIT_BF16) for x in xs]
+        one = [p.apply(c, precision)[0] for p, c in zip(plans, cs)]
+        dc = [d.upload(c) for c in cs]
+        dv = [[d.zeros(x.wave) for _ in range(reps)] for x in xs]
+        rcs = [[], []]
+
+        def work(i):
+            for v in dv[i]:
+                rcs[i].append(lib.bsg_sigma_apply(d.ctx, plans[i].h, plans[i].arena, dc[i], v, 1, precision))
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in (0, 1)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert rcs == [[0] * reps] * 2
+        for i, x in enumerate(xs):
+            for v in dv[i]:
+                assert np.array_equal(d.download(v, x.wave), one[i])
+            plans[i].__exit__()
+    for x, v, c in zip(xs, one, cs):
+        x.agree(v, c[0], precision)
