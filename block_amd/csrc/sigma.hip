@@ -2021,24 +2021,31 @@ void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, 
   }
 }
 
-// The launch lists of one precision mode: every V block's pairs (in device
-// order: the h_fast first ones are the small-block or per-wave kernel's) are
-// cut into work units of about SEG_COST MFMAs per wave; blocks with several
-// units get partial tiles and an ordered reduction.
-int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
-  ModeLists& ml = pc.ml[split];
-  struct Local {
-    std::vector<GUnit> gunits[NCLS];                 // grouped tiles by kernel class
-    std::vector<std::pair<long, int>> sunits[3];     // (cost, segment) of small-block units (up to 16, 24, 32)
-    std::vector<int> bunits;                         // large blocks' units (segments)
-    std::vector<GUnit> wunits[2], punits[3];         // per-wave tiles (16 x 32, 16 x 64), panels (KB = 3, 5, 6)
-    std::vector<int> gq;                             // pairs of the large blocks' units (indices into h_perm)
-    std::vector<PanelPair> pp;
-    std::vector<Seg> segs;
-    std::vector<RedItem> reds;
-    int64_t poff = 0;
-  };
-  std::vector<Local> loc(MAX_PLAN_THREADS);
+// What one host thread's V blocks contribute to a mode's launch lists, with
+// indices of its own
+struct ListPart {
+  std::vector<GUnit> gunits[NCLS];                 // grouped tiles by kernel class
+  std::vector<std::pair<long, int>> sunits[3];     // (cost, segment) of small-block units (up to 16, 24, 32)
+  std::vector<int> bunits;                         // large blocks' units (segments)
+  std::vector<GUnit> wunits[2], punits[3];         // per-wave tiles (16 x 32, 16 x 64), panels (KB = 3, 5, 6)
+  std::vector<int> gq;                             // pairs of the large blocks' units (indices into h_perm)
+  std::vector<PanelPair> pp;
+  std::vector<Seg> segs;
+  std::vector<RedItem> reds;
+  int64_t poff = 0;                                // partial tiles (doubles)
+};
+// How finely pair lists are cut into units: 0 as the kernels like it, 1 to
+// CUT_WHOLE - 1 at 4^level times the costs, CUT_WHOLE not at all (one unit per
+// kernel that a V block's pairs need at least)
+constexpr int CUT_WHOLE = 5;
+
+// Every V block's pairs (in device order: the h_fast first ones are the
+// small-block or per-wave kernel's) cut into work units of about SEG_COST MFMAs
+// per wave; blocks with several units get partial tiles and an ordered
+// reduction.  Returns the number of parts used.
+int cut_lists(const bsg_plan* p, const PlanChunk& pc, bool split, int level, std::vector<ListPart>& loc) {
+  loc.clear();
+  loc.resize(MAX_PLAN_THREADS);
   const long fill = std::max(SEG_COST_MIN, (long)(pc.flops / (2048.0 * UNITS_MIN)));
   const int nvb = (int)pc.h_vb.size();
   // the widest panels wait for each other's few workgroups beside blocks much
@@ -2047,8 +2054,8 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
   int widest = 0;
   for (const bsg_vblock_t& vb : pc.h_vb) widest = std::max(widest, std::max(vb.m, vb.n));
   const int panel_max = widest <= 2 * PANEL_MAX ? PANEL_MAX : 80;
-  const int nth = over_vblocks(pc.h_vb.data(), nvb, pc.n_pairs, [&](int t, int i0, int i1) {
-    Local& L = loc[t];
+  return over_vblocks(pc.h_vb.data(), nvb, pc.n_pairs, [&](int t, int i0, int i1) {
+    ListPart& L = loc[t];
     std::vector<std::pair<int, int>> units;  // (first, count)
     std::vector<char> ukind;
     std::vector<int> pan[3], big, few[3];
@@ -2077,12 +2084,13 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       };
       // at(q): the list's q-th pair; first: its index where the units point
       auto cut = [&](int first, int n, int kind, auto at) {
-        const long lim = std::min(kind == UK_GEMM ? fill / 2 : fill, kind >= UK_SMALL ? SEG_COST_SMALL[kind - UK_SMALL] : SEG_COST);
+        const long lim = std::min(kind == UK_GEMM ? fill / 2 : fill, kind >= UK_SMALL ? SEG_COST_SMALL[kind - UK_SMALL] : SEG_COST)
+                         << (2 * level);
         int start = 0;
         long cost = 0;
         for (int q = 0; q < n; ++q) {
           cost += cost_of(kind, at(q));
-          if (cost >= lim || q + 1 == n) {
+          if ((cost >= lim && level < CUT_WHOLE) || q + 1 == n) {
             units.push_back({first + start, q + 1 - start});
             ukind.push_back((char)kind);
             start = q + 1;
@@ -2115,13 +2123,15 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       };
       if (slow > 0 && wave_vb) cut(base, slow, UK_WAVE, in_perm(base));
       // in FP64 it also takes the pairs of an identity A and a B' it has room for
-      auto few_pair = [&](int q) { return q < base + slow || (!split && sm && std::max(perm[q].k1, perm[q].k2) <= 32); };
+      auto few_pair = [&](int q) {
+        return q < base + slow || (!split && sm && level < CUT_WHOLE && std::max(perm[q].k1, perm[q].k2) <= 32);
+      };
       if (sm) {
         for (auto& x : few) x.clear();
         for (int q = base; q < base + ntot; ++q) {
           if (!few_pair(q)) continue;
           const int k = std::max(std::max(vb.m, vb.n), std::max(perm[q].k1, perm[q].k2));
-          few[k <= 16 ? 0 : (k <= 24 ? 1 : 2)].push_back(q);
+          few[level == CUT_WHOLE ? 2 : (k <= 16 ? 0 : (k <= 24 ? 1 : 2))].push_back(q);
         }
         for (int k = 0; k < 3; ++k)
           if (!few[k].empty()) cut_by_c(few[k], UK_SMALL + k);
@@ -2141,6 +2151,15 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
               big.push_back(q);
             else
               pan[std::max(k, vb.n) <= 48 ? 0 : (std::max(k, vb.n) <= 80 ? 1 : 2)].push_back(q);
+          }
+          if (level == CUT_WHOLE) {  // the widest class, or product tiles, for all
+            std::vector<int>& to = !big.empty() ? big : (pan[2].empty() ? pan[1] : pan[2]);
+            for (auto& x : pan)
+              if (&x != &to) {
+                to.insert(to.end(), x.begin(), x.end());
+                x.clear();
+              }
+            std::sort(to.begin(), to.end());
           }
           for (int k = 0; k < 3; ++k)
             if (!pan[k].empty()) cut_by_c(pan[k], UK_PANEL + k);
@@ -2216,6 +2235,77 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
       }
     }
   });
+}
+
+// Partial tiles (doubles) of a chunk's FP64 and split lists together, were the
+// pair lists cut at fixed costs for the small-block kernel (V blocks and depths
+// up to 32, one class), the grouped and the per-wave tiles alone.
+// BSG_NOALLOC_SCRATCH_DOUBLES was set for lists cut so: what they keep within
+// it, the finer lists of the kernels that came later keep within it too (cut_to_fit).
+int64_t fixed_cut_partials(const bsg_plan* p, const PlanChunk& pc) {
+  int64_t part[MAX_PLAN_THREADS] = {};
+  auto cdiv = [](long a, long b) { return (a + b - 1) / b; };
+  over_vblocks(pc.h_vb.data(), (int)pc.h_vb.size(), pc.n_pairs, [&](int t, int i0, int i1) {
+    for (int i = i0; i < i1; ++i) {
+      const bsg_vblock_t& vb = pc.h_vb[i];
+      const bsg_pair_t* prs = pc.h_perm.get() + pc.h_base[i];
+      const bool sm = small_block(vb), wave_vb = !sm && table_rule(*p->rules, vb.m, vb.n, false) == wave_candidate();
+      const Geom gm = pick_geom(*p->rules, vb.m, vb.n, 6), gs = pick_geom(*p->rules, vb.m, vb.n, 4);
+      auto small = [&](const bsg_pair_t& pr) {
+        const long nrb = cdiv(vb.m, 16), nnb = cdiv(vb.n, 16), njb = cdiv(pr.k2, 16);
+        return (pr.a_off < 0 ? 0 : (pr.b_off < 0 ? nnb : njb) * cdiv(pr.k1, 4) * nrb) +
+               (pr.b_off < 0 ? 0 : njb * 4 * nrb * nnb) + 24;
+      };
+      // units of the first nf pairs (small-block or per-wave tiles) and of the rest
+      auto units = [&](const Geom& g, int nf) {
+        int64_t n = 0;
+        long cost = 0;
+        for (int q = 0; q < vb.count; ++q) {
+          cost += q >= nf ? pair_cost(g, vb.n, prs[q]) : (sm ? small(prs[q]) : wave_cost(vb.n, prs[q]));
+          if (cost < (q < nf && sm ? 1024 : 2048) && q + 1 != nf && q + 1 != vb.count) continue;
+          ++n;
+          cost = 0;
+        }
+        return n > 1 ? n : 0;
+      };
+      const int nf = pc.h_fast[i];
+      int64_t n = units(gm, nf);
+      if (wave_vb)
+        n += units(gs, 0);
+      else if (gm.code != gs.code || gm.nv != gs.nv)
+        n += units(gs, nf);
+      part[t] += n * vb.m * vb.n;
+    }
+  });
+  int64_t sum = 0;
+  for (int64_t x : part) sum += x;
+  return sum;
+}
+
+// The cut of one mode's lists; coarser than the kernels like it where only that
+// keeps the partial tiles within the static scratch and lists cut at fixed costs
+// would have stayed within it (30 blocks of 32 x 32 with 1000 pairs of depth 1
+// each: 10.3 million doubles, 2.6 million one level coarser; 4000 blocks of 60 x
+// 64 with one pair in each of three panel classes: 30.7 million, none as whole
+// lists).  Returns the doubles of the partial tiles; nth: parts used.
+int64_t cut_to_fit(const bsg_plan* p, const PlanChunk& pc, bool split, std::vector<ListPart>& loc, int& nth) {
+  int64_t need = 0;
+  for (int level = 0; level <= CUT_WHOLE; ++level) {
+    nth = cut_lists(p, pc, split, level, loc);
+    need = 0;
+    for (int t = 0; t < nth; ++t) need += loc[t].poff;
+    if (need <= BSG_NOALLOC_SCRATCH_DOUBLES) break;
+    if (level == 0 && fixed_cut_partials(p, pc) > BSG_NOALLOC_SCRATCH_DOUBLES) break;
+  }
+  return need;
+}
+
+// The launch lists of one precision mode
+int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
+  ModeLists& ml = pc.ml[split];
+  std::vector<ListPart> loc;
+  int nth = 0;
+  cut_to_fit(p, pc, split, loc, nth);
   // concatenate with the local indices shifted
   std::vector<GUnit> gunits[NCLS], wunits[2], punits[3];
   std::vector<std::pair<long, int>> sunits[3];
@@ -2225,7 +2315,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
   std::vector<RedItem> reds;
   int64_t poff = 0;
   if (nth == 1) {
-    Local& L = loc[0];
+    ListPart& L = loc[0];
     for (int k = 0; k < NCLS; ++k) gunits[k].swap(L.gunits[k]);
     for (int k = 0; k < 2; ++k) {
       wunits[k].swap(L.wunits[k]);
@@ -2247,7 +2337,7 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     pp.reserve(np);
     reds.reserve(nr);
     for (int t = 0; t < nth; ++t) {
-      Local& L = loc[t];
+      ListPart& L = loc[t];
       const int sb = (int)segs.size(), ppb = (int)pp.size(), gb = (int)gq.size();
       std::vector<char> kind(L.segs.size(), 0);  // 1: the unit's pairs are in pp, 2: in gq
       for (int k = 0; k < 3; ++k) {

@@ -304,3 +304,23 @@ def test_two_threads_apply_two_plans_of_one_context(precision):
             plans[i].__exit__()
     for x, v, c in zip(xs, one, cs):
         x.agree(v, c[0], precision)
+
+
+@pytest.mark.parametrize("m,n,depths,count,blocks", [
+    (32, 32, [(1, 1)], 1000, 30),                    # cut finely, as a superblock of little work
+    (40, 45, [(1, 1), (60, 3), (90, 1)], 1000, 30),  # in three panel classes as well
+    (60, 64, [(8, 8), (50, 5), (90, 3)], 3, 4000),   # one pair in each class of every block
+    (16, 16, [(8, 8), (20, 5), (30, 3), (40, 3)], 4, 12000),
+], ids=["fine", "fine_classes", "classes", "small_classes"])
+def test_allocation_free_call_takes_lists_of_many_small_units(m, n, depths, count, blocks):
+    """Lists whose partial tiles fit the static scratch when cut at fixed costs
+    fit it as they are cut, in both precisions."""
+    print(f"[gpu] allocation-free, {blocks} blocks of {m} x {n}", flush=True)
+    rng = np.random.default_rng(m)
+    x = Products(rng, m, n, depths, count, blocks)
+    c = x.vectors(rng, 1)
+    with Device() as d, Plan(d, x.vbs, x.prs, x.wave, x.arena, True) as p:
+        for precision in (block_amd.FP64, block_amd.SPLIT_BF16):
+            got = p.apply(c, precision, lib.bsg_sigma_apply_noalloc)
+            assert np.array_equal(got, p.apply(c, precision))
+            x.agree(got[0], c[0], precision)
