@@ -20,6 +20,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -1574,6 +1575,7 @@ struct bsg_plan {
   // roots, part_doubles (the largest chunk's) apart
   double* part[2] = {};
   int64_t part_doubles[2] = {};
+  mutable std::atomic<int64_t> split_partials{-1};  // part_doubles[1] to come, once asked for (-1: not yet)
   std::shared_ptr<const RuleSet> rules;  // the tile table when the plan was created
   int32_t batch = 1;         // roots per launch (bsg_plan_set_batch)
   // by precision mode: W scratch of the large blocks' rounds, wroots roots
@@ -2573,7 +2575,19 @@ int bsg_plan_destroy(bsg_plan* p) {
 }
 
 int64_t bsg_plan_arena_extent(const bsg_plan* p) { return p ? p->arena_extent : 0; }
-int64_t bsg_plan_partial_doubles(const bsg_plan* p) { return p ? std::max(p->part_doubles[0], p->part_doubles[1]) : 0; }
+int64_t bsg_plan_partial_doubles(const bsg_plan* p) {
+  if (!p) return 0;
+  int64_t split = p->split_partials;
+  if (split < 0) {  // the split lists' cut, whether or not they are made yet
+    split = 0;
+    std::vector<ListPart> loc;
+    int nth = 0;
+    for (const PlanChunk& pc : p->chunks)
+      split = std::max(split, pc.ml[1].ready ? pc.ml[1].part_doubles : cut_to_fit(p, pc, true, loc, nth));
+    p->split_partials = split;
+  }
+  return std::max(p->part_doubles[0], split);
+}
 
 }  // extern "C"
 

@@ -186,8 +186,8 @@ int bsg_plan_replay(bsg_context* ctx, bsg_plan* plan);
 
 /* Doubles of partial-tile scratch one application of the plan uses (V blocks
  * whose pair list is cut into several work units; 0 if none): the larger of
- * the FP64 application's and, once bsg_plan_split_arena has set it up, the
- * split one's. */
+ * the FP64 application's and the split one's (before bsg_plan_split_arena too,
+ * where the first call works out how the split lists will be cut). */
 int64_t bsg_plan_partial_doubles(const bsg_plan* plan);
 
 /* bsg_sigma_apply without any allocation, for callers that cannot call

@@ -324,3 +324,17 @@ def test_allocation_free_call_takes_lists_of_many_small_units(m, n, depths, coun
             got = p.apply(c, precision, lib.bsg_sigma_apply_noalloc)
             assert np.array_equal(got, p.apply(c, precision))
             x.agree(got[0], c[0], precision)
+
+
+def test_partial_doubles_cover_split_precision_from_the_start():
+    """The partial tiles a plan reports are those of both precisions, before
+    the split set-up as after it."""
+    print("[gpu] partial tiles before the split set-up", flush=True)
+    rng = np.random.default_rng(10)
+    for m, n, depths in ((40, 50, [(45, 47)]), (20, 24, [(9, 24), (33, 40)]), (90, 70, [(80, 85), (3, 100)])):
+        x = Products(rng, m, n, depths, 300, blocks=4)
+        with Device() as d, Plan(d, x.vbs, x.prs, x.wave, x.arena) as p, Plan(d, x.vbs, x.prs, x.wave, x.arena) as q:
+            before = lib.bsg_plan_partial_doubles(p.h)
+            p.split()
+            q.split()
+            assert before == lib.bsg_plan_partial_doubles(p.h) == lib.bsg_plan_partial_doubles(q.h) > 0
