@@ -23,8 +23,8 @@ __device__ inline dbl2 bload128(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_
 enum : int32_t { SP_ARENA = 0, SP_W = 1, SP_C = 2 };
 // out (m x n) += alpha L (m x K) R (K x n).  L is stored m x K row-major
 // (SEG_LT clear) or K x m (set), R K x n (SEG_RT clear) or n x K (set).
-// Shifts: L's and R's space, the half of the W scratch (read by the planner).
-enum : int32_t { SEG_LT = 1, SEG_RT = 2, SEG_LSPACE = 2, SEG_RSPACE = 4, SEG_HALF = 6 };
+// Shifts: L's and R's space.
+enum : int32_t { SEG_LT = 1, SEG_RT = 2, SEG_LSPACE = 2, SEG_RSPACE = 4 };
 struct GemmSeg {
   int64_t l, r;
   double alpha;

@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -1552,10 +1553,9 @@ struct ModeLists {
 };
 
 struct PlanChunk {
-  bsg_vblock_t* d_vb = nullptr;
-  bsg_pair_t* d_pr = nullptr;
-  void* d_blob = nullptr;  // the allocation of both
-  PairS* d_ps = nullptr;   // slice offsets of the pairs (split precision, built lazily)
+  bsg_vblock_t* d_vb = nullptr;  // (with the FP64 lists)
+  bsg_pair_t* d_pr = nullptr;    // pairs in device order and (split) their slice offsets, where the
+  PairS* d_ps = nullptr;         // grouped or per-wave kernels read them
   // host copies for the launch lists: V blocks, pairs in device order (V
   // block i's at h_base[i], its first h_fast[i] the small-block or per-wave
   // kernel's)
@@ -1598,6 +1598,7 @@ struct bsg_plan {
   int64_t ab_elems = 0, c_elems = 0;
   SliceItem *d_ab_items = nullptr, *d_c_items = nullptr;
   SliceChunk *d_ab_chunks = nullptr, *d_c_chunks = nullptr;
+  void* d_slice_lists = nullptr;  // the allocation of these
   int n_ab_chunks = 0, n_c_chunks = 0;
   __bf16 *d_abs = nullptr, *d_cs = nullptr;
   // one captured application (bsg_plan_capture): its executable graph and
@@ -1801,28 +1802,51 @@ int32_t rounds_roots(int64_t w_doubles, int32_t nroot) {
   return (int32_t)std::max<int64_t>(1, std::min<int64_t>(nroot, W_ROOTS / std::max<int64_t>(1, w_doubles)));
 }
 
-// Device arrays of one upload: parts gathered in a host buffer (256-byte
-// aligned), sent with one allocation and one copy, their pointers set then.
+// f(0) .. f(n - 1) on up to nth host threads
+template <class F>
+void on_threads(int nth, int n, F&& f) {
+  std::atomic<int> next{0};
+  auto run = [&] {
+    for (int i; (i = next++) < n;) f(i);
+  };
+  std::vector<std::thread> th;
+  for (int t = 1; t < std::min(nth, n); ++t) th.emplace_back(run);
+  run();
+  for (auto& x : th) x.join();
+}
+
+// Device arrays of one upload (256-byte aligned parts of one host buffer, sent
+// with one allocation and one copy, their pointers set then).  The buffer is
+// written once, by the jobs, on several threads: zeroed, grown and copied list
+// by list it was half of a plan's time.
 struct Blob {
   std::vector<std::pair<void**, size_t>> parts;
-  std::vector<char> data;
-  void add(void** d, const void* h, size_t bytes) {
-    if (bytes == 0) return;
-    const size_t off = (data.size() + 255) & ~(size_t)255;
-    data.resize(off + bytes);
-    std::memcpy(data.data() + off, h, bytes);
-    parts.push_back({d, off});
+  std::vector<std::function<void(char*)>> jobs;  // each writes its share, given the buffer
+  size_t bytes = 0;
+  // room for an array: its place in the buffer
+  template <class P>
+  size_t place(P** d, size_t n) {
+    if (n == 0) return 0;
+    const size_t off = (bytes + 255) & ~(size_t)255;
+    bytes = off + n;
+    parts.push_back({(void**)d, off});
+    return off;
   }
   template <class T, class P>
-  void add(P** d, const std::vector<T>& h) {
-    add((void**)d, h.data(), sizeof(T) * h.size());
+  void add(P** d, std::vector<T> h) {
+    if (h.empty()) return;
+    const size_t off = place(d, sizeof(T) * h.size());
+    jobs.push_back([off, v = std::make_shared<std::vector<T>>(std::move(h))](char* to) {
+      std::memcpy(to + off, v->data(), sizeof(T) * v->size());
+    });
   }
   // false: no memory (nothing is left allocated)
-  bool send(void** blob) {
-    if (data.empty()) return true;
+  bool send(void** blob, int nth) {
+    if (bytes == 0) return true;
+    std::unique_ptr<char[]> h(new char[bytes]);
+    on_threads(nth, (int)jobs.size(), [&](int i) { jobs[i](h.get()); });
     char* d = nullptr;
-    if (hipMalloc((void**)&d, data.size()) != hipSuccess ||
-        hipMemcpy(d, data.data(), data.size(), hipMemcpyHostToDevice) != hipSuccess) {
+    if (hipMalloc((void**)&d, bytes) != hipSuccess || hipMemcpy(d, h.get(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
       (void)hipFree(d);
       return false;
     }
@@ -1852,183 +1876,46 @@ inline bool small_pair(const bsg_pair_t& pr) {
   return (pr.a_off >= 0 && pr.k1 <= 32 && pr.k2 <= 32) || (pr.a_off < 0 && pr.b_off < 0);
 }
 
-// The large blocks' products: segments of the V units (bunits: indices into
-// segs, whose pairs are gq's) and of the W tiles they read, in rounds of about
-// equal W size.
-void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, const std::vector<int>& bunits,
-                   const std::vector<int>& gq, const std::vector<Seg>& segs, bool split) {
-  const bsg_pair_t* perm = pc.h_perm.get();
-  const auto pad8 = [](int k) { return (k + 7) & ~7; };
-  std::vector<GemmUnit> gu;
-  std::vector<GemmSeg> gs;
-  std::vector<GemmAdd> ga, wadd;
-  int64_t wtot = 0, wunit = 0;  // doubles of W: all units, the largest
-  auto w_size = [&](const bsg_vblock_t& vb, const bsg_pair_t& pr) {
-    if (pr.b_off < 0 || (pr.a_off < 0 && !split)) return (int64_t)0;
-    const int64_t n = split ? (3 * (int64_t)vb.m * pad8(pr.k2) + 3) / 4 : (int64_t)vb.m * pr.k2;  // doubles
-    return (n + 1) & ~(int64_t)1;
-  };
-  int64_t wide_tiles = 0;  // W tiles of the larger shape
-  for (int bu : bunits) {
-    const Seg& sg = segs[bu];
-    const bsg_vblock_t& vb = pc.h_vb[sg.vb];
-    int64_t wu = 0;
-    for (int q = 0; q < sg.count; ++q) {
-      const bsg_pair_t& pr = perm[gq[sg.first + q]];
-      wu += w_size(vb, pr);
-      if (split) wide_tiles += ((vb.m + SplitBig::T - 1) / SplitBig::T) * (int64_t)((pr.k2 + SplitBig::T - 1) / SplitBig::T);
-    }
-    wtot += wu;
-    wunit = std::max(wunit, wu);
-  }
-  const bool wide = wide_tiles >= SPLIT_WIDE;
-  // an even number of rounds once W is large enough to be worth two
-  // (a round is closed by the unit that fills it, which may take it past the
-  // target by almost that unit's W)
-  const int64_t room = std::max(W_HALF / 2, W_HALF - wunit);
-  int64_t nround = 1;
-  if (wtot > W_ONE_ROUND) nround = 2 * ((wtot + room * 2 - 1) / (room * 2));
-  // (no pair with a W: one round)
-  const int64_t target = std::max<int64_t>(1, (wtot + nround - 1) / nround);
-  ml.rounds.reserve(nround + 2);
-  std::vector<GUnit> uw[2], uv[2];
-  int64_t wused = 0, wneed[2] = {};
-  std::vector<std::array<std::vector<TileRef>, 4>> rt;  // W tiles, V tiles by shape
-  // a unit's tiles into the list of its tile shape
-  auto put = [&](std::vector<GUnit>(&to)[2], const GemmUnit& u, long cost) {
-    const int shape = wide ? split_shape(u.m, u.n) : 0;
-    const int edge = split ? (shape ? SplitBig::T : SplitSmall::T) : GemmT::TM;
-    GUnit t;
-    t.cost = cost;
-    t.seg = (int)gu.size();
-    t.ntm = (u.m + edge - 1) / edge;
-    t.ntn = (u.n + edge - 1) / edge;
-    to[shape].push_back(t);
-    gu.push_back(u);
-  };
-  auto close_round = [&]() {
-    if (uv[0].empty() && uv[1].empty()) return;
-    int64_t& need = wneed[rt.size() & 1];
-    need = std::max(need, wused);
-    rt.push_back({xcd_order(uw[0]), xcd_order(uw[1]), xcd_order(uv[0]), xcd_order(uv[1])});
-    for (int k = 0; k < 2; ++k) {
-      uw[k].clear();
-      uv[k].clear();
-    }
-    wused = 0;
-  };
-  for (int bu : bunits) {
-    const Seg& sg = segs[bu];
-    const bsg_vblock_t& vb = pc.h_vb[sg.vb];
-    GemmUnit un{};
-    un.out = sg.p_off < 0 ? vb.v_off : sg.p_off;
-    un.kind = sg.p_off < 0 ? GU_V : GU_PART;
-    un.m = vb.m;
-    un.n = vb.n;
-    un.alpha = 1.0;
-    un.add_first = (int32_t)ga.size();
-    std::vector<GemmSeg> mine;
-    long vcost = 0;
-    for (int q = 0; q < sg.count; ++q) {
-      const bsg_pair_t& pr = perm[gq[sg.first + q]];
-      if (pr.a_off < 0 && pr.b_off < 0) {
-        ga.push_back({pr.c_off, pr.alpha});
-        continue;
-      }
-      GemmSeg x{};
-      const int half = (int)(rt.size() & 1);
-      if (split) {
-        // operands are slices with K padded to 8; op(A) C is formed as W^T, and
-        // an identity A's W = alpha C is split like any other W
-        const PairS& ps = pc.h_ps[gq[sg.first + q]];
-        if (pr.b_off < 0) {
-          x = GemmSeg{ps.a, ps.c, pr.alpha * pr.alpha_a, pad8(pr.k1), BS_C << SEG_RSPACE};
-        } else {
-          GemmUnit w{};
-          w.out = 4 * wused;
-          w.kind = GU_W;
-          w.m = pr.k2;
-          w.n = vb.m;
-          w.pad = half;
-          w.first = (int32_t)gs.size();
-          w.alpha = 1.0;
-          if (pr.a_off >= 0) {
-            w.alpha = pr.alpha * pr.alpha_a;
-            w.count = 1;
-            gs.push_back(GemmSeg{ps.c, ps.a, 1.0, pad8(pr.k1), BS_C << SEG_LSPACE});
-          } else {
-            w.add_first = (int32_t)wadd.size();
-            w.add_count = 1;
-            wadd.push_back({pr.c_off, pr.alpha});
-          }
-          put(uw, w, (pr.k1 + 31) / 32 + 4);
-          x = GemmSeg{4 * wused, ps.b, 1.0, pad8(pr.k2), (BS_W << SEG_LSPACE) | half << SEG_HALF};
-          wused += w_size(vb, pr);
-        }
-      } else if (pr.a_off < 0) {  // V += alpha C B'
-        x = GemmSeg{pr.c_off, pr.b_off, pr.alpha, pr.k2, (SP_C << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0)};
-      } else if (pr.b_off < 0) {  // V += alpha op(A) C
-        x = GemmSeg{pr.a_off, pr.c_off, pr.alpha * pr.alpha_a, pr.k1, (SP_C << SEG_RSPACE) | (pr.a_trans ? SEG_LT : 0)};
-      } else {
-        GemmUnit w{};  // W = alpha op(A) C (m x k2)
-        w.out = wused;  // the half's offset is added below
-        w.kind = GU_W;
-        w.m = vb.m;
-        w.n = pr.k2;
-        w.first = (int32_t)gs.size();
-        w.count = 1;
-        w.alpha = pr.alpha * pr.alpha_a;
-        w.pad = half;
-        gs.push_back(GemmSeg{pr.a_off, pr.c_off, 1.0, pr.k1,
-                             (SP_C << SEG_RSPACE) | (pr.a_trans ? SEG_LT : 0)});
-        put(uw, w, (pr.k1 + GKC - 1) / GKC + 4);
-        x = GemmSeg{wused, pr.b_off, 1.0, pr.k2, (SP_W << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0) | half << SEG_HALF};
-        wused += w_size(vb, pr);
-      }
-      vcost += gemm_cost(pr);
-      mine.push_back(x);
-    }
-    un.add_count = (int32_t)ga.size() - un.add_first;
-    un.first = (int32_t)gs.size();
-    un.count = (int32_t)mine.size();
-    gs.insert(gs.end(), mine.begin(), mine.end());
-    put(uv, un, vcost);
-    if (wused >= target) close_round();
-  }
-  close_round();
-  // the second half of the scratch follows the first; the W units' own
-  // additions follow the V units'
-  const int64_t second = split ? 4 * wneed[0] : wneed[0];
-  for (GemmUnit& u : gu) {
-    if (u.kind != GU_W) continue;
-    if (u.pad) u.out += second;
-    u.add_first += (int32_t)ga.size();
-  }
-  static_assert((int)SP_W == (int)BS_W, "one test for both precisions");
-  for (GemmSeg& x : gs)
-    if (((x.flags >> SEG_LSPACE) & 3) == SP_W && ((x.flags >> SEG_HALF) & 1)) x.l += second;
-  ga.insert(ga.end(), wadd.begin(), wadd.end());
-  p->w_doubles[split] = std::max(p->w_doubles[split], wneed[0] + wneed[1]);
-  blob.add(&ml.d_gu, gu);
-  blob.add(&ml.d_gs, gs);
-  blob.add(&ml.d_ga, ga);
-  ml.rounds.resize(rt.size());
-  for (size_t r = 0; r < rt.size(); ++r) {
-    for (int k = 0; k < 2; ++k) {
-      blob.add(&ml.rounds[r].d_w[k], rt[r][k]);
-      blob.add(&ml.rounds[r].d_v[k], rt[r][2 + k]);
-      ml.rounds[r].n_w[k] = (int)rt[r][k].size();
-      ml.rounds[r].n_v[k] = (int)rt[r][2 + k].size();
-    }
-  }
+// W of a large block's pair (doubles; 0: it needs none); split precision: three
+// slices of W, K padded to 8, of an identity A too
+inline int pad8(int k) { return (k + 7) & ~7; }
+inline int64_t w_size(const bsg_vblock_t& vb, const bsg_pair_t& pr, bool split) {
+  if (pr.b_off < 0 || (pr.a_off < 0 && !split)) return 0;
+  const int64_t n = split ? (3 * (int64_t)vb.m * pad8(pr.k2) + 3) / 4 : (int64_t)vb.m * pr.k2;
+  return (n + 1) & ~(int64_t)1;
 }
+// A V unit of the large blocks: the W units (and, split, additions) of its
+// pairs, its segments and additions; then, where they start in the lists and
+// its W in its round's half of the scratch
+struct LargeUnit {
+  int64_t w = 0, w0 = 0;
+  int64_t wide = 0;  // W tiles of the larger split shape
+  long cost = 0;
+  int part = 0, seg = 0;  // the segment: host thread's part, index there
+  int nw = 0, nwseg = 0, nv = 0, nadd = 0, round = 0;
+  int gu0 = 0, gs0 = 0, ga0 = 0, wadd0 = 0;
+  void pair(const bsg_vblock_t& vb, const bsg_pair_t& pr, bool split) {
+    if (split) wide += ((vb.m + SplitBig::T - 1) / SplitBig::T) * (int64_t)((pr.k2 + SplitBig::T - 1) / SplitBig::T);
+    if (pr.a_off < 0 && pr.b_off < 0) {
+      ++nadd;
+      return;
+    }
+    ++nv;
+    cost += gemm_cost(pr);
+    if (const int64_t x = w_size(vb, pr, split)) {
+      w += x;
+      ++nw;
+      nwseg += pr.a_off >= 0;
+    }
+  }
+};
 
 // What one host thread's V blocks contribute to a mode's launch lists, with
 // indices of its own
 struct ListPart {
   std::vector<GUnit> gunits[NCLS];                 // grouped tiles by kernel class
   std::vector<std::pair<long, int>> sunits[3];     // (cost, segment) of small-block units (up to 16, 24, 32)
-  std::vector<int> bunits;                         // large blocks' units (segments)
+  std::vector<LargeUnit> bunits;                   // large blocks' units
   std::vector<GUnit> wunits[2], punits[3];         // per-wave tiles (16 x 32, 16 x 64), panels (KB = 3, 5, 6)
   std::vector<int> gq;                             // pairs of the large blocks' units (indices into h_perm)
   std::vector<PanelPair> pp;
@@ -2186,7 +2073,11 @@ int cut_lists(const bsg_plan* p, const PlanChunk& pc, bool split, int level, std
         L.segs.push_back(sg);
         const int kind = ukind[u];
         if (kind == UK_GEMM) {
-          L.bunits.push_back(si);
+          LargeUnit b;
+          b.part = t;
+          b.seg = si;
+          for (int q = 0; q < sg.count; ++q) b.pair(vb, perm[L.gq[sg.first + q]], split);
+          L.bunits.push_back(b);
           continue;
         }
         long ucost = 0;
@@ -2302,89 +2193,238 @@ int64_t cut_to_fit(const bsg_plan* p, const PlanChunk& pc, bool split, std::vect
   return need;
 }
 
+// The large blocks' products: the V units' segments and the W tiles they read, in
+// rounds of about equal W size.  Every unit's place in the lists and its share
+// of W come first, then the rounds' tiles, units and segments are written on nth
+// threads.
+void plan_products(bsg_plan* p, const PlanChunk& pc, ModeLists& ml, Blob& blob, const std::vector<ListPart>& loc,
+                   const std::vector<int64_t>& part_at, bool split, int nth) {
+  const bsg_pair_t* perm = pc.h_perm.get();
+  auto units = std::make_shared<std::vector<LargeUnit>>();
+  for (const ListPart& L : loc) units->insert(units->end(), L.bunits.begin(), L.bunits.end());
+  std::vector<LargeUnit>& un = *units;
+  const int nu = (int)un.size();
+  if (nu == 0) return;
+  int64_t wtot = 0, wunit = 0, wide_tiles = 0;  // doubles of W: all units, the largest
+  for (const LargeUnit& u : un) {
+    wtot += u.w;
+    wunit = std::max(wunit, u.w);
+    wide_tiles += u.wide;
+  }
+  const bool wide = wide_tiles >= SPLIT_WIDE;
+  // an even number of rounds once W is large enough to be worth two
+  // (a round is closed by the unit that fills it, which may take it past the
+  // target by almost that unit's W)
+  const int64_t room = std::max(W_HALF / 2, W_HALF - wunit);
+  int64_t nround = 1;
+  if (wtot > W_ONE_ROUND) nround = 2 * ((wtot + room * 2 - 1) / (room * 2));
+  // (no pair with a W: one round)
+  const int64_t target = std::max<int64_t>(1, (wtot + nround - 1) / nround);
+  std::vector<int> first(1, 0);  // the rounds' first units
+  int64_t wused = 0, wneed[2] = {};
+  int ngu = 0, ngs = 0, nga = 0, nwadd = 0;
+  for (int i = 0; i < nu; ++i) {
+    LargeUnit& u = un[i];
+    const int r = u.round = (int)first.size() - 1;
+    u.w0 = wused;
+    u.gu0 = ngu;
+    u.gs0 = ngs;
+    u.ga0 = nga;
+    u.wadd0 = nwadd;
+    ngu += u.nw + 1;
+    ngs += u.nwseg + u.nv;
+    nga += u.nadd;
+    nwadd += u.nw - u.nwseg;
+    wused += u.w;
+    wneed[r & 1] = std::max(wneed[r & 1], wused);
+    if (wused >= target && i + 1 < nu) {
+      first.push_back(i + 1);
+      wused = 0;
+    }
+  }
+  first.push_back(nu);
+  const int nr = (int)first.size() - 1;
+  p->w_doubles[split] = std::max(p->w_doubles[split], wneed[0] + wneed[1]);
+  // the rounds' tiles: W (kind 0) and V (kind 1) tiles by shape
+  std::vector<std::array<std::vector<TileRef>, 4>> rt(nr);
+  on_threads(nth, 2 * nr, [&](int j) {
+    const int r = j >> 1, kind = j & 1;
+    std::vector<GUnit> to[2];
+    auto put = [&](int m, int n, int gu, long cost) {
+      const int shape = wide ? split_shape(m, n) : 0;
+      const int edge = split ? (shape ? SplitBig::T : SplitSmall::T) : GemmT::TM;
+      GUnit t;
+      t.cost = cost;
+      t.seg = gu;
+      t.ntm = (m + edge - 1) / edge;
+      t.ntn = (n + edge - 1) / edge;
+      to[shape].push_back(t);
+    };
+    for (int i = first[r]; i < first[r + 1]; ++i) {
+      const LargeUnit& u = un[i];
+      const ListPart& L = loc[u.part];
+      const Seg& sg = L.segs[u.seg];
+      const bsg_vblock_t& vb = pc.h_vb[sg.vb];
+      if (kind) {
+        put(vb.m, vb.n, u.gu0 + u.nw, u.cost);
+        continue;
+      }
+      int gu = u.gu0;
+      for (int q = 0; q < sg.count; ++q) {
+        const bsg_pair_t& pr = perm[L.gq[sg.first + q]];
+        if (w_size(vb, pr, split) > 0)  // W, split: W^T
+          put(split ? pr.k2 : vb.m, split ? vb.m : pr.k2, gu++, (pr.k1 + (split ? 31 : GKC - 1)) / (split ? 32 : GKC) + 4);
+      }
+    }
+    for (int k = 0; k < 2; ++k) rt[r][2 * kind + k] = xcd_order(to[k]);
+  });
+  ml.rounds.resize(nr);
+  for (int r = 0; r < nr; ++r)
+    for (int k = 0; k < 2; ++k) {
+      ml.rounds[r].n_w[k] = (int)rt[r][k].size();
+      ml.rounds[r].n_v[k] = (int)rt[r][2 + k].size();
+      blob.add(&ml.rounds[r].d_w[k], std::move(rt[r][k]));
+      blob.add(&ml.rounds[r].d_v[k], std::move(rt[r][2 + k]));
+    }
+  // units, segments, additions (the W units' own follow the V units'); the
+  // second half of the scratch follows the first
+  static_assert((int)SP_W == (int)BS_W, "one constant for both precisions");
+  const size_t gu_at = blob.place(&ml.d_gu, sizeof(GemmUnit) * ngu), gs_at = blob.place(&ml.d_gs, sizeof(GemmSeg) * ngs),
+               ga_at = blob.place(&ml.d_ga, sizeof(GemmAdd) * (nga + nwadd));
+  const int64_t second = wneed[0];
+  auto write = [=, &pc, &loc, &part_at](char* to, int i) {
+    const LargeUnit& u = (*units)[i];
+    const ListPart& L = loc[u.part];
+    const Seg& sg = L.segs[u.seg];
+    const bsg_vblock_t& vb = pc.h_vb[sg.vb];
+    const int half = u.round & 1;
+    GemmUnit* gu = (GemmUnit*)(to + gu_at) + u.gu0;
+    GemmSeg *ws = (GemmSeg*)(to + gs_at) + u.gs0, *vs = ws + u.nwseg;
+    GemmAdd *ga = (GemmAdd*)(to + ga_at) + u.ga0, *wadd = (GemmAdd*)(to + ga_at) + nga + u.wadd0;
+    int gs0 = u.gs0, wadd0 = nga + u.wadd0;
+    int64_t at = (split ? 4 : 1) * (u.w0 + (half ? second : 0));  // split: BF16 elements
+    for (int q = 0; q < sg.count; ++q) {
+      const int j = L.gq[sg.first + q];
+      const bsg_pair_t& pr = perm[j];
+      if (pr.a_off < 0 && pr.b_off < 0) {
+        *ga++ = GemmAdd{pr.c_off, pr.alpha};
+        continue;
+      }
+      const int64_t w = (split ? 4 : 1) * w_size(vb, pr, split);
+      if (w > 0) {
+        GemmUnit x{};
+        x.out = at;
+        x.kind = GU_W;
+        x.m = split ? pr.k2 : vb.m;
+        x.n = split ? vb.m : pr.k2;
+        x.alpha = 1.0;
+        if (pr.a_off >= 0) {
+          x.alpha = pr.alpha * pr.alpha_a;
+          x.first = gs0++;
+          x.count = 1;
+          *ws++ = split ? GemmSeg{pc.h_ps[j].c, pc.h_ps[j].a, 1.0, pad8(pr.k1), BS_C << SEG_LSPACE}
+                        : GemmSeg{pr.a_off, pr.c_off, 1.0, pr.k1, (SP_C << SEG_RSPACE) | (pr.a_trans ? SEG_LT : 0)};
+        } else {
+          x.add_first = wadd0++;
+          x.add_count = 1;
+          *wadd++ = GemmAdd{pr.c_off, pr.alpha};
+        }
+        *gu++ = x;
+      }
+      if (split) {
+        // operands are slices with K padded to 8; op(A) C is formed as W^T, and
+        // an identity A's W = alpha C is split like any other W
+        const PairS& ps = pc.h_ps[j];
+        *vs++ = w > 0 ? GemmSeg{at, ps.b, 1.0, pad8(pr.k2), BS_W << SEG_LSPACE}
+                      : GemmSeg{ps.a, ps.c, pr.alpha * pr.alpha_a, pad8(pr.k1), BS_C << SEG_RSPACE};
+      } else if (w > 0) {  // V += W B'
+        *vs++ = GemmSeg{at, pr.b_off, 1.0, pr.k2, (SP_W << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0)};
+      } else if (pr.a_off < 0) {  // V += alpha C B'
+        *vs++ = GemmSeg{pr.c_off, pr.b_off, pr.alpha, pr.k2, (SP_C << SEG_LSPACE) | (pr.b_trans ? SEG_RT : 0)};
+      } else {  // V += alpha op(A) C
+        *vs++ = GemmSeg{pr.a_off, pr.c_off, pr.alpha * pr.alpha_a, pr.k1, (SP_C << SEG_RSPACE) | (pr.a_trans ? SEG_LT : 0)};
+      }
+      at += w;
+    }
+    GemmUnit x{};
+    x.out = sg.p_off < 0 ? vb.v_off : part_at[u.part] + sg.p_off;
+    x.kind = sg.p_off < 0 ? GU_V : GU_PART;
+    x.m = vb.m;
+    x.n = vb.n;
+    x.alpha = 1.0;
+    x.first = u.gs0 + u.nwseg;
+    x.count = u.nv;
+    x.add_first = u.ga0;
+    x.add_count = u.nadd;
+    *gu = x;
+  };
+  constexpr int STEP = 64;  // units a thread takes at a time
+  for (int u0 = 0; u0 < nu; u0 += STEP)
+    blob.jobs.push_back([=](char* to) {
+      for (int i = u0; i < std::min(nu, u0 + STEP); ++i) write(to, i);
+    });
+}
+
 // The launch lists of one precision mode
 int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
   ModeLists& ml = pc.ml[split];
   std::vector<ListPart> loc;
   int nth = 0;
   cut_to_fit(p, pc, split, loc, nth);
-  // concatenate with the local indices shifted
+  // concatenate with the parts' indices shifted: units and their order here, the
+  // rest straight into the upload
   std::vector<GUnit> gunits[NCLS], wunits[2], punits[3];
   std::vector<std::pair<long, int>> sunits[3];
-  std::vector<int> bunits, gq;
-  std::vector<PanelPair> pp;
-  std::vector<Seg> segs;
-  std::vector<RedItem> reds;
-  int64_t poff = 0;
-  if (nth == 1) {
-    ListPart& L = loc[0];
-    for (int k = 0; k < NCLS; ++k) gunits[k].swap(L.gunits[k]);
-    for (int k = 0; k < 2; ++k) {
-      wunits[k].swap(L.wunits[k]);
-    }
+  struct Base {
+    size_t segs = 0, pp = 0, reds = 0;
+  };
+  std::vector<Base> at(nth + 1);
+  std::vector<int64_t> part_at(nth + 1, 0);  // partial tiles
+  for (int t = 0; t < nth; ++t) {
+    const ListPart& L = loc[t];
+    const Base& x = at[t];
+    at[t + 1] = Base{x.segs + L.segs.size(), x.pp + L.pp.size(), x.reds + L.reds.size()};
+    part_at[t + 1] = part_at[t] + L.poff;
+    auto shift = [&](std::vector<GUnit>& to, const std::vector<GUnit>& from) {
+      for (GUnit u : from) {
+        u.seg += (int)x.segs;
+        to.push_back(u);
+      }
+    };
+    for (int k = 0; k < NCLS; ++k) shift(gunits[k], L.gunits[k]);
+    for (int k = 0; k < 2; ++k) shift(wunits[k], L.wunits[k]);
     for (int k = 0; k < 3; ++k) {
-      punits[k].swap(L.punits[k]);
-      sunits[k].swap(L.sunits[k]);
-    }
-    bunits.swap(L.bunits);
-    gq.swap(L.gq);
-    pp.swap(L.pp);
-    segs.swap(L.segs);
-    reds.swap(L.reds);
-    poff = L.poff;
-  } else {
-    size_t ns = 0, np = 0, nr = 0;
-    for (int t = 0; t < nth; ++t) ns += loc[t].segs.size(), np += loc[t].pp.size(), nr += loc[t].reds.size();
-    segs.reserve(ns);
-    pp.reserve(np);
-    reds.reserve(nr);
-    for (int t = 0; t < nth; ++t) {
-      ListPart& L = loc[t];
-      const int sb = (int)segs.size(), ppb = (int)pp.size(), gb = (int)gq.size();
-      std::vector<char> kind(L.segs.size(), 0);  // 1: the unit's pairs are in pp, 2: in gq
-      for (int k = 0; k < 3; ++k) {
-        for (const GUnit& u : L.punits[k]) kind[u.seg] = 1;
-        for (const auto& x : L.sunits[k]) kind[x.second] = 1;
-      }
-      for (int s : L.bunits) kind[s] = 2;
-      for (size_t s = 0; s < L.segs.size(); ++s) {
-        Seg sg = L.segs[s];
-        if (kind[s]) sg.first += kind[s] == 1 ? ppb : gb;
-        if (sg.p_off >= 0) sg.p_off += poff;
-        segs.push_back(sg);
-      }
-      auto shift = [&](std::vector<GUnit>& to, const std::vector<GUnit>& from) {
-        for (GUnit u : from) {
-          u.seg += sb;
-          to.push_back(u);
-        }
-      };
-      for (int k = 0; k < NCLS; ++k) shift(gunits[k], L.gunits[k]);
-      for (int k = 0; k < 2; ++k) {
-        shift(wunits[k], L.wunits[k]);
-      }
-      for (int k = 0; k < 3; ++k) {
-        shift(punits[k], L.punits[k]);
-        for (auto x : L.sunits[k]) sunits[k].push_back({x.first, x.second + sb});
-      }
-      for (int s : L.bunits) bunits.push_back(s + sb);
-      gq.insert(gq.end(), L.gq.begin(), L.gq.end());
-      pp.insert(pp.end(), L.pp.begin(), L.pp.end());
-      for (RedItem r : L.reds) {
-        r.p_off += poff;
-        reds.push_back(r);
-      }
-      poff += L.poff;
+      shift(punits[k], L.punits[k]);
+      for (const auto& u : L.sunits[k]) sunits[k].push_back({u.first, u.second + (int)x.segs});
     }
   }
-  ml.part_doubles = poff;
+  const Base& all = at[nth];
+  ml.part_doubles = part_at[nth];
   Blob blob;
-  blob.data.reserve(sizeof(Seg) * segs.size() + sizeof(RedItem) * reds.size() + sizeof(PanelPair) * pp.size() +
-                    8 * segs.size() + (1 << 16));
-  blob.add(&ml.d_seg, segs);
-  blob.add(&ml.d_red, reds);
-  ml.n_red = (int)reds.size();
-  blob.add(&ml.d_pp, pp);
+  if (!split) blob.add(&pc.d_vb, pc.h_vb);
+  const size_t seg_at = blob.place(&ml.d_seg, sizeof(Seg) * all.segs),
+               red_at = blob.place(&ml.d_red, sizeof(RedItem) * all.reds),
+               pp_at = blob.place(&ml.d_pp, sizeof(PanelPair) * all.pp);
+  ml.n_red = (int)all.reds;
+  for (int t = 0; t < nth; ++t)
+    blob.jobs.push_back([&, t](char* to) {
+      const ListPart& L = loc[t];
+      Seg* seg = (Seg*)(to + seg_at) + at[t].segs;
+      for (size_t u = 0; u < L.segs.size(); ++u) {
+        seg[u] = L.segs[u];
+        if (seg[u].p_off >= 0) seg[u].p_off += part_at[t];
+      }
+      for (int k = 0; k < 3; ++k) {
+        for (const GUnit& u : L.punits[k]) seg[u.seg].first += (int)at[t].pp;
+        for (const auto& u : L.sunits[k]) seg[u.second].first += (int)at[t].pp;
+      }
+      if (!L.pp.empty()) std::memcpy(to + pp_at + sizeof(PanelPair) * at[t].pp, L.pp.data(), sizeof(PanelPair) * L.pp.size());
+      RedItem* red = (RedItem*)(to + red_at) + at[t].reds;
+      for (RedItem r : L.reds) {
+        r.p_off += part_at[t];
+        *red++ = r;
+      }
+    });
   // small-block units, costliest first
   for (int k = 0; k < 3; ++k) {
     auto& su = sunits[k];
@@ -2392,18 +2432,18 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     std::vector<int32_t> sq;
     sq.reserve(su.size());
     for (const auto& x : su) sq.push_back(x.second);
-    blob.add(&ml.d_s[k], sq);
     ml.n_s[k] = (int)sq.size();
+    blob.add(&ml.d_s[k], std::move(sq));
   }
   for (int k = 0; k < NCLS; ++k) {
-    const std::vector<TileRef> t = xcd_order(gunits[k]);
-    blob.add(&ml.d_g[k], t);
+    std::vector<TileRef> t = xcd_order(gunits[k]);
     ml.n_g[k] = (int)t.size();
+    blob.add(&ml.d_g[k], std::move(t));
   }
   for (int k = 0; k < 3; ++k) {
-    const std::vector<TileRef> t = xcd_order(punits[k]);
-    blob.add(&ml.d_p[k], t);
+    std::vector<TileRef> t = xcd_order(punits[k]);
     ml.n_p[k] = (int)t.size();
+    blob.add(&ml.d_p[k], std::move(t));
   }
   // per-wave tiles of each width: units (costliest first) go to the least
   // loaded of the 8 XCDs, a unit's tiles in consecutive wave slots of that
@@ -2428,11 +2468,25 @@ int plan_lists(bsg_plan* p, PlanChunk& pc, bool split) {
     std::vector<TileRef> wt(nwg * 32, TileRef{-1, 0, 0, 0});
     for (int x = 0; x < 8; ++x)
       for (size_t e = 0; e < q[x].size(); ++e) wt[((e / 4) * 8 + x) * 4 + e % 4] = q[x][e];
-    blob.add(&ml.d_w[k], wt);
     ml.n_w[k] = (int)wt.size();
+    blob.add(&ml.d_w[k], std::move(wt));
   }
-  if (!bunits.empty()) plan_products(p, pc, ml, blob, bunits, gq, segs, split);
-  if (!blob.send(&ml.d_blob)) return fail(BSG_ERR_NOMEM, "plan lists");
+  plan_products(p, pc, ml, blob, loc, part_at, split, nth);
+  // the pairs as the grouped and per-wave kernels read them, once a list has such units
+  auto send_pairs = [&](auto** d, const auto* h) {
+    if (*d) return true;
+    const size_t bytes = sizeof(*h) * pc.n_pairs;
+    if (hipMalloc((void**)d, bytes) == hipSuccess && hipMemcpy(*d, h, bytes, hipMemcpyHostToDevice) == hipSuccess)
+      return true;
+    (void)hipFree(*d);
+    *d = nullptr;
+    return false;
+  };
+  bool grouped = false;
+  for (int k = 0; k < NCLS; ++k) grouped |= ml.n_g[k] > 0;
+  if (((grouped || ml.n_w[0] > 0 || ml.n_w[1] > 0) && !send_pairs(&pc.d_pr, pc.h_perm.get())) ||
+      (split && grouped && !send_pairs(&pc.d_ps, pc.h_ps.data())) || !blob.send(&ml.d_blob, nth))
+    return fail(BSG_ERR_NOMEM, "plan lists");
   ml.ready = true;
   return BSG_OK;
 }
@@ -2528,18 +2582,6 @@ int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunk
       p->flops_split += L.flops_split;
       p->arena_extent = std::max(p->arena_extent, L.arena_extent);
     }
-    if (np > 0) {
-      const size_t pb = (sizeof(bsg_pair_t) * np + 255) & ~(size_t)255;
-      char* d = nullptr;
-      if (hipMalloc((void**)&d, pb + sizeof(bsg_vblock_t) * ch.n_vblocks) != hipSuccess)
-        return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: plan arrays");
-      pc.d_blob = d;
-      pc.d_pr = (bsg_pair_t*)d;
-      pc.d_vb = (bsg_vblock_t*)(d + pb);
-      if (hipMemcpy(pc.d_pr, pc.h_perm.get(), sizeof(bsg_pair_t) * np, hipMemcpyHostToDevice) != hipSuccess ||
-          hipMemcpy(pc.d_vb, ch.vblocks, sizeof(bsg_vblock_t) * ch.n_vblocks, hipMemcpyHostToDevice) != hipSuccess)
-        return cleanup(BSG_ERR_HIP, "bsg_plan_create: plan arrays");
-    }
     if (plan_lists(p, pc, false) != BSG_OK) return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: plan arrays");
   }
   for (const PlanChunk& pc : p->chunks) p->part_doubles[0] = std::max(p->part_doubles[0], pc.ml[0].part_doubles);
@@ -2555,15 +2597,12 @@ int bsg_plan_destroy(bsg_plan* p) {
   if (!p) return BSG_OK;
   if (p->ctx) (void)hipStreamSynchronize(p->ctx->stream);
   for (auto& c : p->chunks) {
-    (void)hipFree(c.d_blob);
+    (void)hipFree(c.d_pr);
     (void)hipFree(c.d_ps);
     for (auto& ml : c.ml) (void)hipFree(ml.d_blob);
   }
   for (double* x : p->part) (void)hipFree(x);
-  (void)hipFree(p->d_ab_items);
-  (void)hipFree(p->d_c_items);
-  (void)hipFree(p->d_ab_chunks);
-  (void)hipFree(p->d_c_chunks);
+  (void)hipFree(p->d_slice_lists);
   if (p->abs_from_ctx)
     p->ctx->abs_leased = false;
   else
@@ -2687,26 +2726,28 @@ int build_slices(bsg_plan* p) {
       }
       if (pr.b_off >= 0) ps[j].b = ab_slice(pr.b_off, pr.b_trans ? 0 : 1, vb.n, pr.k2);  // B'(k, col) as [col][k]
     });
-    if (!ps.empty()) {
-      HIPCHK(hipMalloc((void**)&pc.d_ps, sizeof(PairS) * ps.size()));
-      HIPCHK(hipMemcpy(pc.d_ps, ps.data(), sizeof(PairS) * ps.size(), hipMemcpyHostToDevice));
-    }
   }
-  auto send = [](const auto& v, auto** d) {
-    if (v.empty()) return true;
-    const size_t bytes = v.size() * sizeof(v[0]);
-    return hipMalloc((void**)d, bytes) == hipSuccess && hipMemcpy(*d, v.data(), bytes, hipMemcpyHostToDevice) == hipSuccess;
-  };
-  for (auto* v : {&p->ab_items, &p->c_items}) {
-    const bool ab = v == &p->ab_items;
-    std::vector<SliceChunk> chunks;
-    chunks.reserve(v->size() + v->size() / 2);
-    for (size_t i = 0; i < v->size(); ++i)
-      for (int g = 0; g < slice_groups((*v)[i]); g += SLICE_GROUPS) chunks.push_back({(int32_t)i, g});
-    (ab ? p->n_ab_chunks : p->n_c_chunks) = (int)chunks.size();
-    if (!send(*v, ab ? &p->d_ab_items : &p->d_c_items) || !send(chunks, ab ? &p->d_ab_chunks : &p->d_c_chunks))
-      return fail(BSG_ERR_NOMEM, "bsg_plan_split_arena: slice recipes");
+  Blob blob;
+  std::vector<int32_t> first[2];  // the items' first chunks
+  for (int c = 0; c < 2; ++c) {  // operators, wavefunction
+    const std::vector<SliceItem>& items = c ? p->c_items : p->ab_items;
+    std::vector<int32_t>& at = first[c];
+    at.assign(items.size() + 1, 0);
+    for (size_t i = 0; i < items.size(); ++i) at[i + 1] = at[i] + (slice_groups(items[i]) + SLICE_GROUPS - 1) / SLICE_GROUPS;
+    const size_t item_at = blob.place(c ? &p->d_c_items : &p->d_ab_items, sizeof(SliceItem) * items.size()),
+                 chunk_at = blob.place(c ? &p->d_c_chunks : &p->d_ab_chunks, sizeof(SliceChunk) * at.back());
+    constexpr size_t STEP = 4096;  // items a thread takes at a time
+    for (size_t i0 = 0; i0 < items.size(); i0 += STEP)
+      blob.jobs.push_back([&items, &at, item_at, chunk_at, i0](char* to) {
+        for (size_t i = i0; i < std::min(items.size(), i0 + STEP); ++i) {
+          ((SliceItem*)(to + item_at))[i] = items[i];
+          SliceChunk* ch = (SliceChunk*)(to + chunk_at) + at[i];
+          for (int g = 0; g < at[i + 1] - at[i]; ++g) ch[g] = SliceChunk{(int32_t)i, g * SLICE_GROUPS};
+        }
+      });
+    (c ? p->n_c_chunks : p->n_ab_chunks) = at.back();
   }
+  if (!blob.send(&p->d_slice_lists, MAX_PLAN_THREADS)) return fail(BSG_ERR_NOMEM, "bsg_plan_split_arena: slice recipes");
   p->slices_built = true;
   return BSG_OK;
 }
