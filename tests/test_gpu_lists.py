@@ -338,3 +338,79 @@ def test_partial_doubles_cover_split_precision_from_the_start():
             p.split()
             q.split()
             assert before == lib.bsg_plan_partial_doubles(p.h) == lib.bsg_plan_partial_doubles(q.h) > 0
+
+
+@BOTH
+def test_two_rounds_of_odd_sizes(precision):
+    """More W than one round holds: two rounds, each in its half of the
+    scratch on its own stream, with odd sizes, several units per block and a
+    block of identity partners among them."""
+    print(f"[gpu] two rounds, precision {precision}", flush=True)
+    rng = np.random.default_rng(11)
+    x = Products(rng, 99, 131, [(97, 103), (101, 129), (3, 111), (120, 1)], 700, blocks=2)
+    # past 2^23 doubles of W; the split ones are three quarters of that and padded
+    w = sum(99 * int(k2) for k2 in x.prs["k2"])
+    assert w * 3 / 4 > 1 << 23
+    c = x.vectors(rng, 3)
+    with Device() as d, Plan(d, x.vbs, x.prs, x.wave, x.arena, precision == block_amd.SPLIT_BF16) as p:
+        one = np.concatenate([p.apply(v, precision) for v in c])
+        check(lib.bsg_plan_set_batch(d.ctx, p.h, 2))
+        assert np.array_equal(p.apply(c, precision), one)
+    for v, u in zip(one, c):
+        x.agree(v, u, precision)
+
+
+def test_wide_split_tiles_at_odd_sizes():
+    """Enough W tiles for the 128 x 128 split tiles, next to 64 x 64 ones where
+    those would pad too much, at odd sizes around both."""
+    print("[gpu] wide split tiles", flush=True)
+    rng = np.random.default_rng(12)
+    lists = [Products(rng, m, n, [(k, 121), (k, 127), (7, 129), (129, 70)], 2600, blocks=1)
+             for m, n, k in ((125, 127, 113), (129, 97, 31), (257, 115, 66), (65, 250, 125))]
+    # one list of all: C blocks, operators and V blocks of the parts one after the other
+    vbs, prs, arena, first, woff, aoff = [], [], [], 0, 0, 0
+    for x in lists:
+        v, p = x.vbs.copy(), x.prs.copy()
+        v["v_off"] += woff
+        v["first"] += first
+        for f in ("a_off", "b_off"):
+            p[f] += aoff
+        p["c_off"] += woff
+        vbs.append(v)
+        prs.append(p)
+        arena.append(x.arena)
+        first, woff, aoff = first + len(p), woff + x.wave, aoff + len(x.arena)
+    vbs, prs, arena = np.concatenate(vbs), np.concatenate(prs), np.concatenate(arena)
+    tiles = sum(-(-int(v["m"]) // 128) * sum(-(-prs["k2"][v["first"]:v["first"] + v["count"]] // 128)) for v in vbs)
+    assert tiles >= 1 << 14
+    c = np.concatenate([x.vectors(rng, 1)[0] for x in lists])
+    with Device() as d, Plan(d, vbs, prs, woff, arena, True) as p:
+        got = p.apply(c, block_amd.SPLIT_BF16)[0]
+    o = 0
+    for x in lists:
+        x.agree(got[o:o + x.wave], c[o:o + x.wave], block_amd.SPLIT_BF16)
+        o += x.wave
+
+
+CANDIDATES = [(p, i) for p in (block_amd.FP64, block_amd.SPLIT_BF16) for i in range(block_amd.tile_candidates(p))]
+
+
+@pytest.mark.parametrize("precision,cand", CANDIDATES, ids=[f"{'split' if p else 'fp64'}{i}" for p, i in CANDIDATES])
+def test_every_tile_candidate(precision, cand):
+    """Every candidate a tile table may name (grouped tiles, wide ones of four
+    and eight wavefronts, per-wave tiles), for all V blocks, with blocks wider
+    than each of their tiles."""
+    print(f"[gpu] tile candidate {cand} of precision {precision}", flush=True)
+    rng = np.random.default_rng(13)
+    shapes, depths = [(33, 35), (64, 48), (70, 129), (17, 257), (35, 390), (20, 775)], [(1, 2), (37, 45), (66, 70), (90, 33)]
+    vbs, prs, wave, wave_c, arena = work_list(rng, shapes, depths, 2)
+    c = np.zeros(wave)
+    c[:wave_c] = rng.standard_normal(wave_c)
+    split = precision == block_amd.SPLIT_BF16
+    try:
+        block_amd.set_tile_table([(1, 1 << 20, 1, 1 << 20, -1 if split else cand, cand if split else -1)])
+        with Device() as d, Plan(d, vbs, prs, wave, arena, split) as p:
+            got = p.apply(c, precision)[0]
+    finally:
+        block_amd.set_tile_table(block_amd.read_tile_table())
+    agree(got, vbs, prs, c, arena, wave, precision)
