@@ -117,7 +117,8 @@ def ramp_leg(ints, cfg, M, ck, verbose=1):
 def sweep_leg(ints, cfg, M, ck, tmp, verbose=1):
     """One full two-site sweep at M from the ramp's saved state, in FP64 and
     with the precision ladder (its split phase on the superblocks with at
-    least half of their flops on BF16 slices); every step starts from the
+    least half of their flops in pairs past the FP64 panels' sizes, where split
+    precision is the faster one); every step starts from the
     previous step's transformed wavefunction.  The FP64 leg saves its final state, whose
     blocks give the kept states of the timed sweep."""
     n = cfg["ramp_sweeps"]

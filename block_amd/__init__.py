@@ -64,6 +64,7 @@ _sig(_h, "blkh_gpu_sigma_apply", ctypes.c_int, [_vp, _dp, _dp])
 _sig(_h, "blkh_gpu_sigma_diag", ctypes.c_int, [_vp, _dp])
 _sig(_h, "blkh_gpu_sigma_flops", ctypes.c_double, [_vp])
 _sig(_h, "blkh_gpu_sigma_split_share", ctypes.c_double, [_vp])
+_sig(_h, "blkh_gpu_sigma_split_gain_share", ctypes.c_double, [_vp])
 _sig(_h, "blkh_gpu_sigma_pairs", ctypes.c_long, [_vp])
 _sig(_h, "blkh_gpu_sigma_phase_flops", ctypes.c_int, [_vp, _dp, _dp])
 _sig(_h, "blkh_gpu_sigma_arena_bytes", ctypes.c_long, [_vp])
@@ -273,6 +274,7 @@ class multiply_h:
     flops = property(lambda s: host_lib.blkh_gpu_sigma_flops(s._h))
     # share of the flops split mode runs on BF16 slices (the rest is FP64)
     split_share = property(lambda s: host_lib.blkh_gpu_sigma_split_share(s._h))
+    split_gain_share = property(lambda s: host_lib.blkh_gpu_sigma_split_gain_share(s._h))
     pairs = property(lambda s: host_lib.blkh_gpu_sigma_pairs(s._h))
     arena_bytes = property(lambda s: host_lib.blkh_gpu_sigma_arena_bytes(s._h))
 
@@ -362,9 +364,9 @@ def dmrg(ints, nelec=None, twoS=0, irrep=None, nroots=1, weights=None, schedule=
     uploads (then host_ahead applies).
     ladder > 0: split-precision sigma until the Davidson residual norm falls
     below it, FP64 after (convergence is always decided on FP64 sigmas), from
-    sweep ladder_from on (0: also in the warm-up), on superblocks whose flops
-    run at least ladder_min_share on BF16 slices (multiply_h.split_share; the
-    rest of a superblock stays FP64 in split mode).
+    sweep ladder_from on (0: also in the warm-up), on superblocks with at least
+    ladder_min_share of their flops in pairs that split precision runs faster
+    (multiply_h.split_gain_share).
     guess: start every step from the previous step's wavefunction carried into
     the new basis (guess_wavefunction.C:524-636), else from the diagonal.
     checkpoint: file the sweep state is written to after every sweep; resume:

@@ -1590,6 +1590,7 @@ struct bsg_plan {
   int64_t arena_extent = 0;  // doubles of operator arena the pairs reach
   double flops = 0.0, flops1 = 0.0, flops2 = 0.0;
   double flops_split = 0.0;  // of flops: the grouped kernels' pairs (BF16 slices in split mode)
+  double flops_past = 0.0;   // of flops: pairs with a side or depth past the panels'
   // split precision: the arena bsg_plan_split_arena sliced, the slice
   // recipes of the operator blocks (once per arena) and of the C blocks
   // (every application) and their BF16 buffers
@@ -2529,7 +2530,7 @@ int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunk
     // kernel's ones, then the rest
     struct Local {
       int64_t arena_extent = 0;
-      double flops = 0.0, flops1 = 0.0, flops2 = 0.0, flops_split = 0.0;
+      double flops = 0.0, flops1 = 0.0, flops2 = 0.0, flops_split = 0.0, flops_past = 0.0;
       bool bad = false;
       std::vector<bsg_pair_t> rest;
     };
@@ -2561,6 +2562,7 @@ int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunk
           L.flops += f1 + f2;
           L.flops1 += f1;
           L.flops2 += f2;
+          if (std::max(std::max(vb.m, vb.n), std::max(pr.k1, pr.k2)) > PANEL_MAX) L.flops_past += f1 + f2;
           const bool f = sm ? small_pair(pr) : wave_vb && (pr.a_off < 0 || pr.k1 <= 4 * wave_ka(wave_nb(vb.n)));
           if (!f || wave_vb) L.flops_split += f1 + f2;  // split mode: every pair of a per-wave block runs on BF16 slices
           if (f)
@@ -2580,6 +2582,7 @@ int bsg_plan_create(bsg_context* ctx, const bsg_chunk_t* chunks, int32_t n_chunk
       p->flops1 += L.flops1;
       p->flops2 += L.flops2;
       p->flops_split += L.flops_split;
+      p->flops_past += L.flops_past;
       p->arena_extent = std::max(p->arena_extent, L.arena_extent);
     }
     if (plan_lists(p, pc, false) != BSG_OK) return cleanup(BSG_ERR_NOMEM, "bsg_plan_create: plan arrays");
@@ -2885,6 +2888,7 @@ int bsg_plan_set_batch(bsg_context* ctx, bsg_plan* p, int32_t nroot) {
 
 double bsg_plan_flops(const bsg_plan* p) { return p ? p->flops : 0.0; }
 double bsg_plan_split_share(const bsg_plan* p) { return p && p->flops > 0.0 ? p->flops_split / p->flops : 0.0; }
+double bsg_plan_split_gain_share(const bsg_plan* p) { return p && p->flops > 0.0 ? p->flops_past / p->flops : 0.0; }
 int bsg_plan_phase_flops(const bsg_plan* p, double* f1, double* f2) {
   if (!p || !f1 || !f2) return fail(BSG_ERR_ARG, "bsg_plan_phase_flops: bad args");
   *f1 = p->flops1;

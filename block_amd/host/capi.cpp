@@ -307,6 +307,7 @@ int blkh_gpu_sigma_diag(void* h, double* out) {
 }
 double blkh_gpu_sigma_flops(void* h) { return static_cast<GpuSigmaHandle*>(h)->sig->flops(); }
 double blkh_gpu_sigma_split_share(void* h) { return static_cast<GpuSigmaHandle*>(h)->sig->split_share(); }
+double blkh_gpu_sigma_split_gain_share(void* h) { return static_cast<GpuSigmaHandle*>(h)->sig->split_gain_share(); }
 int blkh_gpu_sigma_phase_flops(void* h, double* f1, double* f2) {
   return bsg_plan_phase_flops(static_cast<GpuSigmaHandle*>(h)->sig->plan(), f1, f2);
 }

@@ -83,10 +83,11 @@ void block_davidson_device(GpuSigma& h, std::vector<std::vector<double>>& b, std
     project_lower(vec(Bp, 0));
     normalise(vec(Bp, 0));
   }
-  // the ladder's split phase only where split mode moves most of the work
-  // onto BF16 slices: elsewhere the split sigma is mostly the FP64 small-block
-  // kernel, and the restart at the switch would cost more than it saves
-  bool split = ladder > 0.0 && h.split_share() >= min_split_share;
+  // the ladder's split phase only where split mode is the faster one for most
+  // of the work: FP64 runs small blocks in the same kernel and blocks up to 96
+  // as panels, faster than split does, and the restart at the switch would come
+  // on top
+  bool split = ladder > 0.0 && h.split_gain_share() >= min_split_share;
   h.set_precision(split ? BSG_SPLIT_BF16 : BSG_FP64);
   // the first iteration's (and a ladder restart's) nroots sigmas in one launch set
   h.set_batch(nroots);

@@ -112,9 +112,16 @@ int bsg_plan_phase_flops(const bsg_plan* plan, double* phase1, double* phase2);
 /* Share of the flops that BSG_SPLIT_BF16 runs on BF16 slices (the grouped
  * kernels' pairs; the pairs of V blocks up to 32 x 32 stay FP64, except those
  * with an identity A and an operator B).  No counterpart in the
- * reference; the device Davidson skips the split phase of its precision
- * ladder below a share of one half. */
+ * reference. */
 double bsg_plan_split_share(const bsg_plan* plan);
+/* Share of the flops in pairs with a side or a depth past 96, which FP64 runs
+ * as product tiles and BSG_SPLIT_BF16 faster: the device Davidson skips the
+ * split phase of its precision ladder below a share of one half.  FP64 time
+ * over split time of one application, by this share: 36 orbitals, D2h, peak
+ * dimension 40 to 90 (0.0) 0.46 to 0.85, 100 (0.05) 1.04, 110 (0.64) 1.31, 140
+ * (0.97) 1.17; 24 orbitals, C1, 50 to 100 (0.0) 0.61 to 0.88, 120 (0.97) 0.94,
+ * 150 (0.97) 1.10, 313 (0.97) 1.47. */
+double bsg_plan_split_gain_share(const bsg_plan* plan);
 
 /* Doubles of operator arena the plan's pairs reach (the arena passed to
  * bsg_sigma_apply must hold at least this many). */
