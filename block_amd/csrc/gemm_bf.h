@@ -8,9 +8,11 @@
 //   W^T = alpha C^T op(A)^T: a lane holds 4 consecutive W columns of a W row,
 //   which are scaled, split and stored as 8 bytes per slice;
 //   V += alpha W B'.
-// Bound by L2 and LDS traffic: a slice element is 6 bytes for 32 / 6 of the
-// FP64 kernel's product rate, so the tile is as large as the registers of two
-// waves per SIMD hold (128 x 128: 12 TB/s at full rate, half of a 64 x 64's).
+// A slice element is 6 bytes for 32 / 6 of the FP64 kernel's product rate, so the
+// tile is as large as the registers of two waves per SIMD hold (128 x 128: 12
+// TB/s at full rate, half of a 64 x 64's).  Bound by the chunks' way from L2:
+// waves wait half of their time, with only two per SIMD to cover it (counters:
+// matrix pipes busy 18%, LDS 20% and 7% in bank conflicts, HBM 1.9 TB/s).
 // 24 orbitals, C1, M = 500: 4.90 ms per application on 16-row tiles that read
 // every slice fragment for 16 rows, 2.70 so.
 

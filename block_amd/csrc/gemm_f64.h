@@ -8,11 +8,12 @@
 // contraction: one segment for W, the unit's run of pairs for V.  A pair with
 // an identity partner is a single segment of the second kind.
 //
-// Bound by the FP64 matrix pipes (62% of the rate their instruction reaches by
-// itself; the rest is VALU work beside them and tile edges).  24 orbitals, C1,
-// M = 500 (169 GFLOP): 6.19 ms per application on 16-row tiles that kept W on
-// chip and read C and B' per 16 rows, 3.94 so (43 TFLOP/s); 30 orbitals, M =
-// 800, four roots: 114.4 -> 69.7 ms.  At the time of 4.59 ms, 128 x 64 tiles
+// Bound by the FP64 matrix pipes (busy 59% of the time by the counters; 8% of
+// the MFMAs are padding, waves wait 40% of their time for chunks and barriers,
+// LDS is busy 21%, HBM traffic 1.8 TB/s).  24 orbitals, C1, M = 500 (169
+// GFLOP): 6.19 ms per application on 16-row tiles that kept W on chip and read
+// C and B' per 16 rows, 3.94 so (43 TFLOP/s); 30 orbitals, M = 800, four roots:
+// 114.4 -> 69.7 ms.  At the time of 4.59 ms, 128 x 64 tiles
 // of four wavefronts took 5.57, five waves per SIMD instead of four 5.81.
 typedef double dbl2 __attribute__((ext_vector_type(2)));
 __device__ inline dbl2 bload128(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {

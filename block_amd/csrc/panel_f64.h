@@ -17,7 +17,8 @@
 // a 16-byte load takes two K of an operand whose K is contiguous (the C^T rows
 // are permuted, so that W columns come out in that order).
 //
-// Bound by the MFMA chains of too few wavefronts: C's 51 KB of LDS and 168
+// Bound by the MFMA chains of too few wavefronts (matrix pipes busy 50% by the
+// counters; operands at 3.4 TB/s from HBM): C's 51 KB of LDS and 168
 // registers allow ten to twelve per CU, blocks of 65 to 80 rows fill 7.5.  36
 // orbitals, D2h, M = 1000 (330,000 pairs, blocks up to 79): 4.25 ms per
 // application on the grouped and per-wave tiles, 2.3 with this kernel on two

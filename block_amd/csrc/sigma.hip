@@ -1235,9 +1235,12 @@ inline int split_shape(int m, int n) {
   auto area = [&](int64_t t) { return ((m + t - 1) / t) * ((n + t - 1) / t) * t * t; };
   return 2 * area(128) <= 3 * area(64);
 }
-// ... in superblocks that fill the chip with such tiles: at 11,000 W tiles of
-// 128 (C1, peak dimension 250) the smaller shape alone takes 1.28 ms for 1.40
-// with both, at 22,000 2.91 for 2.71 (C1, 313), at 55,000 2.71 for 2.62
+// ... in superblocks that fill the chip with such tiles.  The smaller shape
+// alone and both take, by W tiles of 128: 4,900 0.71 and 0.74 ms (24 orbitals,
+// C1, peak dimension 150), 11,000 1.04 to 1.20 and 1.05 to 1.20 (195 to 220),
+// 10,900 of 20 orbitals 1.28 and 1.40, 13,300 1.80 and 1.69 (250), 17,800 2.28
+// and 2.04 (280), 21,600 2.89 and 2.67 (313), 55,000 2.71 and 2.62 (36 orbitals,
+// D2h, 79), 193,000 15.2 and 15.3 (190)
 constexpr int64_t SPLIT_WIDE = 1 << 14;
 // MFMA instructions per wavefront of one pair in a panel plus a latency
 // allowance
@@ -1863,11 +1866,14 @@ enum UnitKind : char { UK_GROUPED = 0, UK_WAVE = 2, UK_GEMM = 3, UK_PANEL = 4 /*
 // MFMAs per wavefront of a work unit before its pair list is split (small
 // blocks: by width class; half as much or twice as much in the first two
 // takes 217 and 233 us for 208 on the D2h superblock at M = 250)
-// A superblock of little work is cut finer, to about UNITS_MIN units, down to
-// SEG_COST_MIN (several short runs in flight beat one long chain of pairs: a
-// whole application of the 12-site Hubbard chain from host vectors 232 ->
-// 116 us; 192 at least: 143 us, 24: 120 us; 512 units at least instead of
-// 2048: 185 us for 161 on the D2h superblock at M = 250).
+// A superblock of little work is cut finer, down to SEG_COST_MIN: to the cost
+// that makes UNITS_MIN units of its flops, were every MFMA full (several short
+// runs in flight beat one long chain of pairs: a whole application of the
+// 12-site Hubbard chain from host vectors 232 -> 116 us; 192 at least: 143 us,
+// 24: 120 us; 512 units instead of 2048: 185 us for 161 on the D2h superblock
+// at M = 250).  Costs count padded MFMAs and an allowance per pair, so narrow
+// blocks make more units: 36 orbitals, D2h, 9,500 at peak dimension 40, 13,000
+// at 24, 32,000 at 12; 24 orbitals, C1, 1,600 at 60, 5,000 at 30.
 constexpr long SEG_COST_MIN = 48, UNITS_MIN = 2048;
 constexpr long SEG_COST = 2048, SEG_COST_SMALL[3] = {256, 768, 1024};
 
@@ -1938,9 +1944,11 @@ int cut_lists(const bsg_plan* p, const PlanChunk& pc, bool split, int level, std
   loc.resize(MAX_PLAN_THREADS);
   const long fill = std::max(SEG_COST_MIN, (long)(pc.flops / (2048.0 * UNITS_MIN)));
   const int nvb = (int)pc.h_vb.size();
-  // the widest panels wait for each other's few workgroups beside blocks much
-  // larger than they are (C1, peak dimension 313: 4.05 ms for 3.94 with product
-  // tiles from 81 on; 120: 437 us for 466)
+  // panels up to 96, beside blocks past twice that up to 80: blocks of 81 to 96
+  // as panels and as product tiles take, by the widest block, 2.85 and 3.99 ms
+  // (90, 36 orbitals, D2h), 4.40 and 5.92 (101), 6.96 and 7.18 (119), the same
+  // within 1% from 137 to 277 (both symmetries), and 4.13 and 3.99 ms at 309 (24
+  // orbitals, C1), where the few wide panels end after everything else
   int widest = 0;
   for (const bsg_vblock_t& vb : pc.h_vb) widest = std::max(widest, std::max(vb.m, vb.n));
   const int panel_max = widest <= 2 * PANEL_MAX ? PANEL_MAX : 80;

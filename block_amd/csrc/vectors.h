@@ -4,7 +4,7 @@
 // and by launches at small n, so each reads its vectors as few times as its
 // data dependences allow and takes as few kernels.  One Davidson iteration's
 // vector work with 20 vectors of 801,444: 1.13 -> 0.43 ms, with 6 of 13,752:
-// 315 -> 110 us.
+// 318 -> 125 to 141 us.
 constexpr int RB = 256, RMAXB = 512;  // threads, most workgroups of a reduction
 
 // 16-byte accesses to vectors that are only 8-byte aligned

@@ -49,7 +49,9 @@ typedef struct bsg_plan bsg_plan;
  * or k1 x m (a_trans=1); a_off < 0 means A is the identity (W = C, k1 == m).
  * C is the wavefunction block at c_off, k1 x k2 row-major.  B' = op(B)^T from
  * the arena at b_off, stored k2 x n (b_trans=0) or n x k2 (b_trans=1);
- * b_off < 0 means B' is the identity (k2 == n).  W never leaves the chip. */
+ * b_off < 0 means B' is the identity (k2 == n).  W stays on the chip except for
+ * large V blocks (past 96 on a side, split precision 64), whose W goes through
+ * the plan's scratch. */
 typedef struct {
   int64_t a_off, c_off, b_off;
   int32_t k1, k2, a_trans, b_trans;
@@ -57,7 +59,7 @@ typedef struct {
 } bsg_pair_t;
 
 /* V block at v_off (m x n row-major) with pairs [first, first+count), summed
- * in list order (deterministic). */
+ * in a fixed order (deterministic; by kernel and C block, then list order). */
 typedef struct {
   int64_t v_off;
   int32_t m, n, first, count;
@@ -130,8 +132,8 @@ int64_t bsg_plan_arena_extent(const bsg_plan* plan);
 /* Split precision set-up: checks that the arena holds the plan's extent and
  * enables BSG_SPLIT_BF16 for this arena.  On its first call for a plan it
  * allocates the plan's BF16 slice buffers: three slices x = x0 + x1 + x2 of
- * the FP32 rounding of x (exact) for every operator block the grouped kernel
- * reads, in each orientation it reads it (6 B per element and orientation,
+ * the FP32 rounding of x (exact) for every operator block the split-precision
+ * kernels read, in each orientation they read it (6 B per element and orientation,
  * rows padded to a multiple of 8; about 0.75x the FP64 arena), and the
  * transposed slices of the wavefunction's C blocks (6 B per element), which
  * every split-precision application rewrites.  It then slices the arena's
@@ -146,16 +148,18 @@ int bsg_plan_split_arena(bsg_context* ctx, bsg_plan* plan, const double* arena, 
  * int32 (m_lo, m_hi, n_lo, n_hi, fp64, split); a V block of m x n inside a
  * rule's ranges gets tile geometry number fp64 (FP64 grouped kernel) or split
  * (split-precision kernels) of the candidate list, -1 leaving the default (FP64:
- * panels for blocks and contraction depths up to 96 (80 in superblocks with a block past 192), product tiles above;
- * split: the MFMA-count model's geometry up to 64, product tiles above); the first matching rule applies.  Process-wide, read when
+ * panels for blocks and contraction depths up to 96 (80 in superblocks with a
+ * block past 192), product tiles above; split: the MFMA-count model's geometry
+ * up to 64, product tiles above); the first matching rule applies.
+ * Process-wide, read when
  * plans are created (n = 0 clears).  bsg_tile_candidates gives the list's
  * length for a precision.  For FP64 its last entry is not a geometry but the
  * per-wave tile kernel (one wavefront per 16 x 32 V tile, 16 x 64 for blocks
  * wider than 32 columns; no LDS or barriers)
  * for a block's pairs with k1 <= 64 (80 on the 64-wide tiles) or an identity
  * A; the block's other pairs
- * keep the model's geometry, and split mode keeps the grouped BF16 kernel
- * for the whole block.  Blocks of at most 32 x 32 stay on the small-block
+ * keep the model's geometry, and split mode goes by the rule's own split
+ * column.  Blocks of at most 32 x 32 stay on the small-block
  * kernel whatever the rule.  The tuner that measures them is bench.py --tune;
  * block_amd/tile_table.txt holds the committed result. */
 int bsg_set_tile_table(const int32_t* rules, int32_t n);
