@@ -216,9 +216,9 @@ def copy_calibration(n, reps):
 def _short(name):
     """k_sigma<1, 4, 2> from the demangled signature (or from a mangled name
     the profiler left as it was, e.g. a kernel with __bf16 arguments)."""
-    m = re.match(r"_ZN\w*?\d+(k_[a-z_]+)I((?:Li-?\d+E)+)E", name)
+    m = re.match(r"_ZN\w*?\d+(k_[a-z_]+)I(NS_\d+[A-Za-z]+I)?((?:Li-?\d+E)+)E", name)
     if m:
-        return f"{m.group(1)}<{', '.join(re.findall(r'Li(-?[0-9]+)E', m.group(2)))}>"
+        return f"{m.group(1)}<{', '.join(re.findall(r'Li(-?[0-9]+)E', m.group(3)))}>"
     name = name.replace("void ", "").replace("(anonymous namespace)::", "")
     return name.split("(")[0]
 
