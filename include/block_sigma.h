@@ -3,7 +3,9 @@
  * Plain pointers and sizes only.  Every entry point returns BSG_OK (0) or a
  * negative error code; bsg_last_error() gives the message of the last failure
  * on the calling thread.  All work of one context runs on that context's
- * single HIP stream, in call order (the single-stream contract).
+ * single HIP stream, in call order (the single-stream contract); applications
+ * called from several threads run whole, one after the other, each plan from
+ * one thread at a time.
  *
  * Reference interfaces these replace (sanshar/Block 1.1.1):
  *   multiply_h::operator()(Wavefunction& c, Wavefunction& v)   davidson.h:22-29, davidson.C:17-22
@@ -170,7 +172,9 @@ int bsg_tile_candidates(int32_t precision);
  * XCD so they share its operator blocks in L2), the block Davidson's new
  * vectors of one iteration (linear.C:234-258) and state-averaged roots
  * together.  Reallocates the plan's partial tiles and C slices for nroot
- * vectors (after synchronising the context stream). */
+ * vectors (after synchronising the context stream) and takes W scratch for as
+ * many of them as 4 GB hold; where that is fewer than nroot, the large blocks'
+ * kernels run the roots in turns. */
 int bsg_plan_set_batch(bsg_context* ctx, bsg_plan* plan, int32_t nroot);
 
 /* v += H c for nvec vectors stored back to back (stride wave_size doubles),
@@ -207,7 +211,7 @@ int64_t bsg_plan_partial_doubles(const bsg_plan* plan);
  * in a static device array of BSG_NOALLOC_SCRATCH_DOUBLES doubles (64 MiB),
  * one per GPU, held until the process ends; an application that needs more
  * partial tiles is rejected with BSG_ERR_ARG.  The W scratch of large blocks
- * belongs to the plan (made with it) and its context.  Results
+ * is made with the plan and shared by its context's plans.  Results
  * are bitwise those of bsg_sigma_apply.  Every call on one GPU shares that
  * GPU's array: calls that overlap on one GPU (other contexts' streams, other
  * threads) race and must be serialised by the caller.  The plan itself (and,
@@ -298,8 +302,10 @@ int bsg_olsen_precondition(bsg_context* ctx, double* r, const double* c, const d
  * normalise != 0, r is normalised unless |r|^2 <= 1e-15 (BaseOperator.C:
  * 282-287; a caller that projects r further before that Normalise passes 0).
  * B: m device vectors at stride ld.  The scalars stay in device memory, so
- * the loop runs without a host round trip per step; same reductions and
- * order as bsg_dot / bsg_scal / bsg_axpy. */
+ * the loop runs without a host round trip per step.  One kernel per vector: it
+ * normalises, subtracts the projection and forms the next step's |r|^2 and
+ * <r, b>, so rounding differs from the same steps as bsg_dot / bsg_scal /
+ * bsg_axpy calls. */
 int bsg_gs_orthonormalise(bsg_context* ctx, double* r, const double* B, int32_t m, int64_t ld, int64_t n,
                           int32_t normalise);
 
