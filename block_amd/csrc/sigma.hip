@@ -41,6 +41,8 @@ namespace {
 thread_local std::string g_err;
 int fail(int code, const std::string& msg) {
   g_err = msg;
+  // a HIP error reported here is not the next launch's
+  if (code != BSG_ERR_ARG) (void)hipGetLastError();
   return code;
 }
 #define HIPCHK(x)                                                                             \

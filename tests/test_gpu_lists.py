@@ -414,3 +414,19 @@ def test_every_tile_candidate(precision, cand):
     finally:
         block_amd.set_tile_table(block_amd.read_tile_table())
     agree(got, vbs, prs, c, arena, wave, precision)
+
+
+def test_a_refused_allocation_leaves_the_plan_usable():
+    """More roots than memory holds: refused, the plan is as it was and its next
+    applications succeed."""
+    print("[gpu] refused batch", flush=True)
+    rng = np.random.default_rng(14)
+    x = Products(rng, 100, 60, [(40, 50)], 400, blocks=3)
+    c = x.vectors(rng, 2)
+    with Device() as d, Plan(d, x.vbs, x.prs, x.wave, x.arena) as p:
+        one = p.apply(c, block_amd.FP64)
+        assert 8 * lib.bsg_plan_partial_doubles(p.h) << 26 > 1 << 42  # 4 TB
+        assert lib.bsg_plan_set_batch(d.ctx, p.h, 1 << 26) == -3  # BSG_ERR_NOMEM
+        assert np.array_equal(p.apply(c, block_amd.FP64), one)
+        check(lib.bsg_plan_set_batch(d.ctx, p.h, 2))
+        assert np.array_equal(p.apply(c, block_amd.FP64), one)
