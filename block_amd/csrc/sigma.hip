@@ -1089,8 +1089,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // NV = PB is the basic tile; the wide tiles (WR = 1, NR = 1, NV = 4 or 6)
 // cover up to 256 or 384 V columns, so every W column of a pair is formed
 // once per row panel instead of once per column group.  cls: the FP64
-// kernel instantiation (0: <2, 2>, 1: <1, 4>, 2: <1, 6>); the split-precision
-// kernel runs every tile class as basic tiles (JV = JC).  Chosen to minimise
+// kernel instantiation (0: <2, 2>, 1: <1, 4>, 2: <1, 6>, 3: <1, 6> of eight
+// waves; split precision: 2: <1, 4> of eight waves).  Chosen to minimise
 // the MFMA issue time of the block's tiles (per-wave MFMAs per pair, summed
 // over tiles), which counts row padding, idle column slots and GEMM 1
 // repeated per column group.
@@ -1298,7 +1298,7 @@ inline void costliest_first(std::vector<std::pair<long, int>>& v) {
   v.swap(to);
 }
 
-// Launch order of the grouped kernel's tiles.  Workgroup i runs on XCD
+// Launch order of grouped tiles, panels and product tiles.  Workgroup i runs on XCD
 // i mod 8, each XCD with its own L2: the tiles of one work unit share their
 // C and B' blocks, so a unit's tiles go to one XCD, units are spread over
 // the XCDs by cost (costliest first, to the least loaded XCD), each XCD's
@@ -1501,8 +1501,8 @@ struct bsg_context {
   std::mutex wmu;                      // of wscratch
   std::shared_ptr<WScratch> wscratch;
   hipStream_t stream = nullptr;
-  // second stream (default priority) on which the small-block kernel runs
-  // beside the grouped kernel; fork/join events tie it to `stream`
+  // second stream (default priority) for the kernels that run beside those on
+  // `stream` (enqueue_chunk); fork/join events tie it to that
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
   double* red = nullptr;  // two sets of two partial lists (RMAXB each)
@@ -2793,8 +2793,8 @@ int bsg_plan_split_arena(bsg_context* ctx, bsg_plan* p, const double* arena, int
     if (!(p->wscratch[1] = w_scratch(ctx, p->w_doubles[1] * p->wroots[1])))
       return fail(BSG_ERR_NOMEM, "bsg_plan_split_arena: W scratch");
   }
-  // operator slices for the grouped kernel (the small-block kernel splits
-  // in registers), and room for the C slices of one launch's roots
+  // operator slices (the small-block kernel stays FP64), and room for the C
+  // slices of one launch's roots
   if (!p->d_abs && p->ab_elems > 0) {
     if (!ctx->abs_leased) {
       if (ctx->abs_cap < (size_t)p->ab_elems) {
@@ -2909,7 +2909,7 @@ int bsg_plan_phase_flops(const bsg_plan* p, double* f1, double* f2) {
 }  // extern "C"
 
 namespace {
-// Launch one chunk for rs.n roots: the grouped kernels on the context
+// Launch one chunk for rs.n roots: the widest blocks' kernels on the context
 // stream with the side-stream kernels beside them, then the ordered
 // reduction.  ev (optional) receives 5 events: before the fused kernels,
 // around the side stream's kernels, before and after the reduction.

@@ -113,9 +113,9 @@ int bsg_plan_destroy(bsg_plan* plan);
 double bsg_plan_flops(const bsg_plan* plan);
 /* The same split by GEMM: first (W = op(A) C) and second (V += W op(B)^T). */
 int bsg_plan_phase_flops(const bsg_plan* plan, double* phase1, double* phase2);
-/* Share of the flops that BSG_SPLIT_BF16 runs on BF16 slices (the grouped
- * kernels' pairs; the pairs of V blocks up to 32 x 32 stay FP64, except those
- * with an identity A and an operator B).  No counterpart in the
+/* Share of the flops that BSG_SPLIT_BF16 runs on BF16 slices (all pairs but
+ * those of V blocks up to 32 x 32 that the small-block kernel takes, which stay
+ * FP64: depths up to 32 and no identity A with an operator B).  No counterpart in the
  * reference. */
 double bsg_plan_split_share(const bsg_plan* plan);
 /* Share of the flops in pairs with a side or a depth past 96, which FP64 runs
@@ -181,8 +181,8 @@ int bsg_plan_set_batch(bsg_context* ctx, bsg_plan* plan, int32_t nroot);
  * in launches of up to the plan's batch size (bsg_plan_set_batch).
  * arena: device operator arena; c, v: device pointers.
  * precision: BSG_FP64, or BSG_SPLIT_BF16 (BF16 slice products on MFMA with
- * FP32 accumulation per 32-deep step and FP64 sums for the grouped kernels'
- * pairs, FP64 for the small-block kernel's; needs bsg_plan_split_arena on the same
+ * FP32 accumulation per 32-deep step and FP64 sums, FP64 for the small-block
+ * kernel's pairs; needs bsg_plan_split_arena on the same
  * arena first; ~1e-7 relative error). */
 int bsg_sigma_apply(bsg_context* ctx, bsg_plan* plan, const double* arena, const double* c, double* v, int32_t nvec,
                     int32_t precision);
@@ -225,8 +225,7 @@ int bsg_sigma_apply_noalloc(bsg_context* ctx, bsg_plan* plan, const double* aren
  * (c, v: nvec vectors back to back, roots batched as bsg_sigma_apply does)
  * on the context stream with HIP events around every chunk launch.
  * wall_ms: whole loop; kernel_ms[0..2]: summed time of the fused GEMM-pair
- * kernels (grouped kernels on the context stream and the small-block and
- * basic-tile kernels beside them, fork to join), of the partial-tile
+ * kernels (on the context stream and the side stream, fork to join), of the partial-tile
  * reduction and of the side stream's kernels alone; launches[0]: kernel
  * dispatches of all applications (every launch counted), launches[1..2]: 0. */
 int bsg_sigma_profile(bsg_context* ctx, bsg_plan* plan, const double* arena, const double* c, double* v, int32_t nvec,
